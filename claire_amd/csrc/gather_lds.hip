@@ -491,8 +491,9 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
     __syncthreads();
 
     constexpr int P4 = 4 * G::P;
+    constexpr uint32_t kLast = 4u * (G::W * G::P - 3 * G::PITCH - 6);  // last address a stencil plane can start at
     const char* ldsb = reinterpret_cast<const char*>(lds);
-    int cs = 0;
+    uint32_t cs4 = G::HLO * P4;  // (ring slot of plane x1 - HLO, plus HLO)·P4
     // Stencil rows kept in registers across output planes.  A point's
     // stencil spans input planes x1 + o1 … x1 + o1 + 3; when the next plane's
     // point has the same offsets (o1, o2, o3) -- about 95% of points on a
@@ -504,8 +505,8 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
     // read all four planes.  The values and their order of summation are
     // those of the LDS reads, so results are unchanged bit for bit.
     float2 S[4][4][2];
-    int prev_o1 = 0, prev_lb = -1;
-    auto step = [&](auto kconst, int x1, bool first) {
+    int prev_key = std::numeric_limits<int>::min();
+    auto step = [&](auto kconst, int x1) {
         constexpr int K = decltype(kconst)::value;
         const PlanPt& cur = Q[K & 3];
         const float caux = A[K & 3];
@@ -520,9 +521,9 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
         // period's barrier with no landing pending (measured at 256³,
         // outputs identical: adjoint step 103.9 -> 103.1 µs, three-field
         // gather 289.4 -> 287.3 µs).
-        int spare = cs + G::WIN + G::PERIOD - 1;
-        spare -= (spare >= G::W) ? G::W : 0;
-        float* dst = lds + spare * G::P;
+        uint32_t spare = cs4 + (G::WIN + G::PERIOD - 1 - G::HLO) * P4;
+        spare -= (spare >= G::W * P4) ? G::W * P4 : 0;
+        float* dst = lds + spare / 4;
 #pragma unroll
         for (int q = 0; q < G::FILL; ++q)
             if (tid + kLThreads * q < G::NV) store2(dst, q, PRE[K % NPRE][q][0], PRE[K % NPRE][q][1]);
@@ -530,26 +531,31 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
         lagrange_weights(plan_t(cur.w[0]), w1);
         lagrange_weights(plan_t(cur.w[1]), w2);
         lagrange_weights(plan_t(cur.w[2]), w3);
-        // the plan's bound keeps every stencil inside the ring; the clamps
-        // only pin LDS addresses inside the allocation
-        const int lb = min(max(rc + plan_off(cur.w[1]) * (4 * G::PITCH) + 8 * plan_off(cur.w[2]), 0),
-                           4 * (G::P - 3 * G::PITCH - 6));
-        int sw = min(max(cs + G::HLO + plan_off(cur.w[0]), 0), 2 * G::W - 4);
-        sw -= (sw >= G::W) ? G::W : 0;
-        int base[4];
-        base[0] = opaque(sw * P4 + lb);
-#pragma unroll
-        for (int a = 1; a < 4; ++a) base[a] = opaque(base[a - 1] + ((sw + a == G::W) ? P4 - G::W * P4 : P4));
-        // same offsets as the previous plane's point: the same x1 offset and
-        // the same in-plane stencil address (which fixes the x2 and x3 offsets)
-        const int o1 = plan_off(cur.w[0]);
-        const bool reuse = !first && o1 == prev_o1 && lb == prev_lb;
-        prev_o1 = o1;
-        prev_lb = lb;
+        // Byte address of the stencil's first row, counted from the ring slot
+        // of plane x1 - HLO as if the ring did not end: o1·P4 plus the cell's
+        // address within a plane (below P4, so equal keys are equal offsets).
+        const int key = plan_off(cur.w[0]) * P4 + (rc + plan_off(cur.w[1]) * (4 * G::PITCH) + 8 * plan_off(cur.w[2]));
+        const bool reuse = key == prev_key;  // never on a chunk's first plane
+        prev_key = key;
+        // Stencil plane a starts at x = key + (slot + a)·P4, less the ring's
+        // length W·P4 when it has run past the end: as unsigned numbers the
+        // smaller of the two.  The third operand of the minimum only pins the
+        // address inside the allocation (the plan's bound keeps it there).
+        const uint32_t x0 = static_cast<uint32_t>(key) + cs4;
+        // 156 instead of 161 vector instructions per point and step against
+        // comparing and selecting per plane on ring-slot numbers (one-field
+        // gather at 256³ 94.7 -> 94.4 µs, at 128³ 18.8 -> 18.4 µs; 256³ matvec
+        // 1.957 -> 1.944 ms; outputs identical): a step waits on LDS more than
+        // it issues.
+        auto ring = [&](int a) {
+            const uint32_t x = x0 + static_cast<uint32_t>(a * P4);
+            return opaque(static_cast<int>(min(min(x, x - static_cast<uint32_t>(G::W * P4)), kLast)));
+        };
         auto read_plane = [&](int a, float2 (&R)[4][2]) {
+            const int base = ring(a);
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
-                const char* row = ldsb + base[a] + b * 4 * G::PITCH;
+                const char* row = ldsb + base + b * 4 * G::PITCH;
                 R[b][0] = *reinterpret_cast<const float2*>(row);
                 R[b][1] = *reinterpret_cast<const float2*>(row + 16);
             }
@@ -589,7 +595,7 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
                 bstore(ro, epi.apply(v, caux), off, pb);
             if constexpr (Epi::kOut2) bstore(ro2, epi.apply2(v, caux), off, pb);
         }
-        cs = (cs + 1 == G::W) ? 0 : cs + 1;
+        cs4 = (cs4 == (G::W - 1 + G::HLO) * P4) ? G::HLO * P4 : cs4 + P4;
         if constexpr (K % G::PERIOD == G::PERIOD - 1) __syncthreads();
     };
     using K0 = std::integral_constant<int, 0>;
@@ -599,18 +605,16 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
 
     // four planes per trip (the register sets rotate once)
     int x1 = x1s;
-    bool first = true;
     for (; x1 + 3 < x1e; x1 += 4) {
-        step(K0{}, x1, first);
-        step(K1{}, x1 + 1, false);
-        step(K2{}, x1 + 2, false);
-        step(K3{}, x1 + 3, false);
-        first = false;
+        step(K0{}, x1);
+        step(K1{}, x1 + 1);
+        step(K2{}, x1 + 2);
+        step(K3{}, x1 + 3);
     }
     // the last 0-3 planes continue the rotation
-    if (x1 < x1e) step(K0{}, x1, first);
-    if (x1 + 1 < x1e) step(K1{}, x1 + 1, false);
-    if (x1 + 2 < x1e) step(K2{}, x1 + 2, false);
+    if (x1 < x1e) step(K0{}, x1);
+    if (x1 + 1 < x1e) step(K1{}, x1 + 1);
+    if (x1 + 2 < x1e) step(K2{}, x1 + 2);
 }
 
 // Incremental state right-hand sides, streamed with 16-byte accesses:
