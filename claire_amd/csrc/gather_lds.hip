@@ -815,9 +815,6 @@ __global__ __launch_bounds__(256) void k_to_bfp16(const float* __restrict__ in, 
     }
 }
 
-// Planes per block: at most 48, and the chunk count that fills whole rounds
-// of resident blocks (LDS allows 3 blocks per CU for D <= 2, 1 for D <= 4),
-// weighed against the per-block prologue of WIN planes.
 int num_cus() {
     // one device per process; the first call (any thread) queries it
     static const int cus = [] {
@@ -829,7 +826,7 @@ int num_cus() {
     return cus;
 }
 
-// CLAIRE_AMD_GATHER_CHUNK (planes, >= 4) overrides the choice, for tuning.
+// CLAIRE_AMD_GATHER_CHUNK (planes, >= 1) overrides the choice, for tuning.
 int chunk_override() {
     // read at every launch (not cached) so that a process can switch it
     const char* e = std::getenv("CLAIRE_AMD_GATHER_CHUNK");
@@ -846,41 +843,53 @@ bool pair_layout() {
     return on;
 }
 
-// per_cu: resident blocks per CU (the LDS of one block decides it).
-template <int D>
-int choose_chunk(int n1, int64_t tiles, int per_cu) {
-    using G = LdsGeo<D>;
-    if (chunk_override() >= 4) return std::min(chunk_override(), n1);
-    const int64_t slots = static_cast<int64_t>(num_cus()) * per_cu;
-    // Chunks longer than 48 planes measured slower at 256³ (fewer, longer
-    // blocks start and stream in lockstep); 32-43 planes were best.
-    const int cmax = std::min(n1, 48);
-    int best = cmax;
-    double best_score = -1.0;
-    for (int chunk = cmax; chunk >= 4; --chunk) {
-        const int64_t nch = (n1 + chunk - 1) / chunk;
-        if ((n1 + (chunk - 1) - 1) / (chunk - 1) == nch && chunk > 4) continue;  // same count, larger chunk kept
-        const int64_t blocks = tiles * nch;
-        const int64_t rounds = (blocks + slots - 1) / slots;
-        const double fill = static_cast<double>(blocks) / static_cast<double>(rounds * slots);
-        const double score = fill * chunk / static_cast<double>(chunk + G::WIN / 4);
-        if (score > best_score + 1e-9) {
-            best_score = score;
-            best = chunk;
-        }
+// Chunk lengths (planes per block) worth trying, the most promising first, by
+// a model of the launch: with nch chunks a CU runs k = ceil(tiles·nch/CUs)
+// blocks, `per_cu` of them at a time (their LDS decides it), and a block costs
+// its planes plus a prologue worth about kPrologue planes.  A CU that holds
+// fewer blocks than it could is faster per block but slower overall: share[m]
+// is the time of a plane with m resident blocks over that with per_cu
+// (measured: pair layout 0.85 against 1.25 µs, one-value layout 1.0, 1.7 and
+// 2.35 µs).  Against the measured times of 64³ to 512³ the model is within
+// about 10%, so the tuner below times its best few.  What it finds: one full
+// round of long chunks on large grids (256³, one field: 64 planes 90 µs, 32
+// planes 91, 24 planes 97; 512³: 64 planes 626 µs, 24 planes 697, since a
+// chunk re-reads the planes around it), and enough short chunks to reach every
+// CU on small ones (64³: 2 planes 6.7 µs, 4 planes 8.2, 8 planes 11.3).
+constexpr int kMaxChunk = 128;
+constexpr int kCandidates = 6;
+
+std::vector<int> chunk_candidates(int n1, int64_t tiles, int per_cu) {
+    static const double share[4][4] = {
+        {0, 0, 0, 0}, {0, 1.0, 0, 0}, {0, 0.68, 1.0, 0}, {0, 0.43, 0.72, 1.0}};
+    constexpr double kPrologue = 3.0;
+    std::vector<std::pair<double, int>> cost;
+    for (int nch = 1; nch <= n1; ++nch) {
+        const int chunk = (n1 + nch - 1) / nch;
+        if (chunk > kMaxChunk || (!cost.empty() && cost.back().second == chunk)) continue;
+        const int64_t blocks = tiles * ((n1 + chunk - 1) / chunk);
+        const int64_t k = (blocks + num_cus() - 1) / num_cus();
+        const double rounds = static_cast<double>(k / per_cu) + share[per_cu][k % per_cu];
+        cost.emplace_back(rounds * (chunk + kPrologue), chunk);
     }
-    return best;
+    std::sort(cost.begin(), cost.end());
+    std::vector<int> c;
+    for (size_t i = 0; i < cost.size() && i < static_cast<size_t>(kCandidates); ++i) c.push_back(cost[i].second);
+    return c;
 }
 
 // Chunk-length autotuning.  The first launch of a gather shape (bound D,
-// grid, number of fields) times the heuristic's choice and a few other
-// lengths on the launch stream and keeps the fastest for every later launch
-// of that shape.  The chunk length only changes how the planes are split
-// among blocks, not the arithmetic of any point, so every candidate writes
-// the same output; repeating a launch is harmless because no gather writes a
-// buffer it reads (the launchers check it: the steps refuse to run in place,
-// and the RK4 stage sums ping-pong between two buffers).  Tuning is skipped while the stream is being captured into
-// a graph; CLAIRE_AMD_GATHER_TUNE=0 turns it off (the heuristic is used).
+// grid, number of fields) times the candidates on the launch stream, each
+// kTuneRuns times in turn, and keeps the one with the shortest run for every
+// later launch of that shape (a single run each had kept a length up to 10%
+// slower than the best).  The chunk length only changes how the planes are
+// split among blocks, not the arithmetic of any point, so every candidate
+// writes the same output; repeating a launch is harmless because no gather
+// writes a buffer it reads (the launchers check it: the steps refuse to run in
+// place, and the RK4 stage sums ping-pong between two buffers).  Tuning is
+// skipped while the stream is being captured into a graph;
+// CLAIRE_AMD_GATHER_TUNE=0 turns it off (the model's first choice is used).
+constexpr int kTuneRuns = 3;
 struct ShapeKey {
     int d, n1, n2, n3, nz;
     bool operator<(const ShapeKey& o) const {
@@ -900,40 +909,38 @@ bool tuning_enabled() {
 
 // Launches through `launch(chunk)` with the tuned chunk length of `key`,
 // tuning it on the first launch of that shape (see ShapeKey).
-template <class Launch, class Heuristic>
-void tuned_launch(const ShapeKey& key, int n1, hipStream_t st, Launch&& launch, Heuristic&& heuristic) {
-    if (chunk_override() >= 4) return launch(std::min(chunk_override(), n1));
+template <class Launch>
+void tuned_launch(const ShapeKey& key, int64_t tiles, int per_cu, hipStream_t st, Launch&& launch) {
+    if (chunk_override() >= 1) return launch(std::min(chunk_override(), key.n1));
     {
         std::lock_guard<std::mutex> lock(g_tune_mu);
         const auto it = g_tuned.find(key);
         if (it != g_tuned.end()) return launch(it->second);
     }
-    const int guess = heuristic();
+    const std::vector<int> cand = chunk_candidates(key.n1, tiles, per_cu);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (!tuning_enabled() || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
-        return launch(guess);
-    std::vector<int> cand{guess};
-    for (int c : {16, 24, 32, 40, 48})
-        if (c <= n1 && std::find(cand.begin(), cand.end(), c) == cand.end()) cand.push_back(c);
-    launch(guess);  // warm-up; its output is the result
-    int best = guess;
+        return launch(cand[0]);
+    launch(cand[0]);  // warm-up; its output is the result
+    int best = cand[0];
     if (cand.size() > 1) {
         hipEvent_t ev[2];
         CLR_HIP_CHECK(hipEventCreate(&ev[0]));
         CLR_HIP_CHECK(hipEventCreate(&ev[1]));
         float best_ms = std::numeric_limits<float>::max();
-        for (int c : cand) {
-            CLR_HIP_CHECK(hipEventRecord(ev[0], st));
-            launch(c);
-            CLR_HIP_CHECK(hipEventRecord(ev[1], st));
-            CLR_HIP_CHECK(hipEventSynchronize(ev[1]));
-            float ms = 0.f;
-            CLR_HIP_CHECK(hipEventElapsedTime(&ms, ev[0], ev[1]));
-            if (ms < best_ms) {
-                best_ms = ms;
-                best = c;
+        for (int run = 0; run < kTuneRuns; ++run)
+            for (int c : cand) {
+                CLR_HIP_CHECK(hipEventRecord(ev[0], st));
+                launch(c);
+                CLR_HIP_CHECK(hipEventRecord(ev[1], st));
+                CLR_HIP_CHECK(hipEventSynchronize(ev[1]));
+                float ms = 0.f;
+                CLR_HIP_CHECK(hipEventElapsedTime(&ms, ev[0], ev[1]));
+                if (ms < best_ms) {
+                    best_ms = ms;
+                    best = c;
+                }
             }
-        }
         (void)hipEventDestroy(ev[0]);
         (void)hipEventDestroy(ev[1]);
     }
@@ -958,9 +965,7 @@ void launch_lds(const GatherDims& g, const uint32_t* P, const float* f, int64_t 
                                reinterpret_cast<const PlanPt*>(P), f, fzstride, epi, nb, chunk);
     };
     const ShapeKey key{PAIR ? 100 + D : D, g.n1, g.n2, g.n3, nz};
-    tuned_launch(key, g.n1, st, launch, [&] {
-        return choose_chunk<D>(g.n1, static_cast<int64_t>(nt3) * nt2 * nz, PAIR ? 2 : (D <= 2 ? 3 : 1));
-    });
+    tuned_launch(key, static_cast<int64_t>(nt3) * nt2 * nz, PAIR ? 2 : (D <= 2 ? 3 : 1), st, launch);
 }
 
 template <class Epi>
