@@ -432,7 +432,7 @@ int Regularization::GetExtremeEigValsInvOp(ScalarType& emin, ScalarType& emax) {
 // ---------------------------------------------------------------------------
 // SemiLagrangian (src/SemiLagrangian.cpp)
 // ---------------------------------------------------------------------------
-SemiLagrangian::SemiLagrangian(const RegOpt* opt) : m_Opt(opt), m_Scratch(1) {}
+SemiLagrangian::SemiLagrangian(const RegOpt* opt) : m_Opt(opt), m_PlanMax(kPlanBlocks) {}
 
 int SemiLagrangian::Which(const std::string& flag) const {
     if (flag == "state") return 0;
@@ -455,7 +455,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
         int db = -1;
         {
             KernelScope k(m_Opt->prof, "gather_traj_rk4_plan", 24.0 * nl);
-            db = launch_rk2_predictor_plan(m_Opt->domain, vc, sigma, 0.5f * ht, m_P[w].get(), m_Scratch.get(),
+            db = launch_rk2_predictor_plan(m_Opt->domain, vc, sigma, 0.5f * ht, m_P[w].get(), m_PlanMax.get(),
                                            m_Opt->stream);
         }
         if (vc[1] - vc[0] == nl && vc[2] - vc[1] == nl) {
@@ -474,7 +474,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
                 // bytes: point components read (12) + plan (12) (+ X interleaved (12) at the end)
                 KernelScope k(m_Opt->prof, "gather_plan", (stage < 3 ? 24.0 : 36.0) * nl);
                 db = launch_make_plan_soa(g, m_W.get(), stage == 3 ? m_X[w].get() : nullptr, m_P[w].get(),
-                                          m_Scratch.get(), m_Opt->stream);
+                                          m_PlanMax.get(), m_Opt->stream);
                 if (stage == 3) {
                     m_D[w] = db;
                     m_Valid[w] = true;
@@ -497,7 +497,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
             // the Euler predictor's plan: v read (12) + plan written (12) per point
             KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 24.0 * nl);
             dpred = launch_rk2_predictor_plan(m_Opt->domain, vc, sigma, m_Opt->GetTimeStepSize(), m_P[w].get(),
-                                              m_Scratch.get(), m_Opt->stream);
+                                              m_PlanMax.get(), m_Opt->stream);
         }
         if (dpred >= 0 && dpred <= lds_gather_max_displacement() && vc[1] - vc[0] == nl && vc[2] - vc[1] == nl) {
             m_W.resize(3 * static_cast<size_t>(nl));
@@ -509,7 +509,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
             }
             // bytes: X components read (12) + X interleaved (12) + plan (12) per point
             KernelScope k(m_Opt->prof, "gather_plan", 36.0 * nl);
-            m_D[w] = launch_make_plan_soa(g, m_W.get(), m_X[w].get(), m_P[w].get(), m_Scratch.get(), m_Opt->stream);
+            m_D[w] = launch_make_plan_soa(g, m_W.get(), m_X[w].get(), m_P[w].get(), m_PlanMax.get(), m_Opt->stream);
             m_Valid[w] = true;
             return 0;
         }
@@ -521,7 +521,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
     {
         // bytes: X read (12) + packed plan written (12) per point
         KernelScope k(m_Opt->prof, "gather_plan", 24.0 * m_Opt->domain.nl);
-        m_D[w] = launch_make_plan(gather_dims(m_Opt->domain), m_X[w].get(), m_P[w].get(), m_Scratch.get(),
+        m_D[w] = launch_make_plan(gather_dims(m_Opt->domain), m_X[w].get(), m_P[w].get(), m_PlanMax.get(),
                                   m_Opt->stream);
     }
     m_Valid[w] = true;

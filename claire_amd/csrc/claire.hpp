@@ -66,6 +66,28 @@ class DeviceArray {
     size_t n_ = 0;
 };
 
+// Owning allocation of pinned host memory that kernels write to and the host
+// reads after a stream synchronization.
+template <class T>
+class PinnedArray {
+  public:
+    explicit PinnedArray(size_t n) {
+        void* p = nullptr;
+        const hipError_t e = hipHostMalloc(&p, n * sizeof(T), hipHostMallocDefault);
+        if (e != hipSuccess)
+            throw claire_amd::Error(claire_amd::kErrOutOfMemory, "hipHostMalloc of " + std::to_string(n * sizeof(T)) +
+                                                                     " bytes failed: " + hipGetErrorString(e));
+        p_ = static_cast<T*>(p);
+    }
+    ~PinnedArray() { (void)hipHostFree(p_); }
+    PinnedArray(const PinnedArray&) = delete;
+    PinnedArray& operator=(const PinnedArray&) = delete;
+    T* get() const { return p_; }
+
+  private:
+    T* p_ = nullptr;
+};
+
 // Per-kernel-class timing with HIP events recorded on the context stream.
 class Profiler {
   public:
@@ -303,7 +325,7 @@ class SemiLagrangian {
     DeviceArray<float> m_F2;  // RK4 stage sum after stage 2 (LDS path; kept apart from m_F)
     DeviceArray<float> m_W;  // RK2 corrector output, one component per field (LDS path)
     DeviceArray<float> m_Tmp;  // in-place interpolation (the reference's ghost copy), kept between calls
-    DeviceArray<int> m_Scratch;
+    PinnedArray<int> m_PlanMax;  // the plan kernels' block maxima (displacement bounds)
     bool m_Valid[2] = {false, false};
     int m_D[2] = {0, 0};
 };

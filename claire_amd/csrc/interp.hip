@@ -117,13 +117,12 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk2(GatherDims g, HH hh, Traj
     grid_index(g, i, idx);
     const float x[3] = {tp.hx[0] * static_cast<float>(idx[0]), tp.hx[1] * static_cast<float>(idx[1]),
                         tp.hx[2] * static_cast<float>(idx[2])};
-    const double twopi = 2.0 * 3.14159265358979323846;
     float vl[3], q[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         vl[d] = v.in[d][i];
         const float t = x[d] - tp.sht * vl[d];
-        q[d] = static_cast<float>(static_cast<double>(t) / twopi);
+        q[d] = static_cast<float>(over_2pi(static_cast<double>(t)));
     }
     Stencil S;
     setup_stencil(q, g, hh.h, S);
@@ -132,7 +131,7 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk2(GatherDims g, HH hh, Traj
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         const float t = x[d] - tp.shth * (vx[d] + vl[d]);
-        X[3 * i + d] = static_cast<float>(static_cast<double>(t) / twopi);
+        X[3 * i + d] = static_cast<float>(over_2pi(static_cast<double>(t)));
     }
 }
 
@@ -167,14 +166,13 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk4(GatherDims g, HH hh, Rk4P
     if (i >= g.nl) return;
     float x[3];
     grid_point(g, tp.hx, i, x);
-    const double twopi = 2.0 * 3.14159265358979323846;
     float vl[3], q[3];
     if constexpr (STAGE == 1) {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             vl[d] = v.in[d][i];
             const float t = x[d] - tp.shth * vl[d];
-            q[d] = static_cast<float>(static_cast<double>(t) / twopi);
+            q[d] = static_cast<float>(over_2pi(static_cast<double>(t)));
         }
     } else {
         load_q3(X, i, q);
@@ -188,27 +186,26 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk4(GatherDims g, HH hh, Rk4P
         if constexpr (STAGE == 1) {
             F[3 * i + d] = static_cast<float>(static_cast<double>(vl[d]) + 2.0 * static_cast<double>(vx[d]));
             const float t = x[d] - tp.shth * vx[d];
-            X[3 * i + d] = static_cast<float>(static_cast<double>(t) / twopi);
+            X[3 * i + d] = static_cast<float>(over_2pi(static_cast<double>(t)));
         } else if constexpr (STAGE == 2) {
             F[3 * i + d] = static_cast<float>(static_cast<double>(F[3 * i + d]) + 2.0 * static_cast<double>(vx[d]));
             const float t = x[d] - tp.sht * vx[d];
-            X[3 * i + d] = static_cast<float>(static_cast<double>(t) / twopi);
+            X[3 * i + d] = static_cast<float>(over_2pi(static_cast<double>(t)));
         } else {
             const float f = F[3 * i + d] + vx[d];
-            X[3 * i + d] = static_cast<float>((static_cast<double>(x[d]) - tp.s6 * static_cast<double>(f)) / twopi);
+            X[3 * i + d] = static_cast<float>(over_2pi(static_cast<double>(x[d]) - tp.s6 * static_cast<double>(f)));
         }
     }
 }
 
-// Block maximum of `need` into *dmax (one atomic per block).
-__device__ __forceinline__ void block_max_to(int need, int* sh, int* dmax) {
-    sh[threadIdx.x] = need;
+// Block maximum of `need` into bmax[blockIdx.x].
+__device__ __forceinline__ void block_max_to(int need, int* bmax) {
+    __shared__ int sh[kThreads / 64];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) need = max(need, __shfl_xor(need, o, 64));
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = need;
     __syncthreads();
-    for (int s = kThreads / 2; s > 0; s >>= 1) {
-        if (threadIdx.x < s) sh[threadIdx.x] = max(sh[threadIdx.x], sh[threadIdx.x + s]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) atomicMax(dmax, sh[0]);
+    if (threadIdx.x == 0) bmax[blockIdx.x] = max(max(sh[0], sh[1]), max(sh[2], sh[3]));
 }
 
 // Encodes the three axes of foot point q at grid index idx; returns the
@@ -235,14 +232,19 @@ __device__ __forceinline__ int encode_point(const GatherDims& g, const HH& hh, c
 // that every stencil lies within [i − D − 1, i + D + 2] per axis (the window
 // of the LDS-staged gathers).  Points that cannot be encoded (non-finite
 // coordinates) set D to 1 << 20, which routes every gather along this
-// trajectory to the direct kernels on the raw foot points.  A bounded grid
-// strides over the points, so that the blocks' maxima meet in few atomics
-// (one per block: tens of thousands on one address serialize).
-constexpr int kPlanBlocks = 2048;
+// trajectory to the direct kernels on the raw foot points.
+//
+// Each block writes its maximum into its own word of a host-resident array,
+// which the host reduces after the wait that it needs anyway: no word to clear
+// before the launch and no copy after it.  One word for all blocks made the
+// kernels wait for up to 2048 atomics on one address.  Measured with the
+// division-free x/2π (gather_device.hpp): set velocity + both trajectories +
+// one gather at 64³ 281 -> 188 µs, 96³ 391 -> 262, 128³ 462 -> 343, 256³
+// 1703 -> 1627, outputs identical.
+static_assert(kPlanBlocks >= 1 && kThreads == 256, "block_max_to folds four waves");
 
 __global__ __launch_bounds__(kThreads) void k_make_plan(GatherDims g, HH hh, const float* __restrict__ X,
-                                                        PlanPt* __restrict__ P, int* __restrict__ dmax) {
-    __shared__ int sh[kThreads];
+                                                        PlanPt* __restrict__ P, int* __restrict__ bmax) {
     int need = 0;
     const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
     const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
@@ -254,18 +256,14 @@ __global__ __launch_bounds__(kThreads) void k_make_plan(GatherDims g, HH hh, con
         need = max(need, encode_point(g, hh, q, gw.idx, pt));
         P[i] = pt;
     }
-    block_max_to(need, sh, dmax);
+    block_max_to(need, bmax);
 }
-
-__global__ void k_zero_int(int* p) { *p = 0; }
 
 // Plan of the RK2 Euler predictor X̃ = (x − σ·ht·v)/2π, with the same float
 // and double steps as k_traj_rk2 (bounded grid, like k_make_plan).
 __global__ __launch_bounds__(kThreads) void k_predictor_plan(GatherDims g, HH hh, TrajParams tp, P3 v,
-                                                             PlanPt* __restrict__ P, int* __restrict__ dmax) {
-    __shared__ int sh[kThreads];
+                                                             PlanPt* __restrict__ P, int* __restrict__ bmax) {
     int need = 0;
-    const double twopi = 2.0 * 3.14159265358979323846;
     const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
     const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     GridWalk gw(g, i0, stride);
@@ -275,21 +273,20 @@ __global__ __launch_bounds__(kThreads) void k_predictor_plan(GatherDims g, HH hh
         for (int d = 0; d < 3; ++d) {
             const float x = tp.hx[d] * static_cast<float>(gw.idx[d]);
             const float t = x - tp.sht * v.in[d][i];
-            q[d] = static_cast<float>(static_cast<double>(t) / twopi);
+            q[d] = static_cast<float>(over_2pi(static_cast<double>(t)));
         }
         PlanPt pt;
         need = max(need, encode_point(g, hh, q, gw.idx, pt));
         P[i] = pt;
     }
-    block_max_to(need, sh, dmax);
+    block_max_to(need, bmax);
 }
 
 // Plan of foot points given per component (W + d·nl), which are also
 // written interleaved into X (3 floats per point) unless X is null.
 __global__ __launch_bounds__(kThreads) void k_make_plan_soa(GatherDims g, HH hh, const float* __restrict__ W,
                                                             float* __restrict__ X, PlanPt* __restrict__ P,
-                                                            int* __restrict__ dmax) {
-    __shared__ int sh[kThreads];
+                                                            int* __restrict__ bmax) {
     int need = 0;
     const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
     const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
@@ -305,7 +302,7 @@ __global__ __launch_bounds__(kThreads) void k_make_plan_soa(GatherDims g, HH hh,
         need = max(need, encode_point(g, hh, q, gw.idx, pt));
         P[i] = pt;
     }
-    block_max_to(need, sh, dmax);
+    block_max_to(need, bmax);
 }
 
 // Update coefficient c = 1 + ht/2·(α·dX + α·(1 + ht·α·dX)·d), d = ∇·v,
@@ -427,22 +424,27 @@ void launch_trajectory_rk4(const Dims& d, const float* const v[3], float sigma, 
     hipLaunchKernelGGL(k_traj_rk4<3>, dim3(nb), dim3(kThreads), 0, st, g, hh, tp, p, X, F, nb);
 }
 
-int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* scratch, hipStream_t st) {
+namespace {
+// The bound of a plan launch of nb blocks, after waiting for the stream.
+int plan_bound(const int* bmax, int nb, hipStream_t st) {
+    CLR_HIP_CHECK(hipGetLastError());  // a launch that failed wrote no maxima
+    CLR_HIP_CHECK(hipStreamSynchronize(st));
+    return *std::max_element(bmax, bmax + nb);
+}
+}  // namespace
+
+int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* bmax, hipStream_t st) {
     check_gather_dims(g);
     CLR_REQUIRE(g.n1 <= kPlanMaxN && g.n2 <= kPlanMaxN && g.n3 <= kPlanMaxN, kErrUnsupportedSize,
                 "trajectory plans support at most 512 points per axis");
     const int nb = std::min(nblocks_for(g.nl), kPlanBlocks);
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, scratch);
     hipLaunchKernelGGL(k_make_plan, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), X, reinterpret_cast<PlanPt*>(P),
-                       scratch);
-    int h = 0;
-    CLR_HIP_CHECK(hipMemcpyAsync(&h, scratch, sizeof(int), hipMemcpyDeviceToHost, st));
-    CLR_HIP_CHECK(hipStreamSynchronize(st));
-    return h;
+                       bmax);
+    return plan_bound(bmax, nb, st);
 }
 
 int launch_rk2_predictor_plan(const Dims& d, const float* const v[3], float sigma, float ht, uint32_t* P,
-                              int* scratch, hipStream_t st) {
+                              int* bmax, hipStream_t st) {
     const GatherDims g = gather_dims(d);
     check_gather_dims(g);
     CLR_REQUIRE(g.n1 <= kPlanMaxN && g.n2 <= kPlanMaxN && g.n3 <= kPlanMaxN, kErrUnsupportedSize,
@@ -453,27 +455,19 @@ int launch_rk2_predictor_plan(const Dims& d, const float* const v[3], float sigm
     tp.shth = sigma * (0.5f * ht);
     P3 p{{v[0], v[1], v[2]}, {nullptr, nullptr, nullptr}};
     const int nb = std::min(nblocks_for(g.nl), kPlanBlocks);
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, scratch);
     hipLaunchKernelGGL(k_predictor_plan, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), tp, p,
-                       reinterpret_cast<PlanPt*>(P), scratch);
-    int h = 0;
-    CLR_HIP_CHECK(hipMemcpyAsync(&h, scratch, sizeof(int), hipMemcpyDeviceToHost, st));
-    CLR_HIP_CHECK(hipStreamSynchronize(st));
-    return h;
+                       reinterpret_cast<PlanPt*>(P), bmax);
+    return plan_bound(bmax, nb, st);
 }
 
-int launch_make_plan_soa(const GatherDims& g, const float* W, float* X, uint32_t* P, int* scratch, hipStream_t st) {
+int launch_make_plan_soa(const GatherDims& g, const float* W, float* X, uint32_t* P, int* bmax, hipStream_t st) {
     check_gather_dims(g);
     CLR_REQUIRE(g.n1 <= kPlanMaxN && g.n2 <= kPlanMaxN && g.n3 <= kPlanMaxN, kErrUnsupportedSize,
                 "trajectory plans support at most 512 points per axis");
     const int nb = std::min(nblocks_for(g.nl), kPlanBlocks);
-    hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, st, scratch);
     hipLaunchKernelGGL(k_make_plan_soa, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), W, X,
-                       reinterpret_cast<PlanPt*>(P), scratch);
-    int h = 0;
-    CLR_HIP_CHECK(hipMemcpyAsync(&h, scratch, sizeof(int), hipMemcpyDeviceToHost, st));
-    CLR_HIP_CHECK(hipStreamSynchronize(st));
-    return h;
+                       reinterpret_cast<PlanPt*>(P), bmax);
+    return plan_bound(bmax, nb, st);
 }
 
 void launch_adjoint_coeff(const GatherDims& g, const float* X, const float* divv, float ht, float alpha, float* C,

@@ -98,8 +98,10 @@ void launch_trajectory_rk4(const Dims& d, const float* const v[3], float sigma, 
 // the first stencil node from the point (layout in gather_device.hpp).
 // Returns the per-axis stencil displacement bound D in cells (synchronizes
 // the stream); 1 << 20 when a foot point is not finite.  n <= 512 per axis.
-// `scratch` is one device int.
-int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* scratch, hipStream_t st);
+// `bmax`: kPlanBlocks ints of pinned host memory that the device can write
+// (the blocks' bounds; one launch at a time may use them).
+constexpr int kPlanBlocks = 2048;
+int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* bmax, hipStream_t st);
 // RK2 characteristic through the LDS-staged gather, in three passes:
 //   1. the packed plan of the Euler predictor X̃ = (x − σ·ht·v)/2π into P
 //      (launch_rk2_predictor_plan, which returns its displacement bound);
@@ -110,10 +112,10 @@ int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* scra
 //      (launch_make_plan_soa, which returns the bound of X).
 // The foot points equal those of launch_trajectory_rk2.
 int launch_rk2_predictor_plan(const Dims& d, const float* const v[3], float sigma, float ht, uint32_t* P,
-                              int* scratch, hipStream_t st);
+                              int* bmax, hipStream_t st);
 void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, int dbound, const float* const v[3], float sigma,
                                    float ht, float* W, hipStream_t st);
-int launch_make_plan_soa(const GatherDims& g, const float* W, float* X, uint32_t* P, int* scratch, hipStream_t st);
+int launch_make_plan_soa(const GatherDims& g, const float* W, float* X, uint32_t* P, int* bmax, hipStream_t st);
 // RK4 characteristic the same way: the first stage point (x − σ·ht/2·v)/2π
 // is launch_rk2_predictor_plan with ht/2; each stage gathers v along the
 // previous point's plan (bound <= 4), accumulates the stage sum f and writes
