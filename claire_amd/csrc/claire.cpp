@@ -289,6 +289,21 @@ void SpectralOps::Multiplier3(const SpecParams& sp, const float* const in[3], fl
     }
 }
 
+void SpectralOps::Norm3(const SpecParams& sp, const float* const v[3], double* result) {
+    const Dims& d = m_Opt->domain;
+    hipStream_t st = m_Opt->stream;
+    c32* s[3] = {m_Spec[0].get(), m_Spec[1].get(), m_Spec[2].get()};
+    const int64_t np = m_Plan->x1_norm_partials(3);
+    m_NormPartial.resize(static_cast<size_t>(np));
+    { KernelScope k(m_Opt->prof, "fft_x3_r2c", 3.0 * bytes_x3_r2c(d)); m_Plan->x3_r2c_n(v, s, 3, st); }
+    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2_n(s, 3, -1, st); }
+    {
+        KernelScope k(m_Opt->prof, "fft_x1_norm", 24.0 * d.nlc);
+        m_Plan->x1_norm(s, 3, sp, m_NormPartial.get(), st);
+        launch_sum_partials(m_NormPartial.get(), static_cast<int>(np), result, st);
+    }
+}
+
 void SpectralOps::Project(const SpecParams& sp, float* const b[3]) {
     const Dims& d = m_Opt->domain;
     hipStream_t st = m_Opt->stream;
@@ -355,47 +370,19 @@ int Regularization::ApplyInverse(VecField* Ainvx, const VecField* x, bool applys
 int Regularization::EvaluateFunctional(double* R, const VecField* v) {
     *R = 0.0;
     if (m_Opt->beta[0] == 0.0f) return 0;
-    const int64_t nl = m_Opt->domain.nl;
-    const double hd = m_Opt->GetLebesgueMeasure();
-    if (!m_Work) m_Work.reset(new VecField(m_Opt));
-    float* w[3] = {m_Work->m_X1, m_Work->m_X2, m_Work->m_X3};
-    const int norm = Norm();
-    double acc = 0.0;
-    double dots[Reducer::kSlots];
-    if (norm == kRegH1 || norm == kRegH1SN) {
-        // Σ_i ‖∇v_i‖² (src/RegularizationH1SN.cpp:84-141); the nine products
-        // (and ‖v‖² for H1) are read back together and summed in order
-        for (int c = 0; c < 3; ++c) {
-            const float* vc = c == 0 ? v->m_X1 : (c == 1 ? v->m_X2 : v->m_X3);
-            m_Spec->Grad(w, vc);
-            for (int k = 0; k < 3; ++k) m_Red->DotTo(w[k], w[k], nl, 3 * c + k);
-        }
-        if (norm == kRegH1) m_Red->DotTo(v->m_X1, v->m_X1, 3 * nl, 9);
-        m_Red->Fetch(dots, norm == kRegH1 ? 10 : 9);
-        for (int i = 0; i < 9; ++i) acc += dots[i];
-        if (norm == kRegH1) {
-            // ½·hd·β0·(H1v + β1·L2v), src/RegularizationH1.cpp:140-147
-            *R = 0.5 * hd * m_Opt->beta[0] * (acc + m_Opt->beta[1] * dots[9]);
-        } else {
-            *R = 0.5 * hd * m_Opt->beta[0] * acc;
-        }
-        return 0;
-    }
+    // The norms are folded from the spectrum (FFTPlan3D::x1_norm):
+    //   H1    ½·hd·β0·(Σ_i ‖∇v_i‖² + β1·‖v‖²)  src/RegularizationH1.cpp:140-147
+    //   H1SN  ½·hd·β0·Σ_i ‖∇v_i‖²               src/RegularizationH1SN.cpp:84-141
+    //   H2    ½·hd·β0·Σ_i ‖(Δ + √β1)v_i‖²       src/RegularizationH2.cpp:80-81,128,164-166
+    //   H2SN  ½·hd·β0·Σ_i ‖Δv_i‖²               src/RegularizationH2SN.cpp:163
+    SpecParams sp = Params(kOpRegApply);
+    if (sp.norm == kRegH2) sp.beta1 = std::sqrt(sp.beta1);
     const float* in[3] = {v->m_X1, v->m_X2, v->m_X3};
-    SpecParams sp = Params(norm == kRegH2 ? kOpH2Functional : kOpScaledLaplace);
-    if (norm == kRegH2) {
-        // src/RegularizationH2.cpp:80-81,128: multiplier scale·√β0·(lapik + √β1)
-        sp.beta0 = std::sqrt(m_Opt->beta[0]);
-        sp.beta1 = std::sqrt(m_Opt->beta[1]);
-    }
-    m_Spec->Multiplier3(sp, in, w, 1.0f, nullptr, 0.0f);
-    for (int k = 0; k < 3; ++k) m_Red->DotTo(w[k], w[k], nl, k);
-    m_Red->Fetch(dots, 3);
-    for (int k = 0; k < 3; ++k) acc += dots[k];
-    if (norm == kRegH2)
-        *R = 0.5 * hd * acc;                         // src/RegularizationH2.cpp:164-166
-    else
-        *R = 0.5 * m_Opt->beta[0] * hd * acc;        // src/RegularizationH2SN.cpp:163
+    m_Spec->Norm3(sp, in, m_Red->Slot(0));
+    double sum;
+    m_Red->Fetch(&sum, 1);
+    const double hd = m_Opt->GetLebesgueMeasure();
+    *R = 0.5 * hd * m_Opt->beta[0] * (sum / static_cast<double>(m_Opt->domain.nl));
     return 0;
 }
 

@@ -198,6 +198,7 @@ class Reducer {
     // Device address of the result slots (read by kernels that consume the
     // products without a host round trip).
     const double* Slots() const { return m_Result.get(); }
+    double* Slot(int i) { return m_Result.get() + i; }
 
   private:
     double fetch();
@@ -240,6 +241,9 @@ class SpectralOps {
     // out_d = alpha·F⁻¹(m(k)·F(in_d)) + beta·add_d, d = 0..2
     void Multiplier3(const claire_amd::SpecParams& sp, const float* const in[3], float* const out[3], float alpha,
                      const float* const add[3], float beta);
+    // Launches Σ_x |M v|²·N of a vector field, m² of sp.norm (FFTPlan3D::x1_norm),
+    // into *result (device).
+    void Norm3(const claire_amd::SpecParams& sp, const float* const v[3], double* result);
     // b ← b + F⁻¹[x̂] with the projection of sp.op (kOpProjStokes or
     // kOpProjRelaxed), in place on the three components.
     void Project(const claire_amd::SpecParams& sp, float* const b[3]);
@@ -249,6 +253,7 @@ class SpectralOps {
     const RegOpt* m_Opt;
     std::unique_ptr<claire_amd::FFTPlan3D> m_Plan;
     DeviceArray<c32> m_Spec[3];
+    DeviceArray<double> m_NormPartial;  // block sums of Norm3, allocated on its first call
 };
 
 class Regularization {
@@ -269,9 +274,6 @@ class Regularization {
     const RegOpt* m_Opt;
     SpectralOps* m_Spec;
     Reducer* m_Red;
-    // work field of EvaluateFunctional, allocated on its first call and kept
-    // (no allocation inside the Newton loop)
-    std::unique_ptr<VecField> m_Work;
 };
 
 class RegularizationH1 : public Regularization {

@@ -63,8 +63,6 @@ enum SpecOp : int {
     kOpRegApply = 0,     // first/second variation multiplier
     kOpRegInverse = 1,   // inverse
     kOpRegInvSqrt = 2,   // inverse square root
-    kOpH2Functional = 3, // scale·√β0·(lapik + √β1)
-    kOpScaledLaplace = 4,// scale·lapik
     kOpProjStokes = 5,   // CLAIREStokes::ApplyProjection
     kOpProjRelaxed = 6   // CLAIREDivReg::ApplyProjection
 };

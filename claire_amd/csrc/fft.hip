@@ -310,8 +310,7 @@ __device__ __forceinline__ float spec_multiplier(const SpecParams& p, int w1, in
                 case kRegH1SN: return -p.hd * p.scale * b0 * lapik;
                 default: return p.hd * p.scale * b0 * (lapik * lapik);
             }
-        case kOpRegInverse:
-        case kOpRegInvSqrt: {
+        default: {  // kOpRegInverse, kOpRegInvSqrt
             float regop;
             switch (p.norm) {
                 case kRegH1: regop = b0 * (-lapik + b1); break;
@@ -322,8 +321,6 @@ __device__ __forceinline__ float spec_multiplier(const SpecParams& p, int w1, in
             if (p.op == kOpRegInvSqrt) regop = sqrtf(regop);
             return p.scale / regop;
         }
-        case kOpH2Functional: return p.scale * b0 * (lapik + b1);  // b0, b1 hold √β0, √β1
-        default: return p.scale * lapik;
     }
 }
 
@@ -761,6 +758,83 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(Ptr3 ptr, ColGeom 
 }
 
 // ---------------------------------------------------------------------------
+// Norms of the regularization functionals from the spectrum.  By Parseval
+//   Σ_x |M v|² = (1/N)·Σ_k c(k3)·m(k)²·|v̂(k)|²,
+// with c = 2 for the half spectrum's columns 0 < k3 < n3/2, which stand for
+// their mirror images too, and 1 for the others.  The block holds complete x1
+// columns after the forward pass, so it folds them in FP64 and writes one
+// partial sum instead of a spectrum; no inverse transform, gradient field or
+// dot product is left (objective at 192³ 1570 -> 1132 µs, of which the functional
+// 570 -> about 125; at 64³ 423 -> 282).
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ double norm_factor(const SpecParams& p, double k2) {
+    switch (p.norm) {  // m² without the constants the host applies
+        case kRegH1: return k2 + static_cast<double>(p.beta1);   // ‖∇v‖² + β1·‖v‖²
+        case kRegH1SN: return k2;                                // ‖∇v‖²
+        case kRegH2: {                                           // ‖(Δ + √β1)v‖²
+            const double m = static_cast<double>(p.beta1) - k2;  // β1 holds √β1
+            return m * m;
+        }
+        default: return k2 * k2;                                 // ‖Δv‖²
+    }
+}
+
+template <int N>
+__global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_norm(Ptr3 ptr, ColGeom geo, const c32* __restrict__ tw,
+                                                             SpecParams sp, int n2, int n3, int nh,
+                                                             double* __restrict__ partial) {
+    using G = Geo<N>;
+    __shared__ c32 s[G::LDS_ELEMS];
+    using LF = typename Plan<N>::Fwd;
+    constexpr int V = G::V, T = G::T, R0 = First<LF>::value, RL = Last<LF>::value;
+    const int c = threadIdx.x % G::B;
+    const int t = threadIdx.x / G::B;
+    const int64_t cg = static_cast<int64_t>(blockIdx.x) * G::B + c;
+    const bool valid = cg < geo.ncols;
+    const int64_t base = valid ? cg : 0;
+    const int k2 = static_cast<int>(static_cast<uint32_t>(cg) / static_cast<uint32_t>(nh));
+    const int k3 = static_cast<int>(cg) - k2 * nh;
+    const int w2 = wavenum(k2, n2), w3 = wavenum(k3, n3);
+    const uint32_t es8 = static_cast<uint32_t>(geo.estride) * 8u;
+    const uint32_t lane = static_cast<uint32_t>(base) * 8u + static_cast<uint32_t>(t) * es8;
+    const spec_rsrc_t r_in = spec_rsrc(ptr.in[blockIdx.y], geo.ncols * N);
+    c32 v[V];
+#pragma unroll
+    for (int q = 0; q < V / R0; ++q)
+#pragma unroll
+        for (int r = 0; r < R0; ++r) {
+            const c32 x = bload_c(r_in, lane, static_cast<uint32_t>(T * q + r * (N / R0)) * es8);
+            v[q * R0 + r] = valid ? x : c32{0.f, 0.f};
+        }
+    fft_regs<N, -1>(v, s, ColLayout{G::LD}, c, t, tw);
+    double acc = 0.0;
+#pragma unroll
+    for (int q = 0; q < V / RL; ++q) {
+        const int j = t + T * q;
+#pragma unroll
+        for (int r = 0; r < RL; ++r) {
+            const int w1 = wavenum(j + r * (N / RL), N);
+            const double x = static_cast<double>(v[q * RL + r].x), y = static_cast<double>(v[q * RL + r].y);
+            acc += norm_factor(sp, static_cast<double>(w1 * w1 + w2 * w2 + w3 * w3)) * (x * x + y * y);
+        }
+    }
+    if (k3 != 0 && 2 * k3 != n3) acc *= 2.0;
+    // block sum in a fixed order (the thread count need not be a multiple of
+    // a wave): one value per thread through LDS, folded by the first wave
+    static_assert(G::LDS_ELEMS >= G::THREADS, "one double per thread must fit the exchange buffer");
+    double* sh = reinterpret_cast<double*>(s);
+    __syncthreads();
+    sh[threadIdx.x] = acc;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+    double sum = 0.0;
+    for (int i = threadIdx.x; i < G::THREADS; i += 64) sum += sh[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    if (threadIdx.x == 0) partial[static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x] = sum;
+}
+
+// ---------------------------------------------------------------------------
 // Host-side dispatch on the (runtime) transform length.
 // ---------------------------------------------------------------------------
 template <template <int> class F, class... A>
@@ -851,6 +925,23 @@ struct X1Fused {
                 hipLaunchKernelGGL((k_x1_fused<N, kFuseDiv>), grid, dim3(G::THREADS), 0, st, p, geo, tw, sp, n2, n3, nh);
                 break;
         }
+    }
+};
+
+template <int N>
+struct X1Blocks {
+    static void go(int64_t ncols, int64_t* blocks) { *blocks = (ncols + Geo<N>::B - 1) / Geo<N>::B; }
+};
+
+template <int N>
+struct X1Norm {
+    static void go(Ptr3 p, ColGeom geo, const c32* tw, SpecParams sp, int n2, int n3, int nh, int ncomp, double* partial,
+                   hipStream_t st) {
+        using G = Geo<N>;
+        CLR_REQUIRE(geo.ncols * N * 8 < (int64_t(1) << 31), kErrInvalidArgument,
+                    "spectrum field too large for 32-bit buffer offsets");
+        const dim3 grid(static_cast<unsigned>((geo.ncols + G::B - 1) / G::B), ncomp);
+        hipLaunchKernelGGL(k_x1_norm<N>, grid, dim3(G::THREADS), 0, st, p, geo, tw, sp, n2, n3, nh, partial);
     }
 };
 
@@ -976,6 +1067,20 @@ void FFTPlan3D::x1_multiplier(const c32* const in[3], c32* const out[3], int nco
     }
     dispatch_n<X1Fused>(dims.n[0], static_cast<int>(kFuseMult), p, geom_x1(dims), tw[0], sp, dims.n[1], dims.n[2],
                         dims.nh, ncomp, st);
+}
+
+int64_t FFTPlan3D::x1_norm_partials(int ncomp) const {
+    int64_t blocks = 0;
+    dispatch_n<X1Blocks>(dims.n[0], geom_x1(dims).ncols, &blocks);
+    return blocks * ncomp;
+}
+
+void FFTPlan3D::x1_norm(const c32* const in[3], int ncomp, const SpecParams& sp, double* partial,
+                        hipStream_t st) const {
+    CLR_REQUIRE(ncomp >= 1 && ncomp <= 3, kErrInvalidArgument, "1 to 3 fields per FFT pass");
+    Ptr3 p{};
+    for (int d = 0; d < ncomp; ++d) p.in[d] = in[d];
+    dispatch_n<X1Norm>(dims.n[0], p, geom_x1(dims), tw[0], sp, dims.n[1], dims.n[2], dims.nh, ncomp, partial, st);
 }
 
 void FFTPlan3D::x1_grad(const c32* in, c32* const out[3], hipStream_t st) const {

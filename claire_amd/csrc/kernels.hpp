@@ -49,6 +49,12 @@ class FFTPlan3D {
     void x1_multiplier(const c32* const in[3], c32* const out[3], int ncomp, const SpecParams& sp, hipStream_t st) const;
     void x1_grad(const c32* in, c32* const out[3], hipStream_t st) const;
     void x1_div(const c32* const in[3], c32* out, hipStream_t st) const;
+    // Forward x1 pass that ends in a sum: per block Σ c(k3)·m(k)²·|x̂(k)|² over
+    // its columns, m² the regularization norm's (sp.norm; sp.beta1 = β1 for H1,
+    // √β1 for H2), so that the sum of all x1_norm_partials(ncomp) values over N
+    // is Σ_x |M x|² of the ncomp fields.
+    void x1_norm(const c32* const in[3], int ncomp, const SpecParams& sp, double* partial, hipStream_t st) const;
+    int64_t x1_norm_partials(int ncomp) const;
     // Projection of a vector field (sp.op kOpProjStokes or kOpProjRelaxed):
     // x̂_i = g_i·scale·m·(g·b̂) in place of the three spectra.
     void x1_project(c32* const data[3], const SpecParams& sp, hipStream_t st) const;
@@ -257,6 +263,8 @@ void launch_sqdist(const float* a, const float* b, int64_t n, double* partial, d
 void launch_min(const float* a, int64_t n, double* partial, double* result, hipStream_t st);
 void launch_max(const float* a, int64_t n, double* partial, double* result, hipStream_t st);
 void launch_sum(const float* a, int64_t n, double* partial, double* result, hipStream_t st);
+// result = Σ partial[0..np), in a fixed order
+void launch_sum_partials(const double* partial, int np, double* result, hipStream_t st);
 
 // ---------------------------------------------------------------------------
 // Explicit RK2 transport stages (rk2.hip); each follows a spectral grad or

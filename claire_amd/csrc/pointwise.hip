@@ -380,5 +380,8 @@ void launch_max(const float* a, int64_t n, double* partial, double* result, hipS
 void launch_sum(const float* a, int64_t n, double* partial, double* result, hipStream_t st) {
     reduce<kRedSum>(a, nullptr, n, partial, result, st);
 }
+void launch_sum_partials(const double* partial, int np, double* result, hipStream_t st) {
+    hipLaunchKernelGGL(k_reduce_final<kRedSum>, dim3(1), dim3(kThreads), 0, st, partial, np, result);
+}
 
 }  // namespace claire_amd
