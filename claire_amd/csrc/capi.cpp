@@ -512,8 +512,8 @@ int clr_trajectory(clr_ctx* ctx, int flag, float* X_out) {
         const std::string f = flag == CLR_STATE ? "state" : (flag == CLR_ADJOINT ? "adjoint" : "?");
         if (f == "?") throw Error(claire_amd::kErrInvalidArgument, "flag wrong");
         c.EnsureTrajectories();
-        CLR_HIP_CHECK(hipMemcpyAsync(X_out, c.SL()->Trajectory(f), 3 * c.Opt().domain.nl * sizeof(float),
-                                     hipMemcpyDeviceToDevice, c.Opt().stream));
+        c.SL()->GetTrajectory(f, X_out);
+        check_hip_launch();
     });
 }
 

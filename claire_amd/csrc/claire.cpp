@@ -419,7 +419,7 @@ int Regularization::GetExtremeEigValsInvOp(ScalarType& emin, ScalarType& emax) {
 // ---------------------------------------------------------------------------
 // SemiLagrangian (src/SemiLagrangian.cpp)
 // ---------------------------------------------------------------------------
-SemiLagrangian::SemiLagrangian(const RegOpt* opt) : m_Opt(opt), m_PlanMax(kPlanBlocks) {}
+SemiLagrangian::SemiLagrangian(const RegOpt* opt) : m_Opt(opt), m_PlanMax(3 * kPlanBlocks) {}
 
 int SemiLagrangian::Which(const std::string& flag) const {
     if (flag == "state") return 0;
@@ -427,90 +427,83 @@ int SemiLagrangian::Which(const std::string& flag) const {
     throw Error(kErrInvalidArgument, "flag wrong");  // src/SemiLagrangian.cpp:221-223
 }
 
+bool SemiLagrangian::SetVelocity(const float* v, VecField* dst) {
+    const size_t n = 3 * static_cast<size_t>(m_Opt->domain.nl);
+    m_P[0].resize(n);
+    // bytes: v read (12), copied (12) and the plan written (12) per point
+    KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 36.0 * m_Opt->domain.nl);
+    const VelocityBounds b = launch_set_velocity(m_Opt->domain, v, dst->m_X1, PredictorStep(), m_P[0].get(),
+                                                 m_PlanMax.get(), m_Opt->stream);
+    m_PredBound[0] = b.dbound[0];
+    m_PredBound[1] = b.dbound[1];
+    m_PredOrder = m_Opt->rkorder;
+    m_PredInPlan = true;
+    m_Valid[0] = false;  // its plan is gone
+    return b.zero;
+}
+
 int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag) {
     const int w = Which(flag);
-    m_X[w].resize(3 * static_cast<size_t>(m_Opt->domain.nl));
+    CLR_REQUIRE(m_Opt->rkorder == 2 || m_Opt->rkorder == 4, kErrInvalidArgument, "rk order must be 2 or 4");
+    if (m_PredOrder != m_Opt->rkorder) {
+        // the velocity was set before the scheme or the time integrator was
+        VecField same(m_Opt, v->m_X1);
+        SetVelocity(v->m_X1, &same);
+    }
+    const int64_t nl = m_Opt->domain.nl;
+    const size_t n = 3 * static_cast<size_t>(nl);
+    m_X[w].resize(n);
+    m_P[w].resize(n);
+    float* const X = m_X[w].get();
+    uint32_t* const P = m_P[w].get();
+    const GatherDims g = gather_dims(m_Opt->domain);
     const float* vc[3] = {v->m_X1, v->m_X2, v->m_X3};
     const float sigma = w == 0 ? 1.0f : -1.0f;
+    const float ht = m_Opt->GetTimeStepSize();
+    const int dmax = lds_gather_max_displacement();
+    int db = m_PredBound[w];
+    if (db <= dmax && !(w == 0 && m_PredInPlan)) {
+        // bytes: v read (12) + plan written (12) per point
+        KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 24.0 * nl);
+        launch_predictor_plan(m_Opt->domain, vc, sigma, PredictorStep(), P, m_Opt->stream);
+    }
+    if (w == 0) m_PredInPlan = false;
     if (m_Opt->rkorder == 4) {
-        const int64_t nl = m_Opt->domain.nl;
-        const GatherDims g = gather_dims(m_Opt->domain);
-        const float ht = m_Opt->GetTimeStepSize();
-        m_F.resize(3 * static_cast<size_t>(nl));
-        m_P[w].resize(3 * static_cast<size_t>(nl));
-        const int dmax = lds_gather_max_displacement();
-        int db = -1;
-        {
-            KernelScope k(m_Opt->prof, "gather_traj_rk4_plan", 24.0 * nl);
-            db = launch_rk2_predictor_plan(m_Opt->domain, vc, sigma, 0.5f * ht, m_P[w].get(), m_PlanMax.get(),
-                                           m_Opt->stream);
-        }
-        if (vc[1] - vc[0] == nl && vc[2] - vc[1] == nl) {
-            m_W.resize(3 * static_cast<size_t>(nl));
-            m_F2.resize(3 * static_cast<size_t>(nl));
-            // stage sums: stage 1 writes f into m_F, stage 2 reads m_F and
-            // writes m_F2, stage 3 reads m_F2
-            float* const fbuf[4] = {nullptr, m_F.get(), m_F2.get(), nullptr};
-            for (int stage = 1; stage <= 3 && db >= 0 && db <= dmax; ++stage) {
+        m_F.resize(n);
+        m_F2.resize(n);
+        float* const fbuf[4] = {nullptr, m_F.get(), m_F2.get(), nullptr};
+        for (int stage = 1; stage <= 3; ++stage) {
+            if (db <= dmax) {
                 {
                     // 3 × (plan 12 + gathered v 4 + aux 4 + next point 4 (+ f 4)) per point
                     KernelScope k(m_Opt->prof, "gather_traj_rk4", (stage < 3 ? 84.0 : 72.0) * nl);
-                    launch_lds_traj_rk4_stage(stage, m_Opt->domain, m_P[w].get(), db, vc, sigma, ht,
-                                              fbuf[stage - 1], fbuf[stage], m_W.get(), m_Opt->stream);
+                    launch_lds_traj_rk4_stage(stage, m_Opt->domain, P, db, vc, sigma, ht, fbuf[stage - 1],
+                                              fbuf[stage], X, m_Opt->stream);
                 }
-                // bytes: point components read (12) + plan (12) (+ X interleaved (12) at the end)
-                KernelScope k(m_Opt->prof, "gather_plan", (stage < 3 ? 24.0 : 36.0) * nl);
-                db = launch_make_plan_soa(g, m_W.get(), stage == 3 ? m_X[w].get() : nullptr, m_P[w].get(),
-                                          m_PlanMax.get(), m_Opt->stream);
-                if (stage == 3) {
-                    m_D[w] = db;
-                    m_Valid[w] = true;
-                    return 0;
-                }
+                if (stage == 3) break;
+                // bytes: point read (12) + plan (12)
+                KernelScope k(m_Opt->prof, "gather_plan", 24.0 * nl);
+                db = launch_make_plan(g, X, P, m_PlanMax.get(), m_Opt->stream);
+            } else {
+                // this stage's point is out of the LDS window, and so, nearly
+                // always, are the later stages' (their plans are not formed)
+                KernelScope k(m_Opt->prof, "gather_traj_rk4", 48.0 * nl);
+                launch_trajectory_rk4_stage(stage, m_Opt->domain, vc, sigma, ht, X, fbuf[stage - 1], fbuf[stage],
+                                            m_Opt->stream);
             }
         }
-        // bytes: v read (12), v gathered 3× (36), f and X written, read and
-        // rewritten (12 + 12 + 24 + 24 + 12 + 12) per point
-        KernelScope k(m_Opt->prof, "gather_traj_rk4", 144.0 * m_Opt->domain.nl);
-        launch_trajectory_rk4(m_Opt->domain, vc, sigma, m_Opt->GetTimeStepSize(), m_X[w].get(), m_F.get(),
-                              m_Opt->stream);
+    } else if (db <= dmax) {
+        // 3 × (plan 12 + gathered v 4 + v at the point 4 + X component 4) per point
+        KernelScope k(m_Opt->prof, "gather_traj_rk2", 72.0 * nl);
+        launch_lds_traj_rk2_corrector(m_Opt->domain, P, db, vc, sigma, ht, X, m_Opt->stream);
     } else {
-        CLR_REQUIRE(m_Opt->rkorder == 2, kErrInvalidArgument, "rk order must be 2 or 4");
-        const int64_t nl = m_Opt->domain.nl;
-        const GatherDims g = gather_dims(m_Opt->domain);
-        m_P[w].resize(3 * static_cast<size_t>(nl));
-        int dpred = -1;
-        {
-            // the Euler predictor's plan: v read (12) + plan written (12) per point
-            KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 24.0 * nl);
-            dpred = launch_rk2_predictor_plan(m_Opt->domain, vc, sigma, m_Opt->GetTimeStepSize(), m_P[w].get(),
-                                              m_PlanMax.get(), m_Opt->stream);
-        }
-        if (dpred >= 0 && dpred <= lds_gather_max_displacement() && vc[1] - vc[0] == nl && vc[2] - vc[1] == nl) {
-            m_W.resize(3 * static_cast<size_t>(nl));
-            {
-                // 3 × (plan 12 + gathered v 4 + v at the point 4 + X component 4) per point
-                KernelScope k(m_Opt->prof, "gather_traj_rk2", 72.0 * nl);
-                launch_lds_traj_rk2_corrector(m_Opt->domain, m_P[w].get(), dpred, vc, sigma,
-                                              m_Opt->GetTimeStepSize(), m_W.get(), m_Opt->stream);
-            }
-            // bytes: X components read (12) + X interleaved (12) + plan (12) per point
-            KernelScope k(m_Opt->prof, "gather_plan", 36.0 * nl);
-            m_D[w] = launch_make_plan_soa(g, m_W.get(), m_X[w].get(), m_P[w].get(), m_PlanMax.get(), m_Opt->stream);
-            m_Valid[w] = true;
-            return 0;
-        }
         // bytes: v read (12) + v gathered (12) + X written (12) per point
         KernelScope k(m_Opt->prof, "gather_traj_rk2", 36.0 * nl);
-        launch_trajectory_rk2(m_Opt->domain, vc, sigma, m_Opt->GetTimeStepSize(), m_X[w].get(), m_Opt->stream);
+        launch_trajectory_rk2(m_Opt->domain, vc, sigma, ht, X, m_Opt->stream);
     }
-    m_P[w].resize(3 * static_cast<size_t>(m_Opt->domain.nl));
-    {
-        // bytes: X read (12) + packed plan written (12) per point
-        KernelScope k(m_Opt->prof, "gather_plan", 24.0 * m_Opt->domain.nl);
-        m_D[w] = launch_make_plan(gather_dims(m_Opt->domain), m_X[w].get(), m_P[w].get(), m_PlanMax.get(),
-                                  m_Opt->stream);
-    }
+    // bytes: X read (12) + packed plan written (12) per point
+    KernelScope k(m_Opt->prof, "gather_plan", 24.0 * nl);
+    m_D[w] = launch_make_plan(g, X, P, m_PlanMax.get(), m_Opt->stream);
     m_Valid[w] = true;
     return 0;
 }
@@ -523,10 +516,10 @@ TrajectoryPlan SemiLagrangian::Plan(const std::string& flag) const {
 
 bool SemiLagrangian::HasTrajectory(const std::string& flag) const { return m_Valid[Which(flag)]; }
 
-const float* SemiLagrangian::Trajectory(const std::string& flag) const {
+void SemiLagrangian::GetTrajectory(const std::string& flag, float* out) const {
     const int w = Which(flag);
     CLR_REQUIRE(m_Valid[w], kErrState, "trajectory '" + flag + "' has not been computed");
-    return m_X[w].get();
+    launch_interleave(m_Opt->domain.nl, m_X[w].get(), out, m_Opt->stream);
 }
 
 void SemiLagrangian::Gather(float* xo, const float* xi, const std::string& flag) {
@@ -643,8 +636,7 @@ size_t CLAIRE::DeviceBytes() const {
                           nt * 3 * nl + nt * nl + nt * nl + nl + 2 * 3 * nl;
     const size_t halves = m_Opt.precision == 1 ? (2 * nt + 1) * 3 * nl : 0;
     const size_t scales = m_Opt.precision == 1 ? (2 * nt + 1) * 3 * static_cast<size_t>(bfp16_blocks(nl)) : 0;
-    // the corrector / stage-point output, plus the two RK4 stage sums
-    const size_t rk4 = 3 * nl + (m_Opt.rkorder == 4 ? 6 * nl : 0);
+    const size_t rk4 = m_Opt.rkorder == 4 ? 6 * nl : 0;  // the two RK4 stage sums
     const size_t cont = m_Opt.pdetype == 0 ? nl : 0;      // continuity-equation coefficient
     const size_t rk2 = m_Opt.pdesolver == 0 ? 6 * nl : 0;  // RK2 integrator work
     return (floats + rk4 + cont + rk2 + scales) * 4 + halves * 2 + 3 * static_cast<size_t>(m_Opt.domain.nlc) * 8;
@@ -653,12 +645,18 @@ size_t CLAIRE::DeviceBytes() const {
 void CLAIRE::RequireVelocity() const { CLR_REQUIRE(m_HaveVelocity, kErrState, "velocity field not set"); }
 
 int CLAIRE::SetControlVariable(const float* v) {
-    m_VelocityField->SetComponents(v);
+    CLR_REQUIRE(v != nullptr, kErrInvalidArgument, "null input vector");
     m_HaveVelocity = true;
     m_TrajValid = m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
     ++m_GraphEpoch;
     // CLAIREBase::IsVelocityZero (src/CLAIREBase.cpp:578-605): ∞-norm == 0
-    m_VelocityIsZero = m_Red->AbsMax(m_VelocityField->m_X1, 3 * m_Opt.domain.nl) == 0.0;
+    if (UsesTrajectories()) {
+        m_VelocityIsZero = m_SL->SetVelocity(v, m_VelocityField.get());
+    } else {
+        m_SL->ForgetVelocity();
+        m_VelocityField->SetComponents(v);
+        m_VelocityIsZero = m_Red->AbsMax(m_VelocityField->m_X1, 3 * m_Opt.domain.nl) == 0.0;
+    }
     return 0;
 }
 
@@ -723,7 +721,7 @@ int CLAIRE::SolveStateEquation() {
     const int64_t nl = m_Opt.domain.nl;
     const int nt = m_Opt.nt;
     // the SL solves and the continuity equation need the trajectories
-    if (m_Opt.pdesolver == 2 || m_Opt.pdetype == 0) EnsureTrajectories();
+    if (UsesTrajectories()) EnsureTrajectories();
     float* m = m_State.get();
     launch_copy(m_TemplateImage.get(), m, nl, m_Opt.stream);  // m^0 = mT (src/CLAIRE.cpp:1896)
     if (m_VelocityIsZero) {

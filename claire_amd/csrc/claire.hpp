@@ -300,6 +300,13 @@ class RegularizationH2SN : public Regularization {
 class SemiLagrangian {
   public:
     explicit SemiLagrangian(const RegOpt* opt);
+    // Takes over a new velocity: copies it to `dst`, forms the state
+    // trajectory's predictor plan and the predictors' displacement bounds in the
+    // same pass, and returns whether it is zero everywhere.  Trajectories
+    // computed from `dst` afterwards use them.
+    bool SetVelocity(const float* v, VecField* dst);
+    // The velocity field changed without SetVelocity.
+    void ForgetVelocity() { m_PredOrder = 0; }
     // flag "state" (σ = +1) or "adjoint" (σ = −1)
     int ComputeTrajectory(const VecField* v, const std::string& flag);
     int Interpolate(float* xo, const float* xi, const std::string& flag);
@@ -307,8 +314,9 @@ class SemiLagrangian {
     // Out-of-place gathers along a trajectory (no aliasing allowed).
     void Gather(float* xo, const float* xi, const std::string& flag);
     void Gather3(const float* const in[3], float* const out[3], const std::string& flag);
-    // Trajectory X (3 floats per point, normalized by 2π; the reference's m_X)
-    const float* Trajectory(const std::string& flag) const;
+    // Trajectory X into out (3 floats per point, normalized by 2π; the
+    // reference's m_X)
+    void GetTrajectory(const std::string& flag, float* out) const;
     // Interpolation plan of the trajectory (Interp3_Plan after scatter):
     // packed foot points (3 words per point), the raw foot points and the
     // per-axis stencil displacement bound in cells.  Gathers along it use the
@@ -321,13 +329,20 @@ class SemiLagrangian {
   private:
     int Which(const std::string& flag) const;
     const RegOpt* m_Opt;
-    DeviceArray<float> m_X[2];
+    float PredictorStep() const { return (m_Opt->rkorder == 4 ? 0.5f : 1.0f) * m_Opt->GetTimeStepSize(); }
+    DeviceArray<float> m_X[2];  // foot points, one component per field
     DeviceArray<uint32_t> m_P[2];
-    DeviceArray<float> m_F;   // RK4 stage sum f (m_WorkVecField2 of the reference)
-    DeviceArray<float> m_F2;  // RK4 stage sum after stage 2 (LDS path; kept apart from m_F)
-    DeviceArray<float> m_W;  // RK2 corrector output, one component per field (LDS path)
+    // RK4 stage sums f (m_WorkVecField2 of the reference): stage 1 writes m_F,
+    // stage 2 reads it and writes m_F2, which stage 3 reads (no LDS launch
+    // updates an operand in place)
+    DeviceArray<float> m_F, m_F2;
     DeviceArray<float> m_Tmp;  // in-place interpolation (the reference's ghost copy), kept between calls
     PinnedArray<int> m_PlanMax;  // the plan kernels' block maxima (displacement bounds)
+    // What SetVelocity found, for the characteristic scheme m_PredOrder (0: not
+    // known); m_PredInPlan while m_P[0] still holds the predictor's plan.
+    int m_PredOrder = 0;
+    int m_PredBound[2] = {0, 0};
+    bool m_PredInPlan = false;
     bool m_Valid[2] = {false, false};
     int m_D[2] = {0, 0};
 };
@@ -420,6 +435,9 @@ class CLAIRE {
 
   private:
     void RequireVelocity() const;
+    // Whether the selected solvers move along trajectories (the SL solves and
+    // the continuity equation).
+    bool UsesTrajectories() const { return m_Opt.pdesolver == 2 || m_Opt.pdetype == 0; }
     void EnsureStateGradients();
     void EnsureGradientsAtStateTrajectory();
     void IncStateCore(const VecField* vt, float* lt0_out, bool half);

@@ -1027,16 +1027,16 @@ void launch_plan_adjoint_coeff(const TrajectoryPlan& tp, const GatherDims& g, co
 }
 
 void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, int dbound, const float* const v[3], float sigma,
-                                   float ht, float* W, hipStream_t st) {
+                                   float ht, float* X, hipStream_t st) {
     const GatherDims g = gather_dims(d);
     const int64_t vz = v[1] - v[0];
     CLR_REQUIRE(v[2] - v[1] == vz && vz == g.nl, kErrInvalidArgument, "velocity components must be contiguous");
-    EpiTrajRk2 e{v[0], W, g.nl, d.hx[0], d.hx[1], d.hx[2], sigma * (0.5f * ht), 0};
+    EpiTrajRk2 e{v[0], X, g.nl, d.hx[0], d.hx[1], d.hx[2], sigma * (0.5f * ht), 0};
     dispatch(dbound, g, P, v[0], vz, 3, e, st);
 }
 
 void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, int dbound, const float* const v[3],
-                               float sigma, float ht, const float* Fin, float* Fout, float* W, hipStream_t st) {
+                               float sigma, float ht, const float* Fin, float* Fout, float* X, hipStream_t st) {
     const GatherDims g = gather_dims(d);
     const int64_t vz = v[1] - v[0];
     CLR_REQUIRE(v[2] - v[1] == vz && vz == g.nl, kErrInvalidArgument, "velocity components must be contiguous");
@@ -1049,15 +1049,15 @@ void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, int 
     const double s6 = static_cast<double>(sigma) * (static_cast<double>(ht) / 6.0);
     switch (stage) {
         case 1: {
-            EpiTrajRk4<1> e{v[0], W, Fout, g.nl, hx[0], hx[1], hx[2], sigma * hthalf, s6, 0};
+            EpiTrajRk4<1> e{v[0], X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * hthalf, s6, 0};
             return dispatch(dbound, g, P, v[0], vz, 3, e, st);
         }
         case 2: {
-            EpiTrajRk4<2> e{Fin, W, Fout, g.nl, hx[0], hx[1], hx[2], sigma * ht, s6, 0};
+            EpiTrajRk4<2> e{Fin, X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * ht, s6, 0};
             return dispatch(dbound, g, P, v[0], vz, 3, e, st);
         }
         case 3: {
-            EpiTrajRk4<3> e{Fin, W, W, g.nl, hx[0], hx[1], hx[2], 0.0f, s6, 0};  // no second output
+            EpiTrajRk4<3> e{Fin, X, X, g.nl, hx[0], hx[1], hx[2], 0.0f, s6, 0};  // no second output
             return dispatch(dbound, g, P, v[0], vz, 3, e, st);
         }
         default:

@@ -67,6 +67,13 @@ __device__ __forceinline__ void load_q3(const float* X, int64_t i, float q[3]) {
     q[2] = X[3 * i + 2];
 }
 
+// Points of a trajectory: component d of point i at X[d·nl + i].
+__device__ __forceinline__ void load_point(const float* X, int64_t nl, int64_t i, float q[3]) {
+    q[0] = X[i];
+    q[1] = X[nl + i];
+    q[2] = X[2 * nl + i];
+}
+
 __global__ __launch_bounds__(kThreads) void k_gather1(GatherDims g, HH hh, const float* __restrict__ f,
                                                       const float* __restrict__ X, float* __restrict__ out, int nblocks) {
     const int64_t i = point_index(nblocks);
@@ -85,21 +92,6 @@ struct P3 {
     const float* in[3];
     float* out[3];
 };
-
-__global__ __launch_bounds__(kThreads) void k_gather3(GatherDims g, HH hh, P3 p, const float* __restrict__ X,
-                                                      int nblocks) {
-    const int64_t i = point_index(nblocks);
-    if (i >= g.nl) return;
-    float q[3];
-    load_q3(X, i, q);
-    Stencil S;
-    setup_stencil(q, g, hh.h, S);
-    float r[3];
-    eval_stencil<3>(p.in, S, g, r);
-    p.out[0][i] = r[0];
-    p.out[1][i] = r[1];
-    p.out[2][i] = r[2];
-}
 
 // SemiLagrangian::ComputeTrajectoryRK2 (src/SemiLagrangian.cpp:192-288)
 // with the Euler predictor kept in registers.
@@ -131,7 +123,7 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk2(GatherDims g, HH hh, Traj
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         const float t = x[d] - tp.shth * (vx[d] + vl[d]);
-        X[3 * i + d] = static_cast<float>(over_2pi(static_cast<double>(t)));
+        X[d * g.nl + i] = static_cast<float>(over_2pi(static_cast<double>(t)));
     }
 }
 
@@ -141,8 +133,9 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk2(GatherDims g, HH hh, Traj
 //            X² = (x − σ·ht/2·v(X¹))/2π;
 //   STAGE 2: f += 2·v(X²), X³ = (x − σ·ht·v(X²))/2π;
 //   STAGE 3: f += v(X³), X = (x − σ·(ht/6)·f)/2π.
-// f (3 floats per point, interleaved like X) and the stage points live in F
-// and X between launches.  Precision follows the reference: f += 2.0·vX in
+// f and the stage points live in F and X between launches, per component
+// (stages may come from here or from the LDS-staged gathers, whichever the
+// displacement of the point they read allows).  Precision follows the reference: f += 2.0·vX in
 // double, the last update and every division by 2π in double.
 struct Rk4Params {
     float hx[3];
@@ -161,7 +154,7 @@ __device__ __forceinline__ void grid_point(const GatherDims& g, const float hx[3
 
 template <int STAGE>
 __global__ __launch_bounds__(kThreads) void k_traj_rk4(GatherDims g, HH hh, Rk4Params tp, P3 v,
-                                                       float* __restrict__ X, float* __restrict__ F, int nblocks) {
+                                                       float* __restrict__ X, const float* Fin, float* Fout, int nblocks) {
     const int64_t i = point_index(nblocks);
     if (i >= g.nl) return;
     float x[3];
@@ -175,7 +168,7 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk4(GatherDims g, HH hh, Rk4P
             q[d] = static_cast<float>(over_2pi(static_cast<double>(t)));
         }
     } else {
-        load_q3(X, i, q);
+        load_point(X, g.nl, i, q);
     }
     Stencil S;
     setup_stencil(q, g, hh.h, S);
@@ -184,28 +177,35 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk4(GatherDims g, HH hh, Rk4P
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         if constexpr (STAGE == 1) {
-            F[3 * i + d] = static_cast<float>(static_cast<double>(vl[d]) + 2.0 * static_cast<double>(vx[d]));
+            Fout[d * g.nl + i] = static_cast<float>(static_cast<double>(vl[d]) + 2.0 * static_cast<double>(vx[d]));
             const float t = x[d] - tp.shth * vx[d];
-            X[3 * i + d] = static_cast<float>(over_2pi(static_cast<double>(t)));
+            X[d * g.nl + i] = static_cast<float>(over_2pi(static_cast<double>(t)));
         } else if constexpr (STAGE == 2) {
-            F[3 * i + d] = static_cast<float>(static_cast<double>(F[3 * i + d]) + 2.0 * static_cast<double>(vx[d]));
+            Fout[d * g.nl + i] = static_cast<float>(static_cast<double>(Fin[d * g.nl + i]) + 2.0 * static_cast<double>(vx[d]));
             const float t = x[d] - tp.sht * vx[d];
-            X[3 * i + d] = static_cast<float>(over_2pi(static_cast<double>(t)));
+            X[d * g.nl + i] = static_cast<float>(over_2pi(static_cast<double>(t)));
         } else {
-            const float f = F[3 * i + d] + vx[d];
-            X[3 * i + d] = static_cast<float>(over_2pi(static_cast<double>(x[d]) - tp.s6 * static_cast<double>(f)));
+            const float f = Fin[d * g.nl + i] + vx[d];
+            X[d * g.nl + i] = static_cast<float>(over_2pi(static_cast<double>(x[d]) - tp.s6 * static_cast<double>(f)));
         }
     }
 }
 
-// Block maximum of `need` into bmax[blockIdx.x].
-__device__ __forceinline__ void block_max_to(int need, int* bmax) {
-    __shared__ int sh[kThreads / 64];
+// Block maxima of K values into bmax[k·kPlanBlocks + blockIdx.x].
+template <int K>
+__device__ __forceinline__ void block_max_to(int (&v)[K], int* bmax) {
+    __shared__ int sh[K][kThreads / 64];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) need = max(need, __shfl_xor(need, o, 64));
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = need;
+    for (int k = 0; k < K; ++k) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[k] = max(v[k], __shfl_xor(v[k], o, 64));
+        if ((threadIdx.x & 63) == 0) sh[k][threadIdx.x >> 6] = v[k];
+    }
     __syncthreads();
-    if (threadIdx.x == 0) bmax[blockIdx.x] = max(max(sh[0], sh[1]), max(sh[2], sh[3]));
+    if (threadIdx.x < K) {
+        const int* m = sh[threadIdx.x];
+        bmax[threadIdx.x * kPlanBlocks + blockIdx.x] = max(max(m[0], m[1]), max(m[2], m[3]));
+    }
 }
 
 // Encodes the three axes of foot point q at grid index idx; returns the
@@ -245,64 +245,72 @@ static_assert(kPlanBlocks >= 1 && kThreads == 256, "block_max_to folds four wave
 
 __global__ __launch_bounds__(kThreads) void k_make_plan(GatherDims g, HH hh, const float* __restrict__ X,
                                                         PlanPt* __restrict__ P, int* __restrict__ bmax) {
-    int need = 0;
+    int need[1] = {0};
     const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
     const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     GridWalk gw(g, i0, stride);
     for (int64_t i = i0; i < g.nl; i += stride, gw.advance(g)) {
         float q[3];
-        load_q3(X, i, q);
+        load_point(X, g.nl, i, q);
         PlanPt pt;
-        need = max(need, encode_point(g, hh, q, gw.idx, pt));
+        need[0] = max(need[0], encode_point(g, hh, q, gw.idx, pt));
         P[i] = pt;
     }
     block_max_to(need, bmax);
 }
 
-// Plan of the RK2 Euler predictor X̃ = (x − σ·ht·v)/2π, with the same float
-// and double steps as k_traj_rk2 (bounded grid, like k_make_plan).
-__global__ __launch_bounds__(kThreads) void k_predictor_plan(GatherDims g, HH hh, TrajParams tp, P3 v,
+// Plan of the Euler predictor X̃ = (x − σ·ht·v)/2π, with the same float and
+// double steps as k_traj_rk2 (bounded grid, like k_make_plan).
+//   SETV = false: the plan alone, its bound known already.
+//   SETV = true:  the first pass over a new velocity, which it copies to `vout`
+//                 (unless that is where it lies): the predictor's plan for σ and
+//                 the bounds for σ and −σ, which differ where the extremes of v
+//                 do, and whether any |v| > 0.  In place of a copy, a reduction
+//                 over v and a plan launch per direction, each with a wait.
+// With the foot points kept per component (no interleaved copy beside the plan),
+// set velocity + both trajectories + one gather went from 187 to 134 µs at 64³,
+// 342 to 285 at 128³, 1602 to 1451 at 256³ and 12.5 to 11.5 ms at 512³.
+template <bool SETV>
+__global__ __launch_bounds__(kThreads) void k_predictor_plan(GatherDims g, HH hh, TrajParams tp, P3 v, float* vout,
                                                              PlanPt* __restrict__ P, int* __restrict__ bmax) {
-    int need = 0;
+    int need[3] = {0, 0, 0};
     const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
     const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     GridWalk gw(g, i0, stride);
     for (int64_t i = i0; i < g.nl; i += stride, gw.advance(g)) {
-        float q[3];
+        float q[3], r[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             const float x = tp.hx[d] * static_cast<float>(gw.idx[d]);
-            const float t = x - tp.sht * v.in[d][i];
-            q[d] = static_cast<float>(over_2pi(static_cast<double>(t)));
+            const float vd = v.in[d][i];
+            q[d] = static_cast<float>(over_2pi(static_cast<double>(x - tp.sht * vd)));
+            if constexpr (SETV) {
+                r[d] = static_cast<float>(over_2pi(static_cast<double>(x + tp.sht * vd)));
+                need[2] |= fabsf(vd) > 0.0f;
+                if (vout) vout[d * g.nl + i] = vd;
+            }
         }
         PlanPt pt;
-        need = max(need, encode_point(g, hh, q, gw.idx, pt));
+        const int a = encode_point(g, hh, q, gw.idx, pt);
         P[i] = pt;
+        if constexpr (SETV) {
+            need[0] = max(need[0], a);
+            need[1] = max(need[1], encode_point(g, hh, r, gw.idx, pt));
+        }
     }
-    block_max_to(need, bmax);
+    if constexpr (SETV) block_max_to(need, bmax);
 }
 
-// Plan of foot points given per component (W + d·nl), which are also
-// written interleaved into X (3 floats per point) unless X is null.
-__global__ __launch_bounds__(kThreads) void k_make_plan_soa(GatherDims g, HH hh, const float* __restrict__ W,
-                                                            float* __restrict__ X, PlanPt* __restrict__ P,
-                                                            int* __restrict__ bmax) {
-    int need = 0;
-    const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
-    const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    GridWalk gw(g, i0, stride);
-    for (int64_t i = i0; i < g.nl; i += stride, gw.advance(g)) {
-        const float q[3] = {W[i], W[g.nl + i], W[2 * g.nl + i]};
-        if (X) {
-            X[3 * i + 0] = q[0];
-            X[3 * i + 1] = q[1];
-            X[3 * i + 2] = q[2];
-        }
-        PlanPt pt;
-        need = max(need, encode_point(g, hh, q, gw.idx, pt));
-        P[i] = pt;
-    }
-    block_max_to(need, bmax);
+// Points given per component, interleaved: 3 floats per point.
+__global__ __launch_bounds__(kThreads) void k_interleave(int64_t nl, const float* __restrict__ X,
+                                                         float* __restrict__ out) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    if (i >= nl) return;
+    float q[3];
+    load_point(X, nl, i, q);
+    out[3 * i + 0] = q[0];
+    out[3 * i + 1] = q[1];
+    out[3 * i + 2] = q[2];
 }
 
 // Update coefficient c = 1 + ht/2·(α·dX + α·(1 + ht·α·dX)·d), d = ∇·v,
@@ -316,7 +324,7 @@ __global__ __launch_bounds__(kThreads) void k_adjoint_coeff(GatherDims g, HH hh,
     const int64_t i = point_index(nblocks);
     if (i >= g.nl) return;
     float q[3];
-    load_q3(X, i, q);
+    load_point(X, g.nl, i, q);
     Stencil S;
     setup_stencil(q, g, hh.h, S);
     const float* fs[1] = {divv};
@@ -340,7 +348,7 @@ __global__ __launch_bounds__(kThreads) void k_gather_direct(GatherDims g, HH hh,
     epi.select(blockIdx.y);
     const float aux = epi.aux(i);
     float q[3];
-    load_q3(X, i, q);
+    load_point(X, g.nl, i, q);
     Stencil S;
     setup_stencil(q, g, hh.h, S);
     const float* fs[1] = {f};
@@ -367,6 +375,20 @@ void check_gather_dims(const GatherDims& g) {
     CLR_REQUIRE(g.nl < (int64_t(1) << 31), kErrInvalidArgument, "grid too large for 32-bit stencil offsets");
 }
 
+void require_plan_size(const GatherDims& g) {
+    check_gather_dims(g);
+    CLR_REQUIRE(g.n1 <= kPlanMaxN && g.n2 <= kPlanMaxN && g.n3 <= kPlanMaxN, kErrUnsupportedSize,
+                "trajectory plans support at most 512 points per axis");
+}
+
+TrajParams traj_params(const Dims& d, float sigma, float ht) {
+    TrajParams tp;
+    for (int a = 0; a < 3; ++a) tp.hx[a] = d.hx[a];
+    tp.sht = sigma * ht;
+    tp.shth = sigma * (0.5f * ht);
+    return tp;
+}
+
 template <class Epi>
 void launch_direct(const GatherDims& g, const float* X, const float* f, int64_t fz, int nz, const Epi& e,
                    hipStream_t st) {
@@ -385,31 +407,20 @@ void launch_gather1(const GatherDims& g, const float* f, const float* X, float* 
     hipLaunchKernelGGL(k_gather1, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), f, X, out, nb);
 }
 
-void launch_gather3(const GatherDims& g, const float* const f[3], const float* X, float* const out[3], hipStream_t st) {
-    check_gather_dims(g);
-    const int nb = nblocks_for(g.nl);
-    P3 p{{f[0], f[1], f[2]}, {out[0], out[1], out[2]}};
-    hipLaunchKernelGGL(k_gather3, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), p, X, nb);
-}
-
 void launch_trajectory_rk2(const Dims& d, const float* const v[3], float sigma, float ht, float* X, hipStream_t st) {
     const GatherDims g = gather_dims(d);
     check_gather_dims(g);
     const int nb = nblocks_for(g.nl);
-    TrajParams tp;
-    for (int a = 0; a < 3; ++a) tp.hx[a] = d.hx[a];
-    const float hthalf = 0.5f * ht;
-    tp.sht = sigma * ht;
-    tp.shth = sigma * hthalf;
     P3 p{{v[0], v[1], v[2]}, {nullptr, nullptr, nullptr}};
-    hipLaunchKernelGGL(k_traj_rk2, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), tp, p, X, nb);
+    hipLaunchKernelGGL(k_traj_rk2, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), traj_params(d, sigma, ht), p, X, nb);
 }
 
-void launch_trajectory_rk4(const Dims& d, const float* const v[3], float sigma, float ht, float* X, float* F,
-                           hipStream_t st) {
+void launch_trajectory_rk4_stage(int stage, const Dims& d, const float* const v[3], float sigma, float ht, float* X,
+                                 const float* Fin, float* Fout, hipStream_t st) {
     const GatherDims g = gather_dims(d);
     check_gather_dims(g);
-    CLR_REQUIRE(F != nullptr && F != X, kErrInvalidArgument, "RK4 trajectory needs a separate 3-field work buffer");
+    CLR_REQUIRE(stage >= 1 && stage <= 3, kErrInvalidArgument, "RK4 stage must be 1, 2 or 3");
+    CLR_REQUIRE((stage == 1 || Fin) && (stage == 3 || Fout), kErrInvalidArgument, "RK4 stage needs its stage sums");
     const int nb = nblocks_for(g.nl);
     Rk4Params tp;
     for (int a = 0; a < 3; ++a) tp.hx[a] = d.hx[a];
@@ -419,9 +430,12 @@ void launch_trajectory_rk4(const Dims& d, const float* const v[3], float sigma, 
     tp.s6 = static_cast<double>(sigma) * (static_cast<double>(ht) / 6.0);
     P3 p{{v[0], v[1], v[2]}, {nullptr, nullptr, nullptr}};
     const HH hh = make_hh(g);
-    hipLaunchKernelGGL(k_traj_rk4<1>, dim3(nb), dim3(kThreads), 0, st, g, hh, tp, p, X, F, nb);
-    hipLaunchKernelGGL(k_traj_rk4<2>, dim3(nb), dim3(kThreads), 0, st, g, hh, tp, p, X, F, nb);
-    hipLaunchKernelGGL(k_traj_rk4<3>, dim3(nb), dim3(kThreads), 0, st, g, hh, tp, p, X, F, nb);
+    if (stage == 1)
+        hipLaunchKernelGGL(k_traj_rk4<1>, dim3(nb), dim3(kThreads), 0, st, g, hh, tp, p, X, Fin, Fout, nb);
+    else if (stage == 2)
+        hipLaunchKernelGGL(k_traj_rk4<2>, dim3(nb), dim3(kThreads), 0, st, g, hh, tp, p, X, Fin, Fout, nb);
+    else
+        hipLaunchKernelGGL(k_traj_rk4<3>, dim3(nb), dim3(kThreads), 0, st, g, hh, tp, p, X, Fin, Fout, nb);
 }
 
 namespace {
@@ -434,40 +448,40 @@ int plan_bound(const int* bmax, int nb, hipStream_t st) {
 }  // namespace
 
 int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* bmax, hipStream_t st) {
-    check_gather_dims(g);
-    CLR_REQUIRE(g.n1 <= kPlanMaxN && g.n2 <= kPlanMaxN && g.n3 <= kPlanMaxN, kErrUnsupportedSize,
-                "trajectory plans support at most 512 points per axis");
+    require_plan_size(g);
     const int nb = std::min(nblocks_for(g.nl), kPlanBlocks);
     hipLaunchKernelGGL(k_make_plan, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), X, reinterpret_cast<PlanPt*>(P),
                        bmax);
     return plan_bound(bmax, nb, st);
 }
 
-int launch_rk2_predictor_plan(const Dims& d, const float* const v[3], float sigma, float ht, uint32_t* P,
-                              int* bmax, hipStream_t st) {
+VelocityBounds launch_set_velocity(const Dims& d, const float* v, float* vout, float ht, uint32_t* P, int* bmax,
+                                   hipStream_t st) {
     const GatherDims g = gather_dims(d);
-    check_gather_dims(g);
-    CLR_REQUIRE(g.n1 <= kPlanMaxN && g.n2 <= kPlanMaxN && g.n3 <= kPlanMaxN, kErrUnsupportedSize,
-                "trajectory plans support at most 512 points per axis");
-    TrajParams tp;
-    for (int a = 0; a < 3; ++a) tp.hx[a] = d.hx[a];
-    tp.sht = sigma * ht;
-    tp.shth = sigma * (0.5f * ht);
-    P3 p{{v[0], v[1], v[2]}, {nullptr, nullptr, nullptr}};
+    require_plan_size(g);
+    P3 p{{v, v + g.nl, v + 2 * g.nl}, {nullptr, nullptr, nullptr}};
     const int nb = std::min(nblocks_for(g.nl), kPlanBlocks);
-    hipLaunchKernelGGL(k_predictor_plan, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), tp, p,
-                       reinterpret_cast<PlanPt*>(P), bmax);
-    return plan_bound(bmax, nb, st);
+    hipLaunchKernelGGL(k_predictor_plan<true>, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g),
+                       traj_params(d, 1.0f, ht), p, v == vout ? nullptr : vout, reinterpret_cast<PlanPt*>(P), bmax);
+    VelocityBounds b;
+    b.dbound[0] = plan_bound(bmax, nb, st);
+    b.dbound[1] = *std::max_element(bmax + kPlanBlocks, bmax + kPlanBlocks + nb);
+    b.zero = *std::max_element(bmax + 2 * kPlanBlocks, bmax + 2 * kPlanBlocks + nb) == 0;
+    return b;
 }
 
-int launch_make_plan_soa(const GatherDims& g, const float* W, float* X, uint32_t* P, int* bmax, hipStream_t st) {
-    check_gather_dims(g);
-    CLR_REQUIRE(g.n1 <= kPlanMaxN && g.n2 <= kPlanMaxN && g.n3 <= kPlanMaxN, kErrUnsupportedSize,
-                "trajectory plans support at most 512 points per axis");
+void launch_predictor_plan(const Dims& d, const float* const v[3], float sigma, float ht, uint32_t* P,
+                           hipStream_t st) {
+    const GatherDims g = gather_dims(d);
+    require_plan_size(g);
+    P3 p{{v[0], v[1], v[2]}, {nullptr, nullptr, nullptr}};
     const int nb = std::min(nblocks_for(g.nl), kPlanBlocks);
-    hipLaunchKernelGGL(k_make_plan_soa, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), W, X,
-                       reinterpret_cast<PlanPt*>(P), bmax);
-    return plan_bound(bmax, nb, st);
+    hipLaunchKernelGGL(k_predictor_plan<false>, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g),
+                       traj_params(d, sigma, ht), p, nullptr, reinterpret_cast<PlanPt*>(P), nullptr);
+}
+
+void launch_interleave(int64_t nl, const float* X, float* out, hipStream_t st) {
+    hipLaunchKernelGGL(k_interleave, dim3(nblocks_for(nl)), dim3(kThreads), 0, st, nl, X, out);
 }
 
 void launch_adjoint_coeff(const GatherDims& g, const float* X, const float* divv, float ht, float alpha, float* C,

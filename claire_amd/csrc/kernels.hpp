@@ -78,8 +78,9 @@ size_t noalloc_grad_bytes(const int nx[3]);
 void grad_noalloc(const int nx[3], const float* f, float* g, hipStream_t st);
 
 // ---------------------------------------------------------------------------
-// Semi-Lagrangian gathers (interp.hip, gather_lds.hip).  X: normalized query
-// points, interleaved xyz (3 floats per grid point).
+// Semi-Lagrangian gathers (interp.hip, gather_lds.hip).  X: foot points over
+// 2π, one component per field (component d of point i at X[d·nl + i]), except
+// for launch_gather1, whose query points are interleaved xyz.
 // ---------------------------------------------------------------------------
 struct GatherDims {
     int n1, n2, n3;
@@ -88,50 +89,64 @@ struct GatherDims {
 
 GatherDims gather_dims(const Dims& d);
 
-// out = f(X)
+// out = f(X), X interleaved (3 floats per point), any displacement
 void launch_gather1(const GatherDims& g, const float* f, const float* X, float* out, hipStream_t st);
-// out_d = f_d(X), d = 0..2 (shared stencil weights)
-void launch_gather3(const GatherDims& g, const float* const f[3], const float* X, float* const out[3], hipStream_t st);
-// RK2 characteristic, Euler predictor and velocity gather fused:
+// out = X, interleaved
+void launch_interleave(int64_t nl, const float* X, float* out, hipStream_t st);
+// RK2 characteristic, Euler predictor and velocity gather fused, any
+// displacement:
 //   X̃ = (x − σ·ht·v)/2π,  X = (x − σ·ht/2·(v(X̃) + v))/2π
 void launch_trajectory_rk2(const Dims& d, const float* const v[3], float sigma, float ht, float* X, hipStream_t st);
-// RK4 characteristic (three launches); F: work buffer of 3·nl floats.
-void launch_trajectory_rk4(const Dims& d, const float* const v[3], float sigma, float ht, float* X, float* F,
-                           hipStream_t st);
+// Stage 1 to 3 of the RK4 characteristic, any displacement: reads v at the
+// stage point in X (stage 1: at the first stage point, formed from v) and
+// replaces it by the next one; stage sums as in launch_lds_traj_rk4_stage,
+// except that Fout may be Fin.
+void launch_trajectory_rk4_stage(int stage, const Dims& d, const float* const v[3], float sigma, float ht, float* X,
+                                 const float* Fin, float* Fout, hipStream_t st);
 
 // Packed plan of a trajectory: 3 words per point (12 B), one per axis, the
 // fraction t ∈ [1,2) of the rescaled coordinate u = q·N + 3 and the offset of
 // the first stencil node from the point (layout in gather_device.hpp).
 // Returns the per-axis stencil displacement bound D in cells (synchronizes
 // the stream); 1 << 20 when a foot point is not finite.  n <= 512 per axis.
-// `bmax`: kPlanBlocks ints of pinned host memory that the device can write
+// `bmax`: 3·kPlanBlocks ints of pinned host memory that the device can write
 // (the blocks' bounds; one launch at a time may use them).
 constexpr int kPlanBlocks = 2048;
 int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* bmax, hipStream_t st);
 // RK2 characteristic through the LDS-staged gather, in three passes:
 //   1. the packed plan of the Euler predictor X̃ = (x − σ·ht·v)/2π into P
-//      (launch_rk2_predictor_plan, which returns its displacement bound);
+//      (launch_set_velocity or launch_predictor_plan);
 //   2. v gathered along it with the corrector as epilogue,
-//      X = (x − σ·ht/2·(v(X̃) + v))/2π, one component per field of W (3·nl
-//      floats; launch_lds_traj_rk2_corrector, bound <= 4);
-//   3. X interleaved into X (3 floats per point) and its plan into P
-//      (launch_make_plan_soa, which returns the bound of X).
-// The foot points equal those of launch_trajectory_rk2.
-int launch_rk2_predictor_plan(const Dims& d, const float* const v[3], float sigma, float ht, uint32_t* P,
-                              int* bmax, hipStream_t st);
+//      X = (x − σ·ht/2·(v(X̃) + v))/2π (launch_lds_traj_rk2_corrector, bound
+//      <= 4);
+//   3. the plan of X into P (launch_make_plan, which returns its bound).
+// The foot points equal those of launch_trajectory_rk2 up to FMA contraction.
+//
+// First pass over a new velocity v (3·nl): copies it to vout (unless v ==
+// vout), writes the predictor's plan for σ = +1 and returns the displacement
+// bounds of the predictors for σ = +1 and −1 and whether v is zero
+// (synchronizes the stream).
+struct VelocityBounds {
+    int dbound[2];
+    bool zero;
+};
+VelocityBounds launch_set_velocity(const Dims& d, const float* v, float* vout, float ht, uint32_t* P, int* bmax,
+                                   hipStream_t st);
+// The predictor's plan alone.
+void launch_predictor_plan(const Dims& d, const float* const v[3], float sigma, float ht, uint32_t* P,
+                           hipStream_t st);
 void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, int dbound, const float* const v[3], float sigma,
-                                   float ht, float* W, hipStream_t st);
-int launch_make_plan_soa(const GatherDims& g, const float* W, float* X, uint32_t* P, int* bmax, hipStream_t st);
-// RK4 characteristic the same way: the first stage point (x − σ·ht/2·v)/2π
-// is launch_rk2_predictor_plan with ht/2; each stage gathers v along the
+                                   float ht, float* X, hipStream_t st);
+// RK4 characteristic the same way: the plan of the first stage point
+// (x − σ·ht/2·v)/2π is the predictor's with ht/2; each stage gathers v along the
 // previous point's plan (bound <= 4), accumulates the stage sum f and writes
-// the next point per component into W (the final X at stage 3), whose plan
-// launch_make_plan_soa builds (X null for the intermediate points).  Stage 1
+// the next point into X (the foot point at stage 3), whose plan
+// launch_make_plan builds.  Stage 1
 // writes f into Fout (Fin unused), stage 2 reads Fin and writes Fout (two
 // distinct buffers: no launch updates an operand in place, so a gather may
 // be repeated while its chunk length is tuned), stage 3 reads Fin.
 void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, int dbound, const float* const v[3],
-                               float sigma, float ht, const float* Fin, float* Fout, float* W, hipStream_t st);
+                               float sigma, float ht, const float* Fin, float* Fout, float* X, hipStream_t st);
 // The LDS-staged gathers need D <= lds_gather_max_displacement().
 int lds_gather_max_displacement();
 // Update coefficient per point: C = 1 + ht/2·(α·dX + α·(1 + ht·α·dX)·d)
@@ -142,7 +157,7 @@ void launch_adjoint_coeff(const GatherDims& g, const float* X, const float* divv
                           hipStream_t st);
 
 // A trajectory as the gathers see it: the packed plan, the raw foot points
-// (3 floats per point, /2π) and the plan's displacement bound.
+// (one component per field) and the plan's displacement bound.
 struct TrajectoryPlan {
     const uint32_t* P;
     const float* X;
