@@ -511,7 +511,7 @@ int clr_trajectory(clr_ctx* ctx, int flag, float* X_out) {
         reg::CLAIRE& c = C(ctx);
         const std::string f = flag == CLR_STATE ? "state" : (flag == CLR_ADJOINT ? "adjoint" : "?");
         if (f == "?") throw Error(claire_amd::kErrInvalidArgument, "flag wrong");
-        c.EnsureTrajectories();
+        c.EnsureTrajectory(f);
         c.SL()->GetTrajectory(f, X_out);
         check_hip_launch();
     });
@@ -521,7 +521,7 @@ namespace {
 void ensure_traj(reg::CLAIRE& c, int flag) {
     const std::string f = flag == CLR_STATE ? "state" : (flag == CLR_ADJOINT ? "adjoint" : "?");
     if (f == "?") throw Error(claire_amd::kErrInvalidArgument, "flag wrong");
-    c.EnsureTrajectories();
+    c.EnsureTrajectory(f);
 }
 }  // namespace
 

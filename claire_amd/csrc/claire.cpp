@@ -88,83 +88,66 @@ void Profiler::reset() {
 // ---------------------------------------------------------------------------
 // Reducer (FP64)
 // ---------------------------------------------------------------------------
-Reducer::Reducer(const RegOpt* opt) : m_Opt(opt), m_Partial(2 * kReduceBlocks), m_Result(kSlots) {}
+Reducer::Reducer(const RegOpt* opt) : m_Opt(opt), m_Partial(3 * kReduceBlocks), m_Result(kSlots), m_Host(kSlots) {}
 
 void Reducer::DotAlpha(const float* p, const float* w, IntType n, claire_amd::PcgState* s) {
     KernelScope k(m_Opt->prof, "reduce_dot", 8.0 * n);
     launch_dot_pcg_alpha(p, w, n, m_Partial.get(), m_Result.get(), s, m_Opt->stream);
 }
 
-void Reducer::DotsBeta(const float* r, const float* z, IntType n, claire_amd::PcgState* s) {
+void Reducer::DotsBeta(const float* r, const float* z, IntType n, claire_amd::PcgState* s,
+                       claire_amd::PcgState* host) {
     KernelScope k(m_Opt->prof, "reduce_dot2", 8.0 * n);
-    launch_dots_pcg_beta(r, z, n, m_Partial.get(), m_Result.get(), s, m_Opt->stream);
+    launch_dots_pcg_beta(r, z, n, m_Partial.get(), m_Result.get(), s, host, m_Opt->stream);
 }
 
 void Reducer::DotTo(const float* a, const float* b, IntType n, int slot) {
     CLR_REQUIRE(slot >= 0 && slot < kSlots, kErrInvalidArgument, "reduction slot out of range");
     KernelScope k(m_Opt->prof, "reduce_dot", 8.0 * n);
-    launch_dot(a, b, n, m_Partial.get(), m_Result.get() + slot, m_Opt->stream);
+    launch_dot(a, b, n, m_Partial.get(), m_Result.get() + slot, m_Host.get() + slot, m_Opt->stream);
+}
+
+void Reducer::SqDistTo(const float* a, const float* b, IntType n, int slot) {
+    CLR_REQUIRE(slot >= 0 && slot < kSlots, kErrInvalidArgument, "reduction slot out of range");
+    KernelScope k(m_Opt->prof, "reduce_sqdist", 8.0 * n);
+    launch_sqdist(a, b, n, m_Partial.get(), m_Result.get() + slot, m_Host.get() + slot, m_Opt->stream);
+}
+
+void Reducer::SumPartialsTo(const double* partial, int np, int slot) {
+    CLR_REQUIRE(slot >= 0 && slot < kSlots, kErrInvalidArgument, "reduction slot out of range");
+    launch_sum_partials(partial, np, m_Result.get() + slot, m_Host.get() + slot, m_Opt->stream);
 }
 
 void Reducer::Fetch(double* out, int nslots) {
     CLR_REQUIRE(nslots >= 1 && nslots <= kSlots, kErrInvalidArgument, "reduction slot count out of range");
-    CLR_HIP_CHECK(hipMemcpyAsync(out, m_Result.get(), sizeof(double) * nslots, hipMemcpyDeviceToHost, m_Opt->stream));
+    CLR_HIP_CHECK(hipGetLastError());  // a launch that failed wrote no result
     CLR_HIP_CHECK(hipStreamSynchronize(m_Opt->stream));
-}
-
-double Reducer::fetch() {
-    double h = 0.0;
-    CLR_HIP_CHECK(hipMemcpyAsync(&h, m_Result.get(), sizeof(double), hipMemcpyDeviceToHost, m_Opt->stream));
-    CLR_HIP_CHECK(hipStreamSynchronize(m_Opt->stream));
-    return h;
+    std::copy(m_Host.get(), m_Host.get() + nslots, out);
 }
 
 double Reducer::Dot(const float* a, const float* b, IntType n) {
-    {
-        KernelScope k(m_Opt->prof, "reduce_dot", 8.0 * n);
-        launch_dot(a, b, n, m_Partial.get(), m_Result.get(), m_Opt->stream);
-    }
-    return fetch();
+    DotTo(a, b, n, 0);
+    double r = 0.0;
+    Fetch(&r, 1);
+    return r;
 }
 
 double Reducer::AbsMax(const float* a, IntType n) {
     {
         KernelScope k(m_Opt->prof, "reduce_absmax", 4.0 * n);
-        launch_absmax(a, n, m_Partial.get(), m_Result.get(), m_Opt->stream);
+        launch_absmax(a, n, m_Partial.get(), m_Result.get(), m_Host.get(), m_Opt->stream);
     }
-    return fetch();
+    double r = 0.0;
+    Fetch(&r, 1);
+    return r;
 }
 
-double Reducer::Min(const float* a, IntType n) {
+void Reducer::Stats(const float* a, IntType n, double out[3]) {
     {
-        KernelScope k(m_Opt->prof, "reduce_min", 4.0 * n);
-        launch_min(a, n, m_Partial.get(), m_Result.get(), m_Opt->stream);
+        KernelScope k(m_Opt->prof, "reduce_stats", 4.0 * n);
+        launch_stats(a, n, m_Partial.get(), m_Host.get(), m_Opt->stream);
     }
-    return fetch();
-}
-
-double Reducer::Max(const float* a, IntType n) {
-    {
-        KernelScope k(m_Opt->prof, "reduce_max", 4.0 * n);
-        launch_max(a, n, m_Partial.get(), m_Result.get(), m_Opt->stream);
-    }
-    return fetch();
-}
-
-double Reducer::Sum(const float* a, IntType n) {
-    {
-        KernelScope k(m_Opt->prof, "reduce_sum", 4.0 * n);
-        launch_sum(a, n, m_Partial.get(), m_Result.get(), m_Opt->stream);
-    }
-    return fetch();
-}
-
-double Reducer::SqDist(const float* a, const float* b, IntType n) {
-    {
-        KernelScope k(m_Opt->prof, "reduce_sqdist", 8.0 * n);
-        launch_sqdist(a, b, n, m_Partial.get(), m_Result.get(), m_Opt->stream);
-    }
-    return fetch();
+    Fetch(out, 3);
 }
 
 // ---------------------------------------------------------------------------
@@ -289,7 +272,7 @@ void SpectralOps::Multiplier3(const SpecParams& sp, const float* const in[3], fl
     }
 }
 
-void SpectralOps::Norm3(const SpecParams& sp, const float* const v[3], double* result) {
+void SpectralOps::Norm3(const SpecParams& sp, const float* const v[3], Reducer* red, int slot) {
     const Dims& d = m_Opt->domain;
     hipStream_t st = m_Opt->stream;
     c32* s[3] = {m_Spec[0].get(), m_Spec[1].get(), m_Spec[2].get()};
@@ -300,7 +283,7 @@ void SpectralOps::Norm3(const SpecParams& sp, const float* const v[3], double* r
     {
         KernelScope k(m_Opt->prof, "fft_x1_norm", 24.0 * d.nlc);
         m_Plan->x1_norm(s, 3, sp, m_NormPartial.get(), st);
-        launch_sum_partials(m_NormPartial.get(), static_cast<int>(np), result, st);
+        red->SumPartialsTo(m_NormPartial.get(), static_cast<int>(np), slot);
     }
 }
 
@@ -367,9 +350,7 @@ int Regularization::ApplyInverse(VecField* Ainvx, const VecField* x, bool applys
     return 0;
 }
 
-int Regularization::EvaluateFunctional(double* R, const VecField* v) {
-    *R = 0.0;
-    if (m_Opt->beta[0] == 0.0f) return 0;
+void Regularization::FunctionalTo(const VecField* v, int slot) {
     // The norms are folded from the spectrum (FFTPlan3D::x1_norm):
     //   H1    ½·hd·β0·(Σ_i ‖∇v_i‖² + β1·‖v‖²)  src/RegularizationH1.cpp:140-147
     //   H1SN  ½·hd·β0·Σ_i ‖∇v_i‖²               src/RegularizationH1SN.cpp:84-141
@@ -378,11 +359,21 @@ int Regularization::EvaluateFunctional(double* R, const VecField* v) {
     SpecParams sp = Params(kOpRegApply);
     if (sp.norm == kRegH2) sp.beta1 = std::sqrt(sp.beta1);
     const float* in[3] = {v->m_X1, v->m_X2, v->m_X3};
-    m_Spec->Norm3(sp, in, m_Red->Slot(0));
+    m_Spec->Norm3(sp, in, m_Red, slot);
+}
+
+double Regularization::FunctionalOf(double sum) const {
+    const double hd = m_Opt->GetLebesgueMeasure();
+    return 0.5 * hd * m_Opt->beta[0] * (sum / static_cast<double>(m_Opt->domain.nl));
+}
+
+int Regularization::EvaluateFunctional(double* R, const VecField* v) {
+    *R = 0.0;
+    if (m_Opt->beta[0] == 0.0f) return 0;
+    FunctionalTo(v, 0);
     double sum;
     m_Red->Fetch(&sum, 1);
-    const double hd = m_Opt->GetLebesgueMeasure();
-    *R = 0.5 * hd * m_Opt->beta[0] * (sum / static_cast<double>(m_Opt->domain.nl));
+    *R = FunctionalOf(sum);
     return 0;
 }
 
@@ -647,7 +638,8 @@ void CLAIRE::RequireVelocity() const { CLR_REQUIRE(m_HaveVelocity, kErrState, "v
 int CLAIRE::SetControlVariable(const float* v) {
     CLR_REQUIRE(v != nullptr, kErrInvalidArgument, "null input vector");
     m_HaveVelocity = true;
-    m_TrajValid = m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
+    DropTrajectories();
+    m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
     ++m_GraphEpoch;
     // CLAIREBase::IsVelocityZero (src/CLAIREBase.cpp:578-605): ∞-norm == 0
     if (UsesTrajectories()) {
@@ -683,35 +675,47 @@ int CLAIRE::SetReferenceImage(const float* mR) {
     return 0;
 }
 
-void CLAIRE::EnsureTrajectories() {
+void CLAIRE::EnsureTrajectory(const std::string& flag) {
     RequireVelocity();
-    if (m_TrajValid) return;
+    if (flag == "state")
+        EnsureStateTrajectory();
+    else
+        EnsureAdjointTrajectory();
+}
+
+void CLAIRE::EnsureStateTrajectory() {
+    RequireVelocity();
+    if (m_StateTrajValid) return;
     m_SL->ComputeTrajectory(m_VelocityField.get(), "state");
-    m_SL->ComputeTrajectory(m_VelocityField.get(), "adjoint");
-    // div v and the adjoint update coefficient at every point
-    // (src/CLAIRE.cpp:2614-2635 / 3907-3927 compute ∇·v and (∇·v)(X) per solve)
+    m_StateTrajValid = true;
+    ++m_GraphEpoch;
+}
+
+void CLAIRE::EnsureDivergence() {
+    RequireVelocity();
+    if (m_DivValid) return;
     const float* vc[3] = {m_VelocityField->m_X1, m_VelocityField->m_X2, m_VelocityField->m_X3};
     m_Spectral->Div(m_Scalar.get(), vc);
+    m_DivValid = true;
+}
+
+void CLAIRE::EnsureAdjointTrajectory() {
+    RequireVelocity();
+    if (m_AdjTrajValid) return;
+    m_SL->ComputeTrajectory(m_VelocityField.get(), "adjoint");
+    // the adjoint update coefficient at every point from ∇·v
+    // (src/CLAIRE.cpp:2614-2635 / 3907-3927 compute ∇·v and (∇·v)(X) per solve)
     if (m_Opt.regmodel == kModelStokes) {
         // incompressible adjoints are pure transport (src/CLAIREStokes.cpp:169-406): c = 1
         launch_fill(m_AdjCoeff.get(), 1.0f, m_Opt.domain.nl, m_Opt.stream);
     } else {
+        EnsureDivergence();
         // bytes: plan 12 + div v gathered 4 + div v 4 + C 4 per point
         KernelScope k(m_Opt.prof, "gather_adjoint_coeff", 24.0 * m_Opt.domain.nl);
         launch_plan_adjoint_coeff(m_SL->Plan("adjoint"), gather_dims(m_Opt.domain), m_Scalar.get(),
                                   m_Opt.GetTimeStepSize(), 1.0f, m_AdjCoeff.get(), m_Opt.stream);
     }
-    if (m_Opt.pdetype == 0) {
-        // continuity-equation state update m^{j+1} = c·m^j(X_s) with
-        // c = 1 − ht/2·(dX + (1 − ht·dX)·d), d = ∇·v, dX = d(X_s): the α = −1
-        // form of the coefficient on the state trajectory
-        // (SolveContinuityEquationSL, src/CLAIRE.cpp:2813-2835)
-        m_StateCoeff.resize(static_cast<size_t>(m_Opt.domain.nl));
-        KernelScope k(m_Opt.prof, "gather_state_coeff", 24.0 * m_Opt.domain.nl);
-        launch_plan_adjoint_coeff(m_SL->Plan("state"), gather_dims(m_Opt.domain), m_Scalar.get(),
-                                  m_Opt.GetTimeStepSize(), -1.0f, m_StateCoeff.get(), m_Opt.stream);
-    }
-    m_TrajValid = true;
+    m_AdjTrajValid = true;
     ++m_GraphEpoch;
 }
 
@@ -721,15 +725,26 @@ int CLAIRE::SolveStateEquation() {
     const int64_t nl = m_Opt.domain.nl;
     const int nt = m_Opt.nt;
     // the SL solves and the continuity equation need the trajectories
-    if (UsesTrajectories()) EnsureTrajectories();
     float* m = m_State.get();
     launch_copy(m_TemplateImage.get(), m, nl, m_Opt.stream);  // m^0 = mT (src/CLAIRE.cpp:1896)
     if (m_VelocityIsZero) {
         for (int j = 1; j <= nt; ++j) launch_copy(m, m + j * nl, nl, m_Opt.stream);  // src/CLAIRE.cpp:1909-1920
     } else if (m_Opt.pdetype == 0) {
         // SolveContinuityEquationSL (src/CLAIRE.cpp:2735-2854)
+        EnsureStateTrajectory();
         const TrajectoryPlan tp = m_SL->Plan("state");
         const GatherDims g = gather_dims(m_Opt.domain);
+        if (!m_StateCoeffValid) {
+            // state update m^{j+1} = c·m^j(X_s) with c = 1 − ht/2·(dX + (1 −
+            // ht·dX)·d), d = ∇·v, dX = d(X_s): the α = −1 form of the
+            // coefficient on the state trajectory (src/CLAIRE.cpp:2813-2835)
+            EnsureDivergence();
+            m_StateCoeff.resize(static_cast<size_t>(nl));
+            KernelScope k(m_Opt.prof, "gather_state_coeff", 24.0 * nl);
+            launch_plan_adjoint_coeff(tp, g, m_Scalar.get(), m_Opt.GetTimeStepSize(), -1.0f, m_StateCoeff.get(),
+                                      m_Opt.stream);
+            m_StateCoeffValid = true;
+        }
         for (int j = 0; j < nt; ++j) {
             KernelScope k(m_Opt.prof, "continuity_step", 24.0 * nl);
             launch_plan_adjoint_step(tp, g, m_StateCoeff.get(), m + j * nl, m + (j + 1) * nl, m_Opt.stream);
@@ -737,6 +752,7 @@ int CLAIRE::SolveStateEquation() {
     } else if (m_Opt.pdesolver == 0) {
         Rk2StateSteps();  // SolveStateEquationRK2 (src/CLAIRE.cpp:1995-2105)
     } else {
+        EnsureStateTrajectory();
         for (int j = 0; j < nt; ++j)  // src/CLAIRE.cpp:2153-2163
             m_SL->Gather(m + (j + 1) * nl, m + j * nl, "state");
     }
@@ -760,7 +776,7 @@ void CLAIRE::EnsureStateGradients() {
 
 void CLAIRE::EnsureGradientsAtStateTrajectory() {
     EnsureStateGradients();
-    EnsureTrajectories();
+    EnsureStateTrajectory();
     if (m_GradMXValid) return;
     const int64_t nl = m_Opt.domain.nl;
     for (int j = 0; j < m_Opt.nt; ++j) {  // (∇m^j)(X_s), src/CLAIRE.cpp:3243-3247
@@ -793,34 +809,31 @@ int CLAIRE::ComputeDetDefGrad(bool inverse, float* jac, double stats[3]) {
     // (src/DeformationFields.cpp:315-388, 636-740): J⁰ = 1, then nt SL steps
     // along the state trajectory J^{j+1} = C·J^j(X_s) with
     // C = 1 + ht/2·(α·dX + α·(1 + ht·α·dX)·d), d = ∇·v, dX = d(X_s), α = ±1.
-    RequireVelocity();
-    EnsureTrajectories();
+    EnsureStateTrajectory();
+    EnsureDivergence();
     const int64_t nl = m_Opt.domain.nl;
     const int nt = m_Opt.nt;
     const GatherDims g = gather_dims(m_Opt.domain);
-    // work space of the problem, free outside a solve: ∇·v in m_Scalar, the
-    // coefficient in the first slot of the inc-state decrements m_S
-    float* divv = m_Scalar.get();
+    // work space of the problem, free outside a solve: the coefficient in the
+    // first slot of the inc-state decrements m_S
     float* coeff = m_S.get();
-    const float* vc[3] = {m_VelocityField->m_X1, m_VelocityField->m_X2, m_VelocityField->m_X3};
-    m_Spectral->Div(divv, vc);
     const TrajectoryPlan tp = m_SL->Plan("state");
     {
         KernelScope k(m_Opt.prof, "gather_det_coeff", 24.0 * nl);
-        launch_plan_adjoint_coeff(tp, g, divv, m_Opt.GetTimeStepSize(), inverse ? -1.0f : 1.0f, coeff, m_Opt.stream);
+        launch_plan_adjoint_coeff(tp, g, m_Scalar.get(), m_Opt.GetTimeStepSize(), inverse ? -1.0f : 1.0f, coeff,
+                                  m_Opt.stream);
     }
     float* buf[2] = {m_IncState[0].get(), m_IncState[1].get()};
     launch_fill(buf[0], 1.0f, nl, m_Opt.stream);
+    const float* J = buf[0];
     for (int j = 0; j < nt; ++j) {
+        float* next = (j == nt - 1 && jac) ? jac : buf[(j + 1) % 2];  // the last step writes the caller's field
         KernelScope k(m_Opt.prof, "det_step", 24.0 * nl);
-        launch_plan_adjoint_step(tp, g, coeff, buf[j % 2], buf[(j + 1) % 2], m_Opt.stream);
+        launch_plan_adjoint_step(tp, g, coeff, J, next, m_Opt.stream);
+        J = next;
     }
-    const float* J = buf[nt % 2];
-    stats[0] = m_Red->Min(J, nl);
-    stats[1] = m_Red->Max(J, nl);
-    stats[2] = m_Red->Sum(J, nl) / static_cast<double>(nl);
-    if (jac) launch_copy(J, jac, nl, m_Opt.stream);
-    CLR_HIP_CHECK(hipStreamSynchronize(m_Opt.stream));
+    m_Red->Stats(J, nl, stats);
+    stats[2] /= static_cast<double>(nl);
     return 0;
 }
 
@@ -836,7 +849,8 @@ int CLAIRE::SetRKOrder(int order) {
     CLR_REQUIRE(order == 2 || order == 4, kErrInvalidArgument, "options for rk order are 2 and 4");
     if (order != m_Opt.rkorder) {
         m_Opt.rkorder = order;
-        m_TrajValid = m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
+        DropTrajectories();
+        m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
     }
     return 0;
 }
@@ -845,7 +859,8 @@ int CLAIRE::SetPDEType(int type) {
     CLR_REQUIRE(type == 0 || type == 1, kErrInvalidArgument, "pde type must be 0 (continuity) or 1 (transport)");
     if (type != m_Opt.pdetype) {
         m_Opt.pdetype = type;
-        m_TrajValid = m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
+        DropTrajectories();
+        m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
         ++m_GraphEpoch;
     }
     return 0;
@@ -872,11 +887,11 @@ void CLAIRE::EnsureMatVecCaches() {
         return;
     }
     EnsureGradientsAtStateTrajectory();
+    if (!m_VelocityIsZero) EnsureAdjointTrajectory();
     if (m_Opt.precision == 1) EnsureHalfGradients();
 }
 
 int CLAIRE::PrepareHessian() {
-    if (m_Opt.pdesolver == 2) EnsureTrajectories();
     EnsureMatVecCaches();
     CLR_HIP_CHECK(hipStreamSynchronize(m_Opt.stream));
     return 0;
@@ -1215,6 +1230,7 @@ int CLAIRE::SolveAdjointEquation() {
     CLR_REQUIRE(m_HaveReference, kErrState, "reference image not set");
     if (!m_StateValid) SolveStateEquation();
     EnsureStateGradients();
+    if (m_Opt.pdesolver == 2 && !m_VelocityIsZero) EnsureAdjointTrajectory();
     const int64_t nl = m_Opt.domain.nl;
     // λ¹ = mR − m^nt (src/DistanceMeasureSL2.cpp:198-205)
     launch_sub(m_ReferenceImage.get(), m_State.get() + m_Opt.nt * nl, m_Lam.get(), nl, m_Opt.stream);
@@ -1249,7 +1265,8 @@ int CLAIRE::SetRegModel(int model) {
                 kErrInvalidArgument, "registration model must be 0 (compressible), 1 (Stokes) or 2 (relaxed Stokes)");
     if (model != m_Opt.regmodel) {
         m_Opt.regmodel = model;
-        m_TrajValid = m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
+        DropTrajectories();
+        m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
         ++m_GraphEpoch;
     }
     return 0;
@@ -1261,13 +1278,16 @@ int CLAIRE::EvaluateObjective(double* J, double* D, double* R, const float* v) {
     SolveStateEquation();
     const int64_t nl = m_Opt.domain.nl;
     const double hd = m_Opt.GetLebesgueMeasure();
-    // ½·hd·Σ(mR − m^nt)²/nc (src/DistanceMeasureSL2.cpp:124-147)
-    *D = 0.5 * hd * m_Red->SqDist(m_ReferenceImage.get(), m_State.get() + m_Opt.nt * nl, nl);
-    *R = 0.0;
-    if (!m_VelocityIsZero) {
-        m_Regularization->EvaluateFunctional(R, m_VelocityField.get());
-        if (m_Opt.regmodel == kModelRelaxedStokes) *R += DivergencePenalty();
-    }
+    // ½·hd·Σ(mR − m^nt)²/nc (src/DistanceMeasureSL2.cpp:124-147) and the
+    // regularization's sum, fetched with one wait
+    const bool reg = !m_VelocityIsZero && m_Opt.beta[0] != 0.0f;
+    double sums[2] = {0.0, 0.0};
+    m_Red->SqDistTo(m_ReferenceImage.get(), m_State.get() + m_Opt.nt * nl, nl, 0);
+    if (reg) m_Regularization->FunctionalTo(m_VelocityField.get(), 1);
+    m_Red->Fetch(sums, reg ? 2 : 1);
+    *D = 0.5 * hd * sums[0];
+    *R = reg ? m_Regularization->FunctionalOf(sums[1]) : 0.0;
+    if (!m_VelocityIsZero && m_Opt.regmodel == kModelRelaxedStokes) *R += DivergencePenalty();
     *J = *D + *R;
     return 0;
 }
@@ -1288,9 +1308,8 @@ int CLAIRE::EvaluateGradient(float* g, const float* v) {
 // stores the gradient with its components reversed and sums in that order).
 double CLAIRE::DivergencePenalty() {
     const int64_t nl = m_Opt.domain.nl;
-    const float* vc[3] = {m_VelocityField->m_X1, m_VelocityField->m_X2, m_VelocityField->m_X3};
-    float* d = m_Scalar.get();
-    m_Spectral->Div(d, vc);
+    EnsureDivergence();
+    const float* d = m_Scalar.get();
     float* gd[3] = {m_WorkVecField1->m_X3, m_WorkVecField1->m_X2, m_WorkVecField1->m_X1};
     m_Spectral->Grad(gd, d);
     m_Red->DotTo(m_WorkVecField1->m_X1, m_WorkVecField1->m_X1, nl, 0);

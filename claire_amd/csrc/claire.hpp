@@ -181,29 +181,29 @@ class Reducer {
     explicit Reducer(const RegOpt* opt);
     double Dot(const float* a, const float* b, IntType n);
     double AbsMax(const float* a, IntType n);
-    double SqDist(const float* a, const float* b, IntType n);
-    double Min(const float* a, IntType n);
-    double Max(const float* a, IntType n);
-    double Sum(const float* a, IntType n);
+    // minimum, maximum and sum
+    void Stats(const float* a, IntType n, double out[3]);
     // Several dot products into result slots (0 <= slot < kSlots), read back
     // with one synchronization by Fetch: the host waits once instead of
     // once per product.
     static constexpr int kSlots = 16;
     void DotTo(const float* a, const float* b, IntType n, int slot);
+    void SqDistTo(const float* a, const float* b, IntType n, int slot);
+    void SumPartialsTo(const double* partial, int np, int slot);
     // The CG products with the CG scalar step fused into the final sum:
     // slot 0 = pᵀw then α; slots 1, 2 = rᵀr, rᵀz (one pass) then β.
     void DotAlpha(const float* p, const float* w, IntType n, claire_amd::PcgState* s);
-    void DotsBeta(const float* r, const float* z, IntType n, claire_amd::PcgState* s);
+    // (the CG state also to *host, pinned)
+    void DotsBeta(const float* r, const float* z, IntType n, claire_amd::PcgState* s, claire_amd::PcgState* host);
     void Fetch(double* out, int nslots);
     // Device address of the result slots (read by kernels that consume the
     // products without a host round trip).
     const double* Slots() const { return m_Result.get(); }
-    double* Slot(int i) { return m_Result.get() + i; }
 
   private:
-    double fetch();
     const RegOpt* m_Opt;
     DeviceArray<double> m_Partial, m_Result;
+    PinnedArray<double> m_Host;  // m_Result as the host sees it
 };
 
 class VecField {
@@ -242,8 +242,8 @@ class SpectralOps {
     void Multiplier3(const claire_amd::SpecParams& sp, const float* const in[3], float* const out[3], float alpha,
                      const float* const add[3], float beta);
     // Launches Σ_x |M v|²·N of a vector field, m² of sp.norm (FFTPlan3D::x1_norm),
-    // into *result (device).
-    void Norm3(const claire_amd::SpecParams& sp, const float* const v[3], double* result);
+    // into slot `slot` of `red`.
+    void Norm3(const claire_amd::SpecParams& sp, const float* const v[3], Reducer* red, int slot);
     // b ← b + F⁻¹[x̂] with the projection of sp.op (kOpProjStokes or
     // kOpProjRelaxed), in place on the three components.
     void Project(const claire_amd::SpecParams& sp, float* const b[3]);
@@ -261,6 +261,11 @@ class Regularization {
     Regularization(const RegOpt* opt, SpectralOps* spec, Reducer* red) : m_Opt(opt), m_Spec(spec), m_Red(red) {}
     virtual ~Regularization() = default;
     virtual int EvaluateFunctional(double* R, const VecField* v);
+    // The same in two parts, for a caller with more to reduce before its wait:
+    // launches the sum into slot `slot` of the reducer, and the functional from
+    // the fetched sum.
+    void FunctionalTo(const VecField* v, int slot);
+    double FunctionalOf(double sum) const;
     virtual int EvaluateGradient(VecField* dvR, const VecField* v);
     virtual int HessianMatVec(VecField* dvvR, const VecField* vtilde) { return EvaluateGradient(dvvR, vtilde); }
     virtual int ApplyInverse(VecField* Ainvx, const VecField* x, bool applysqrt);
@@ -430,7 +435,10 @@ class CLAIRE {
     // (DeformationFields::ComputeDetDefGrad); jac may be null; stats receive
     // min, max and mean.
     int ComputeDetDefGrad(bool inverse, float* jac, double stats[3]);
-    void EnsureTrajectories();
+    // The trajectories of the current velocity, each computed when something
+    // first moves along it (a line-search trial or det(∇y) never needs the
+    // adjoint one), with ∇·v and the adjoint update coefficient.
+    void EnsureTrajectory(const std::string& flag);
     int SolveIncAdjointFrom(const float* mtilde);
 
   private:
@@ -438,6 +446,10 @@ class CLAIRE {
     // Whether the selected solvers move along trajectories (the SL solves and
     // the continuity equation).
     bool UsesTrajectories() const { return m_Opt.pdesolver == 2 || m_Opt.pdetype == 0; }
+    void EnsureStateTrajectory();
+    void EnsureAdjointTrajectory();
+    void EnsureDivergence();  // m_Scalar = ∇·v
+    void DropTrajectories() { m_StateTrajValid = m_AdjTrajValid = m_DivValid = m_StateCoeffValid = false; }
     void EnsureStateGradients();
     void EnsureGradientsAtStateTrajectory();
     void IncStateCore(const VecField* vt, float* lt0_out, bool half);
@@ -495,7 +507,7 @@ class CLAIRE {
     DeviceArray<float> m_GradMX;         // (∇m^j)(X_s), nt·3·nl
     DeviceArray<float> m_S;              // inc-state decrements, nt·nl
     DeviceArray<float> m_Lam;            // adjoint time series λ^0..λ^nt, (nt+1)·nl
-    DeviceArray<float> m_Scalar;         // nl work
+    DeviceArray<float> m_Scalar;         // ∇·v (m_DivValid)
     DeviceArray<float> m_AdjCoeff;       // nl: adjoint update coefficient at every point
     DeviceArray<float> m_StateCoeff;     // nl: continuity-equation state coefficient (pdetype 0 only)
     DeviceArray<float> m_Rk2Work;        // 6·nl, RK2 integrators only: a vector field, rhs0, rhs1 / m̄
@@ -510,7 +522,8 @@ class CLAIRE {
 
     bool m_HaveVelocity = false, m_HaveIncVelocity = false, m_HaveTemplate = false, m_HaveReference = false;
     bool m_VelocityIsZero = false;
-    bool m_TrajValid = false, m_StateValid = false, m_GradMValid = false, m_GradMXValid = false;
+    bool m_StateTrajValid = false, m_AdjTrajValid = false, m_DivValid = false, m_StateCoeffValid = false;
+    bool m_StateValid = false, m_GradMValid = false, m_GradMXValid = false;
 };
 
 }  // namespace reg

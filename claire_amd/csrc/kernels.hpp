@@ -234,7 +234,8 @@ void launch_waxpy(float alpha, const float* x, const float* y, float* w, int64_t
 void launch_sub(const float* x, const float* y, float* z, int64_t n, hipStream_t st);
 
 // FP64 reductions.  `partial` must hold kReduceBlocks doubles and `result`
-// one double (device memory).
+// one double (device memory); the result is written to `host` too, pinned host
+// memory that the host reads after a stream synchronization (no copy to queue).
 constexpr int kReduceBlocks = 1024;
 
 // Device-resident scalars of a conjugate-gradient solve (reg::Optimizer::Pcg),
@@ -269,17 +270,19 @@ void launch_axpy2_pcg(const PcgState* s, const float* p, float* d, const float* 
 void launch_dot_pcg_alpha(const float* p, const float* w, int64_t n, double* partial, double* slots, PcgState* s,
                           hipStream_t st);
 // slots[1] = rᵀr and slots[2] = rᵀz in one pass (partial: 2·kReduceBlocks
-// doubles), then the stopping test and the β step
+// doubles), then the stopping test and the β step; the state after it also
+// goes to *host (pinned)
 void launch_dots_pcg_beta(const float* r, const float* z, int64_t n, double* partial, double* slots, PcgState* s,
-                          hipStream_t st);
-void launch_dot(const float* a, const float* b, int64_t n, double* partial, double* result, hipStream_t st);
-void launch_absmax(const float* a, int64_t n, double* partial, double* result, hipStream_t st);
-void launch_sqdist(const float* a, const float* b, int64_t n, double* partial, double* result, hipStream_t st);
-void launch_min(const float* a, int64_t n, double* partial, double* result, hipStream_t st);
-void launch_max(const float* a, int64_t n, double* partial, double* result, hipStream_t st);
-void launch_sum(const float* a, int64_t n, double* partial, double* result, hipStream_t st);
+                          PcgState* host, hipStream_t st);
+void launch_dot(const float* a, const float* b, int64_t n, double* partial, double* result, double* host,
+                hipStream_t st);
+void launch_absmax(const float* a, int64_t n, double* partial, double* result, double* host, hipStream_t st);
+void launch_sqdist(const float* a, const float* b, int64_t n, double* partial, double* result, double* host,
+                   hipStream_t st);
+// host[0..2] = minimum, maximum and sum (partial: 3·kReduceBlocks doubles)
+void launch_stats(const float* a, int64_t n, double* partial, double* host, hipStream_t st);
 // result = Σ partial[0..np), in a fixed order
-void launch_sum_partials(const double* partial, int np, double* result, hipStream_t st);
+void launch_sum_partials(const double* partial, int np, double* result, double* host, hipStream_t st);
 
 // ---------------------------------------------------------------------------
 // Explicit RK2 transport stages (rk2.hip); each follows a spectral grad or

@@ -201,12 +201,77 @@ __global__ __launch_bounds__(kThreads) void k_reduce_partial(const float* __rest
 
 template <int OP>
 __global__ __launch_bounds__(kThreads) void k_reduce_final(const double* __restrict__ partial, int np,
-                                                           double* __restrict__ result) {
+                                                           double* __restrict__ result, double* __restrict__ host) {
     __shared__ double sh[kThreads];
     double acc = red_init<OP>();
     for (int i = threadIdx.x; i < np; i += kThreads) acc = red_combine<OP>(acc, partial[i]);
     const double r = block_reduce<OP>(acc, sh);
-    if (threadIdx.x == 0) result[0] = r;
+    if (threadIdx.x == 0) {
+        result[0] = r;
+        host[0] = r;
+    }
+}
+
+// Minimum, maximum and sum in one pass, each folded as k_reduce_partial folds
+// it; partials of value k at partial[k·gridDim.x].
+template <bool VEC>
+__global__ __launch_bounds__(kThreads) void k_stats_partial(const float* __restrict__ a, int64_t n,
+                                                            double* __restrict__ partial) {
+    __shared__ double sh[kThreads];
+    double lo = red_init<kRedMin>(), hi = red_init<kRedMax>(), sum = 0.0;
+    auto fold = [&](float x) {
+        lo = red_step<kRedMin>(lo, x, 0.f);
+        hi = red_step<kRedMax>(hi, x, 0.f);
+        sum = red_step<kRedSum>(sum, x, 0.f);
+    };
+    const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    if constexpr (VEC) {
+        const int64_t n4 = n >> 2;
+        const float4* a4 = reinterpret_cast<const float4*>(a);
+        for (int64_t i = first; i < n4; i += stride) {
+            const float4 x = a4[i];
+            fold(x.x);
+            fold(x.y);
+            fold(x.z);
+            fold(x.w);
+        }
+        const int64_t tail = 4 * n4 + threadIdx.x;
+        if (blockIdx.x == 0 && tail < n) fold(a[tail]);
+    } else {
+        for (int64_t i = first; i < n; i += stride) fold(a[i]);
+    }
+    lo = block_reduce<kRedMin>(lo, sh);
+    __syncthreads();
+    hi = block_reduce<kRedMax>(hi, sh);
+    __syncthreads();
+    sum = block_reduce<kRedSum>(sum, sh);
+    if (threadIdx.x == 0) {
+        partial[blockIdx.x] = lo;
+        partial[gridDim.x + blockIdx.x] = hi;
+        partial[2 * gridDim.x + blockIdx.x] = sum;
+    }
+}
+
+__global__ __launch_bounds__(kThreads) void k_stats_final(const double* __restrict__ partial, int np,
+                                                          double* __restrict__ host) {
+    __shared__ double sh[kThreads];
+    double lo = red_init<kRedMin>(), hi = red_init<kRedMax>(), sum = 0.0;
+    for (int i = threadIdx.x; i < np; i += kThreads) {
+        lo = red_combine<kRedMin>(lo, partial[i]);
+        hi = red_combine<kRedMax>(hi, partial[np + i]);
+        sum = red_combine<kRedSum>(sum, partial[2 * np + i]);
+    }
+    lo = block_reduce<kRedMin>(lo, sh);
+    __syncthreads();
+    hi = block_reduce<kRedMax>(hi, sh);
+    __syncthreads();
+    sum = block_reduce<kRedSum>(sum, sh);
+    if (threadIdx.x == 0) {
+        host[0] = lo;
+        host[1] = hi;
+        host[2] = sum;
+    }
 }
 
 // Two dot products a·b and a·c in one pass, each folded exactly as
@@ -266,10 +331,11 @@ __global__ __launch_bounds__(kThreads) void k_reduce_partial_dot2(const float* _
 // Final sums of the CG products, then the CG scalar step on thread 0:
 //   NSUM = 1: slots[0] = pᵀw, then α (as k_pcg_alpha);
 //   NSUM = 2: slots[1] = rᵀr, slots[2] = rᵀz, then the stopping test and β
-//             (as k_pcg_beta).
+//             (as k_pcg_beta), and the state copied to *host.
 template <int NSUM>
 __global__ __launch_bounds__(kThreads) void k_reduce_final_pcg(const double* __restrict__ partial, int np,
-                                                               double* __restrict__ slots, PcgState* s) {
+                                                               double* __restrict__ slots, PcgState* s,
+                                                               PcgState* __restrict__ host) {
     __shared__ double sh[kThreads];
     double sums[NSUM];
 #pragma unroll
@@ -287,18 +353,20 @@ __global__ __launch_bounds__(kThreads) void k_reduce_final_pcg(const double* __r
         slots[1] = sums[0];
         slots[2] = sums[1];
         pcg_beta(s, sums[0], sums[1]);
+        *host = *s;
     }
 }
 
 template <int OP>
-void reduce(const float* a, const float* b, int64_t n, double* partial, double* result, hipStream_t st) {
+void reduce(const float* a, const float* b, int64_t n, double* partial, double* result, double* host,
+            hipStream_t st) {
     const uintptr_t align = reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b ? b : a);
     if ((align & 15u) == 0)
         hipLaunchKernelGGL((k_reduce_partial<OP, true>), dim3(kReduceBlocks), dim3(kThreads), 0, st, a, b, n, partial);
     else
         hipLaunchKernelGGL((k_reduce_partial<OP, false>), dim3(kReduceBlocks), dim3(kThreads), 0, st, a, b, n,
                            partial);
-    hipLaunchKernelGGL(k_reduce_final<OP>, dim3(1), dim3(kThreads), 0, st, partial, kReduceBlocks, result);
+    hipLaunchKernelGGL(k_reduce_final<OP>, dim3(1), dim3(kThreads), 0, st, partial, kReduceBlocks, result, host);
 }
 
 }  // namespace
@@ -346,10 +414,11 @@ void launch_dot_pcg_alpha(const float* p, const float* w, int64_t n, double* par
     else
         hipLaunchKernelGGL((k_reduce_partial<kRedDot, false>), dim3(kReduceBlocks), dim3(kThreads), 0, st, p, w, n,
                            partial);
-    hipLaunchKernelGGL(k_reduce_final_pcg<1>, dim3(1), dim3(kThreads), 0, st, partial, kReduceBlocks, slots, s);
+    hipLaunchKernelGGL(k_reduce_final_pcg<1>, dim3(1), dim3(kThreads), 0, st, partial, kReduceBlocks, slots, s,
+                       nullptr);
 }
 void launch_dots_pcg_beta(const float* r, const float* z, int64_t n, double* partial, double* slots, PcgState* s,
-                          hipStream_t st) {
+                          PcgState* host, hipStream_t st) {
     const uintptr_t align = reinterpret_cast<uintptr_t>(r) | reinterpret_cast<uintptr_t>(z);
     if ((align & 15u) == 0)
         hipLaunchKernelGGL(k_reduce_partial_dot2<true>, dim3(kReduceBlocks), dim3(kThreads), 0, st, r, r, z, n,
@@ -357,31 +426,32 @@ void launch_dots_pcg_beta(const float* r, const float* z, int64_t n, double* par
     else
         hipLaunchKernelGGL(k_reduce_partial_dot2<false>, dim3(kReduceBlocks), dim3(kThreads), 0, st, r, r, z, n,
                            partial);
-    hipLaunchKernelGGL(k_reduce_final_pcg<2>, dim3(1), dim3(kThreads), 0, st, partial, kReduceBlocks, slots, s);
+    hipLaunchKernelGGL(k_reduce_final_pcg<2>, dim3(1), dim3(kThreads), 0, st, partial, kReduceBlocks, slots, s,
+                       host);
 }
 void launch_xpay_pcg(const PcgState* s, float* p, const float* z, int64_t n, hipStream_t st) {
     if (n > 0) hipLaunchKernelGGL(k_xpay_pcg, dim3(blocks_for(n)), dim3(kThreads), 0, st, s, p, z, n);
 }
-void launch_dot(const float* a, const float* b, int64_t n, double* partial, double* result, hipStream_t st) {
-    reduce<kRedDot>(a, b, n, partial, result, st);
+void launch_dot(const float* a, const float* b, int64_t n, double* partial, double* result, double* host,
+                hipStream_t st) {
+    reduce<kRedDot>(a, b, n, partial, result, host, st);
 }
-void launch_absmax(const float* a, int64_t n, double* partial, double* result, hipStream_t st) {
-    reduce<kRedAbsMax>(a, nullptr, n, partial, result, st);
+void launch_absmax(const float* a, int64_t n, double* partial, double* result, double* host, hipStream_t st) {
+    reduce<kRedAbsMax>(a, nullptr, n, partial, result, host, st);
 }
-void launch_sqdist(const float* a, const float* b, int64_t n, double* partial, double* result, hipStream_t st) {
-    reduce<kRedSqDist>(a, b, n, partial, result, st);
+void launch_sqdist(const float* a, const float* b, int64_t n, double* partial, double* result, double* host,
+                   hipStream_t st) {
+    reduce<kRedSqDist>(a, b, n, partial, result, host, st);
 }
-void launch_min(const float* a, int64_t n, double* partial, double* result, hipStream_t st) {
-    reduce<kRedMin>(a, nullptr, n, partial, result, st);
+void launch_stats(const float* a, int64_t n, double* partial, double* host, hipStream_t st) {
+    if ((reinterpret_cast<uintptr_t>(a) & 15u) == 0)
+        hipLaunchKernelGGL(k_stats_partial<true>, dim3(kReduceBlocks), dim3(kThreads), 0, st, a, n, partial);
+    else
+        hipLaunchKernelGGL(k_stats_partial<false>, dim3(kReduceBlocks), dim3(kThreads), 0, st, a, n, partial);
+    hipLaunchKernelGGL(k_stats_final, dim3(1), dim3(kThreads), 0, st, partial, kReduceBlocks, host);
 }
-void launch_max(const float* a, int64_t n, double* partial, double* result, hipStream_t st) {
-    reduce<kRedMax>(a, nullptr, n, partial, result, st);
-}
-void launch_sum(const float* a, int64_t n, double* partial, double* result, hipStream_t st) {
-    reduce<kRedSum>(a, nullptr, n, partial, result, st);
-}
-void launch_sum_partials(const double* partial, int np, double* result, hipStream_t st) {
-    hipLaunchKernelGGL(k_reduce_final<kRedSum>, dim3(1), dim3(kThreads), 0, st, partial, np, result);
+void launch_sum_partials(const double* partial, int np, double* result, double* host, hipStream_t st) {
+    hipLaunchKernelGGL(k_reduce_final<kRedSum>, dim3(1), dim3(kThreads), 0, st, partial, np, result, host);
 }
 
 }  // namespace claire_amd

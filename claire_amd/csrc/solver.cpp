@@ -11,7 +11,7 @@ namespace reg {
 using namespace claire_amd;
 
 Optimizer::Optimizer(CLAIRE* problem)
-    : m_Prob(problem), m_N(3 * problem->Opt().domain.nl) {
+    : m_Prob(problem), m_N(3 * problem->Opt().domain.nl), m_HostState(1) {
     const size_t n = static_cast<size_t>(m_N);
     m_G.resize(n);
     m_D.resize(n);
@@ -100,7 +100,7 @@ void Optimizer::PcgIteration(bool inline_matvec, const GNOptions& opt) {
     red->DotAlpha(p, w, m_N, s);
     launch_axpy2_pcg(s, p, d, w, r, m_N, Stream());
     Precond(r, z, opt);
-    red->DotsBeta(r, z, m_N, s);
+    red->DotsBeta(r, z, m_N, s, m_HostState.get());
     launch_xpay_pcg(s, p, z, m_N, Stream());
 }
 
@@ -172,8 +172,9 @@ int Optimizer::Pcg(const float* g, double rtol, const GNOptions& opt, GNReport& 
                 PcgIteration(false, opt);
         }
         ++runs;
-        CLR_HIP_CHECK(hipMemcpyAsync(&hs, m_State.get(), sizeof(PcgState), hipMemcpyDeviceToHost, Stream()));
+        CLR_HIP_CHECK(hipGetLastError());  // a launch that failed wrote no state
         CLR_HIP_CHECK(hipStreamSynchronize(Stream()));
+        hs = *m_HostState.get();
         its = hs.k;
         if (hs.done || its >= kmax) break;
         // iterations still needed if the residual keeps its decay rate

@@ -81,6 +81,7 @@ class Optimizer {
     CLAIRE* m_Prob;
     IntType m_N;
     DeviceArray<claire_amd::PcgState> m_State;
+    PinnedArray<claire_amd::PcgState> m_HostState;  // the state after each queued iteration
     // A captured CG iteration, replayed while the problem's graph epoch and
     // the operator options stay the same.
     hipGraphExec_t m_IterGraph = nullptr;
