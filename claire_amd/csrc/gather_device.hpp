@@ -204,9 +204,13 @@ __device__ __forceinline__ bool plan_encode(float u, int idx, int n, uint32_t& w
 // says whether there is an operand at all.  Epilogues with kCoord need the
 // point's grid indices and provide apply_at(f(X), aux, i1, i2, i3) instead;
 // kOut2 adds a second output, apply2(f(X), aux) into outp2() (LDS kernel
-// only).
+// only).  kRowFrom1 is the order in which the pair-layout kernel contracts a
+// stencil row: the FMA chain starts at node 1 (as in the one-value kernels)
+// instead of node 0, so that the trajectory stages give the same bits from
+// either layout.
 // ---------------------------------------------------------------------------
 struct EpiPlain {  // out = f(X)
+    static constexpr bool kRowFrom1 = false;
     static constexpr bool kHasAux = false;
     static constexpr bool kCoord = false;
     static constexpr bool kOut2 = false;
@@ -221,6 +225,7 @@ struct EpiPlain {  // out = f(X)
 };
 
 struct EpiIncStep {  // out = sign·(f(X) − s)   (src/CLAIRE.cpp:3228-3273)
+    static constexpr bool kRowFrom1 = false;
     static constexpr bool kHasAux = true;
     static constexpr bool kCoord = false;
     static constexpr bool kOut2 = false;
@@ -236,6 +241,7 @@ struct EpiIncStep {  // out = sign·(f(X) − s)   (src/CLAIRE.cpp:3228-3273)
 };
 
 struct EpiAdjStep {  // out = c·f(X)   (src/CLAIRE.cpp:2668-2673, 3955-3962)
+    static constexpr bool kRowFrom1 = false;
     static constexpr bool kHasAux = true;
     static constexpr bool kCoord = false;
     static constexpr bool kOut2 = false;
@@ -254,6 +260,7 @@ struct EpiAdjStep {  // out = c·f(X)   (src/CLAIRE.cpp:2668-2673, 3955-3962)
 // k_adjoint_coeff: the SL adjoint step for α = 1 on the adjoint trajectory,
 // det(∇y^{±1}) and the continuity equation for α = ±1 on the state one).
 struct EpiAdjCoeff {
+    static constexpr bool kRowFrom1 = false;
     static constexpr bool kHasAux = true;
     static constexpr bool kCoord = false;
     static constexpr bool kOut2 = false;
@@ -277,6 +284,7 @@ struct EpiAdjCoeff {
 // X_z = (x_z − σ·ht/2·(v_z(X̃) + v_z(x)))/2π, stored per component (out +
 // z·zstride); aux is v_z at the point.  Same expressions as k_traj_rk2.
 struct EpiTrajRk2 {
+    static constexpr bool kRowFrom1 = true;
     static constexpr bool kHasAux = true;
     static constexpr bool kCoord = true;
     static constexpr bool kOut2 = false;
@@ -315,6 +323,7 @@ struct EpiTrajRk2 {
 // stage sum, in a buffer other than aux (stage 3 has no out2).
 template <int STAGE>
 struct EpiTrajRk4 {
+    static constexpr bool kRowFrom1 = true;
     static constexpr bool kHasAux = true;
     static constexpr bool kCoord = true;
     static constexpr bool kOut2 = STAGE < 3;

@@ -582,7 +582,8 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
             for (int b = 0; b < 4; ++b) {
                 const float2 lo = S[(K + a) & 3][b][0];
                 const float2 hi = S[(K + a) & 3][b][1];
-                const float r = w3[0] * lo.x + w3[1] * lo.y + w3[2] * hi.x + w3[3] * hi.y;
+                const float r01 = Epi::kRowFrom1 ? fmaf(w3[0], lo.x, w3[1] * lo.y) : fmaf(w3[1], lo.y, w3[0] * lo.x);
+                const float r = fmaf(w3[3], hi.y, fmaf(w3[2], hi.x, r01));
                 sa += w2[b] * r;
             }
             v += w1[a] * sa;
@@ -833,8 +834,9 @@ int chunk_override() {
     return e ? std::atoi(e) : 0;
 }
 
-// CLAIRE_AMD_GATHER_PAIR=0 selects the one-value-per-entry layout for single-field D <= 2 gathers
-// (three blocks per CU) instead of the pair layout (two), for comparison.
+// CLAIRE_AMD_GATHER_PAIR=0 selects the one-value-per-entry layout for every
+// D <= 2 gather (three blocks per CU) instead of the pair layout (two), for
+// comparison.
 bool pair_layout() {
     static const bool on = [] {
         const char* e = std::getenv("CLAIRE_AMD_GATHER_PAIR");
@@ -974,13 +976,16 @@ void dispatch(int dbound, const GatherDims& g, const uint32_t* P, const float* f
     CLR_REQUIRE(g.n1 >= 4 && g.n2 >= 4 && g.n3 >= 4, kErrInvalidArgument, "gather needs n >= 4 per axis");
     CLR_REQUIRE(g.nl < (int64_t(1) << 28), kErrInvalidArgument, "grid too large for 32-bit buffer byte offsets");
     CLR_REQUIRE(dbound >= 0 && dbound <= 4, kErrInvalidArgument, "displacement bound too large for the LDS gather");
-    // The pair layout is faster for one field per launch (the solves' steps:
-    // 110 µs against 115 at 256³, before later changes to both kernels) and
-    // for plain three-field gathers (295 against 300 µs); the trajectory
-    // stages were 6-12% slower with it (two blocks per CU instead of three)
-    // and now only match the one-value layout, so they keep that one.
+    // The pair layout (two blocks per CU) is faster than the one-value layout
+    // (three) for one field per launch (the solves' steps: 110 µs against 115
+    // at 256³, before later changes to both kernels), for plain three-field
+    // gathers, and for the trajectory stages from about 80³ points on: set
+    // velocity + state trajectory + one gather 615 -> 580 µs at 256³, 4.63 ->
+    // 4.35 ms at 512³, 125 -> 121 µs at 128³, 89.9 -> 89.0 at 96³.  Below, the
+    // third resident block counts for more: 58.6 against 56.9 µs at 64³.
     constexpr bool kPlain = std::is_same<Epi, EpiPlain>::value;
-    if (dbound <= 2 && (nz == 1 || kPlain) && pair_layout())
+    constexpr int64_t kPairStagePoints = int64_t(1) << 19;
+    if (dbound <= 2 && (nz == 1 || kPlain || g.nl >= kPairStagePoints) && pair_layout())
         launch_lds<2, true>(g, P, f, fzstride, nz, epi, st);
     else if (dbound <= 2)
         launch_lds<2, false>(g, P, f, fzstride, nz, epi, st);
