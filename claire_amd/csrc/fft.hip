@@ -394,6 +394,27 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_row_r2c(R2CPtrs ptr, int64_
 // The imaginary parts of the k3 = 0 and k3 = n3/2 coefficients are ignored
 // (FFTW c2r convention).
 // ---------------------------------------------------------------------------
+// Calls use(e, load(e)) for the e < n of this thread's part of [0, MOST), in
+// batches whose loads are all issued before the first value is used.
+template <int MOST, int THREADS, class Load, class Use>
+__device__ __forceinline__ void flat_copy(int n, Load&& load, Use&& use) {
+    constexpr int ITER = (MOST + THREADS - 1) / THREADS, BATCH = 15;
+#pragma unroll 1
+    for (int i0 = 0; i0 < ITER; i0 += BATCH) {
+        decltype(load(0)) x[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int e = threadIdx.x + THREADS * (i0 + i);
+            if (e < n) x[i] = load(e);
+        }
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+            const int e = threadIdx.x + THREADS * (i0 + i);
+            if (e < n) use(e, x[i]);
+        }
+    }
+}
+
 // ADD: some field has an added term (its values are loaded before the
 // transform, in registers the plain pass does not need).
 template <int N, bool ADD>
@@ -491,6 +512,39 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_row_c2r(C2RPtrs ptr, int64_
                 reinterpret_cast<float4*>(ob)[m] = o;
             }
         }
+    } else if constexpr (ADD) {
+        // Rows that are no multiple of 16 bytes, with an added field: the
+        // block's rows, contiguous in memory, are staged through LDS and
+        // written value by value with consecutive lanes on consecutive values,
+        // as the added field is read.  (Written from the registers, in runs of
+        // 5 values with a dependent read of the added field each, the
+        // three-field pass took 171 µs at 256×192×150, where moving its bytes
+        // takes about 50; the Hessian matvec there 1113 -> 1014 µs.  Without
+        // the added field staging gains nothing there and loses 4% at
+        // 64×64×150, and the passes' other accesses lose up to 10% by it at
+        // every length whose rows have fewer than 16 threads.)
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < V / RL; ++q) {
+            const int j = t + T * q;
+#pragma unroll
+            for (int r = 0; r < RL; ++r) s[lay(j + r * (N / RL), c)] = v[q * RL + r];
+        }
+        __syncthreads();
+        const int64_t r0 = 2 * static_cast<int64_t>(blockIdx.x) * G::B;
+        const int rows = nrows - r0 < 2 * G::B ? static_cast<int>(nrows - r0) : 2 * G::B;
+        const float* sf = reinterpret_cast<const float*>(s);
+        float* dst = out + r0 * N;
+        const float* ad = add ? add + r0 * N : nullptr;
+        auto value = [&](int e) {
+            const int row = e / N;
+            return alpha * sf[2 * lay(e - row * N, row >> 1) + (row & 1)];
+        };
+        if (ad)  // may be dst: each value is read before it is written
+            flat_copy<2 * G::B * N, G::THREADS>(
+                rows * N, [&](int e) { return ad[e]; }, [&](int e, float x) { dst[e] = value(e) + beta * x; });
+        else
+            for (int e = threadIdx.x; e < rows * N; e += G::THREADS) dst[e] = value(e);
     } else {
 #pragma unroll
         for (int q = 0; q < V / RL; ++q) {
@@ -499,8 +553,8 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_row_c2r(C2RPtrs ptr, int64_
             for (int r = 0; r < RL; ++r) {
                 const int n = j + r * (N / RL);
                 const c32 z = v[q * RL + r];
-                if (va) oa[n] = aa ? alpha * z.x + beta * aa[n] : alpha * z.x;
-                if (vb) ob[n] = ab ? alpha * z.y + beta * ab[n] : alpha * z.y;
+                if (va) oa[n] = alpha * z.x;
+                if (vb) ob[n] = alpha * z.y;
             }
         }
     }
