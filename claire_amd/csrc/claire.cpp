@@ -209,9 +209,8 @@ int VecField::WAXPY(ScalarType a, const VecField* x, const VecField* y) {
 // ---------------------------------------------------------------------------
 // SpectralOps (AccFFT replacement)
 // ---------------------------------------------------------------------------
-SpectralOps::SpectralOps(const RegOpt* opt) : m_Opt(opt), m_Plan(new FFTPlan3D(opt->domain)) {
-    for (auto& s : m_Spec) s.resize(static_cast<size_t>(opt->domain.nlc));
-}
+SpectralOps::SpectralOps(const RegOpt* opt)
+    : m_Opt(opt), m_Plan(new FFTPlan3D(opt->domain)), m_Spec(3 * static_cast<size_t>(opt->domain.nlc)) {}
 
 namespace {
 double bytes_x3_r2c(const Dims& d) { return 4.0 * d.nl + 8.0 * d.nlc; }
@@ -219,88 +218,138 @@ double bytes_col(const Dims& d) { return 16.0 * d.nlc; }
 double bytes_x3_c2r(const Dims& d, bool add) { return 8.0 * d.nlc + 4.0 * d.nl + (add ? 4.0 * d.nl : 0.0); }
 }  // namespace
 
+namespace {
+// Spacing of a vector field's components (the passes take equally spaced ones).
+template <class T>
+int64_t spacing(T* const v[3]) {
+    CLR_REQUIRE(v[2] - v[1] == v[1] - v[0], kErrInvalidArgument, "vector components must be equally spaced");
+    return v[1] - v[0];
+}
+}  // namespace
+
 void SpectralOps::R2C(const float* in, c32* out) {
     const Dims& d = m_Opt->domain;
     hipStream_t st = m_Opt->stream;
-    { KernelScope k(m_Opt->prof, "fft_x3_r2c", bytes_x3_r2c(d)); m_Plan->x3_r2c(in, out, st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", bytes_col(d)); m_Plan->x2(out, -1, st); }
+    { KernelScope k(m_Opt->prof, "fft_x3_r2c", bytes_x3_r2c(d)); m_Plan->x3_r2c(in, 0, out, 0, 1, st); }
+    { KernelScope k(m_Opt->prof, "fft_x2", bytes_col(d)); m_Plan->x2(out, 0, 1, -1, st); }
     { KernelScope k(m_Opt->prof, "fft_x1", bytes_col(d)); m_Plan->x1(out, -1, st); }
 }
 
-void SpectralOps::C2R(c32* in, float* out, float alpha, const float* add, float beta) {
+void SpectralOps::C2R(c32* in, float* out) {
     const Dims& d = m_Opt->domain;
     hipStream_t st = m_Opt->stream;
     { KernelScope k(m_Opt->prof, "fft_x1", bytes_col(d)); m_Plan->x1(in, +1, st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", bytes_col(d)); m_Plan->x2(in, +1, st); }
-    { KernelScope k(m_Opt->prof, "fft_x3_c2r", bytes_x3_c2r(d, add)); m_Plan->x3_c2r(in, out, st, alpha, add, beta); }
+    { KernelScope k(m_Opt->prof, "fft_x2", bytes_col(d)); m_Plan->x2(in, 0, 1, +1, st); }
+    { KernelScope k(m_Opt->prof, "fft_x3_c2r", bytes_x3_c2r(d, false)); m_Plan->x3_c2r(in, 0, out, 0, 1, st); }
 }
 
-void SpectralOps::Grad(float* const g[3], const float* f) {
+void SpectralOps::Grad(float* const g[3], const float* f) { Gradients(g[0], 0, spacing(g), f, 0, 1, m_Spec.get()); }
+
+// Gradients of n fields f + j·fs (component d to g + j·gs + d·gc) over `spec`,
+// 3·n half spectra.
+void SpectralOps::Gradients(float* g, int64_t gs, int64_t gc, const float* f, int64_t fs, int n, c32* spec) {
     const Dims& d = m_Opt->domain;
+    const int64_t ss = d.nlc;
     hipStream_t st = m_Opt->stream;
-    c32* s[3] = {m_Spec[0].get(), m_Spec[1].get(), m_Spec[2].get()};
-    { KernelScope k(m_Opt->prof, "fft_x3_r2c", bytes_x3_r2c(d)); m_Plan->x3_r2c(f, s[0], st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", bytes_col(d)); m_Plan->x2(s[0], -1, st); }
-    { KernelScope k(m_Opt->prof, "fft_x1_grad", 32.0 * d.nlc); m_Plan->x1_grad(s[0], s, st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2_n(s, 3, +1, st); }
-    { KernelScope k(m_Opt->prof, "fft_x3_c2r", 3.0 * bytes_x3_c2r(d, false)); m_Plan->x3_c2r_n(s, g, 3, st); }
+    CLR_REQUIRE(n == 1 || gs == 3 * gc, kErrInvalidArgument, "a series' gradients must be equally spaced fields");
+    {
+        KernelScope k(m_Opt->prof, "fft_x3_r2c", n * bytes_x3_r2c(d));
+        m_Plan->x3_r2c(f, fs, spec, 3 * ss, n, st);
+    }
+    { KernelScope k(m_Opt->prof, "fft_x2", n * bytes_col(d)); m_Plan->x2(spec, 3 * ss, n, -1, st); }
+    {
+        KernelScope k(m_Opt->prof, "fft_x1_grad", 32.0 * n * d.nlc);
+        m_Plan->x1_grad(spec, 3 * ss, spec, 3 * ss, ss, n, st);
+    }
+    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * n * bytes_col(d)); m_Plan->x2(spec, ss, 3 * n, +1, st); }
+    {
+        KernelScope k(m_Opt->prof, "fft_x3_c2r", 3.0 * n * bytes_x3_c2r(d, false));
+        m_Plan->x3_c2r(spec, ss, g, gc, 3 * n, st);
+    }
+}
+
+int SpectralOps::SeriesFields(int n) const {
+    const int64_t most = std::max<int64_t>(1, kSeriesPoints / m_Opt->domain.nl);
+    const int groups = static_cast<int>((n + most - 1) / most);
+    return (n + groups - 1) / groups;
+}
+
+void SpectralOps::GradSeries(float* g, const float* f, int n) {
+    const Dims& d = m_Opt->domain;
+    const int per = SeriesFields(n);
+    if (per > 1) m_SeriesSpec.resize(3 * static_cast<size_t>(per) * d.nlc);
+    for (int j = 0; j < n; j += per)
+        Gradients(g + 3 * j * d.nl, 3 * d.nl, d.nl, f + j * d.nl, d.nl, std::min(per, n - j),
+                  per > 1 ? m_SeriesSpec.get() : m_Spec.get());
 }
 
 void SpectralOps::Div(float* out, const float* const v[3]) {
     const Dims& d = m_Opt->domain;
+    const int64_t ss = d.nlc;
     hipStream_t st = m_Opt->stream;
-    c32* s[3] = {m_Spec[0].get(), m_Spec[1].get(), m_Spec[2].get()};
-    { KernelScope k(m_Opt->prof, "fft_x3_r2c", 3.0 * bytes_x3_r2c(d)); m_Plan->x3_r2c_n(v, s, 3, st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2_n(s, 3, -1, st); }
-    { KernelScope k(m_Opt->prof, "fft_x1_div", 32.0 * d.nlc); m_Plan->x1_div(s, s[0], st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", bytes_col(d)); m_Plan->x2(s[0], +1, st); }
-    { KernelScope k(m_Opt->prof, "fft_x3_c2r", bytes_x3_c2r(d, false)); m_Plan->x3_c2r(s[0], out, st); }
+    c32* s = m_Spec.get();
+    {
+        KernelScope k(m_Opt->prof, "fft_x3_r2c", 3.0 * bytes_x3_r2c(d));
+        m_Plan->x3_r2c(v[0], spacing(v), s, ss, 3, st);
+    }
+    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2(s, ss, 3, -1, st); }
+    { KernelScope k(m_Opt->prof, "fft_x1_div", 32.0 * d.nlc); m_Plan->x1_div(s, ss, s, st); }
+    { KernelScope k(m_Opt->prof, "fft_x2", bytes_col(d)); m_Plan->x2(s, 0, 1, +1, st); }
+    { KernelScope k(m_Opt->prof, "fft_x3_c2r", bytes_x3_c2r(d, false)); m_Plan->x3_c2r(s, 0, out, 0, 1, st); }
 }
 
 void SpectralOps::Multiplier3(const SpecParams& sp, const float* const in[3], float* const out[3], float alpha,
                               const float* const add[3], float beta) {
     const Dims& d = m_Opt->domain;
+    const int64_t ss = d.nlc;
     hipStream_t st = m_Opt->stream;
-    c32* s[3] = {m_Spec[0].get(), m_Spec[1].get(), m_Spec[2].get()};
-    { KernelScope k(m_Opt->prof, "fft_x3_r2c", 3.0 * bytes_x3_r2c(d)); m_Plan->x3_r2c_n(in, s, 3, st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2_n(s, 3, -1, st); }
-    { KernelScope k(m_Opt->prof, "fft_x1_mult", 3.0 * bytes_col(d)); m_Plan->x1_multiplier(s, s, 3, sp, st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2_n(s, 3, +1, st); }
+    c32* s = m_Spec.get();
+    {
+        KernelScope k(m_Opt->prof, "fft_x3_r2c", 3.0 * bytes_x3_r2c(d));
+        m_Plan->x3_r2c(in[0], spacing(in), s, ss, 3, st);
+    }
+    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2(s, ss, 3, -1, st); }
+    { KernelScope k(m_Opt->prof, "fft_x1_mult", 3.0 * bytes_col(d)); m_Plan->x1_multiplier(s, ss, 3, sp, st); }
+    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2(s, ss, 3, +1, st); }
     {
         KernelScope k(m_Opt->prof, "fft_x3_c2r", 3.0 * bytes_x3_c2r(d, add != nullptr));
-        m_Plan->x3_c2r_n(s, out, 3, st, alpha, add, beta);
+        m_Plan->x3_c2r(s, ss, out[0], spacing(out), 3, st, alpha, add ? add[0] : nullptr, add ? spacing(add) : 0, beta);
     }
 }
 
 void SpectralOps::Norm3(const SpecParams& sp, const float* const v[3], Reducer* red, int slot) {
     const Dims& d = m_Opt->domain;
+    const int64_t ss = d.nlc;
     hipStream_t st = m_Opt->stream;
-    c32* s[3] = {m_Spec[0].get(), m_Spec[1].get(), m_Spec[2].get()};
+    c32* s = m_Spec.get();
     const int64_t np = m_Plan->x1_norm_partials(3);
     m_NormPartial.resize(static_cast<size_t>(np));
-    { KernelScope k(m_Opt->prof, "fft_x3_r2c", 3.0 * bytes_x3_r2c(d)); m_Plan->x3_r2c_n(v, s, 3, st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2_n(s, 3, -1, st); }
+    {
+        KernelScope k(m_Opt->prof, "fft_x3_r2c", 3.0 * bytes_x3_r2c(d));
+        m_Plan->x3_r2c(v[0], spacing(v), s, ss, 3, st);
+    }
+    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2(s, ss, 3, -1, st); }
     {
         KernelScope k(m_Opt->prof, "fft_x1_norm", 24.0 * d.nlc);
-        m_Plan->x1_norm(s, 3, sp, m_NormPartial.get(), st);
+        m_Plan->x1_norm(s, ss, 3, sp, m_NormPartial.get(), st);
         red->SumPartialsTo(m_NormPartial.get(), static_cast<int>(np), slot);
     }
 }
 
 void SpectralOps::Project(const SpecParams& sp, float* const b[3]) {
     const Dims& d = m_Opt->domain;
+    const int64_t ss = d.nlc, bs = spacing(b);
     hipStream_t st = m_Opt->stream;
-    c32* s[3] = {m_Spec[0].get(), m_Spec[1].get(), m_Spec[2].get()};
-    const float* in[3] = {b[0], b[1], b[2]};
-    { KernelScope k(m_Opt->prof, "fft_x3_r2c", 3.0 * bytes_x3_r2c(d)); m_Plan->x3_r2c_n(in, s, 3, st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2_n(s, 3, -1, st); }
-    { KernelScope k(m_Opt->prof, "fft_x1_project", 3.0 * bytes_col(d)); m_Plan->x1_project(s, sp, st); }
-    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2_n(s, 3, +1, st); }
+    c32* s = m_Spec.get();
+    { KernelScope k(m_Opt->prof, "fft_x3_r2c", 3.0 * bytes_x3_r2c(d)); m_Plan->x3_r2c(b[0], bs, s, ss, 3, st); }
+    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2(s, ss, 3, -1, st); }
+    { KernelScope k(m_Opt->prof, "fft_x1_project", 3.0 * bytes_col(d)); m_Plan->x1_project(s, ss, sp, st); }
+    { KernelScope k(m_Opt->prof, "fft_x2", 3.0 * bytes_col(d)); m_Plan->x2(s, ss, 3, +1, st); }
     {
         // b + F⁻¹[x̂]: the c2r epilogue adds the field in place (the AXPY of
         // src/CLAIREStokes.cpp:536, src/CLAIREDivReg.cpp:452)
         KernelScope k(m_Opt->prof, "fft_x3_c2r", 3.0 * bytes_x3_c2r(d, true));
-        m_Plan->x3_c2r_n(s, b, 3, st, 1.0f, in, 1.0f);
+        m_Plan->x3_c2r(s, ss, b[0], bs, 3, st, 1.0f, b[0], bs, 1.0f);
     }
 }
 
@@ -630,7 +679,7 @@ size_t CLAIRE::DeviceBytes() const {
     const size_t rk4 = m_Opt.rkorder == 4 ? 6 * nl : 0;  // the two RK4 stage sums
     const size_t cont = m_Opt.pdetype == 0 ? nl : 0;      // continuity-equation coefficient
     const size_t rk2 = m_Opt.pdesolver == 0 ? 6 * nl : 0;  // RK2 integrator work
-    return (floats + rk4 + cont + rk2 + scales) * 4 + halves * 2 + 3 * static_cast<size_t>(m_Opt.domain.nlc) * 8;
+    return (floats + rk4 + cont + rk2 + scales) * 4 + halves * 2 + (3 + m_Spectral->SeriesSpectra(m_Opt.nt + 1)) * static_cast<size_t>(m_Opt.domain.nlc) * 8;
 }
 
 void CLAIRE::RequireVelocity() const { CLR_REQUIRE(m_HaveVelocity, kErrState, "velocity field not set"); }
@@ -764,12 +813,7 @@ int CLAIRE::SolveStateEquation() {
 void CLAIRE::EnsureStateGradients() {
     if (!m_StateValid) SolveStateEquation();
     if (m_GradMValid) return;
-    const int64_t nl = m_Opt.domain.nl;
-    for (int j = 0; j <= m_Opt.nt; ++j) {
-        float* gj = m_GradM.get() + 3 * j * nl;
-        float* g[3] = {gj, gj + nl, gj + 2 * nl};
-        m_Spectral->Grad(g, m_State.get() + j * nl);
-    }
+    m_Spectral->GradSeries(m_GradM.get(), m_State.get(), m_Opt.nt + 1);
     m_GradMValid = true;
     m_GradMXValid = m_HalfValid = false;
 }

@@ -327,26 +327,32 @@ __device__ __forceinline__ float spec_multiplier(const SpecParams& p, int w1, in
 // ---------------------------------------------------------------------------
 // x3 pass, real -> half complex.  Rows 2p and 2p+1 are packed as a + i·b.
 // ---------------------------------------------------------------------------
-// Up to three fields per launch: blockIdx.y selects the field (a vector
-// field's components go through one launch instead of three).
+// Several fields per launch, equally spaced in memory: blockIdx.y selects the
+// field (a vector field's components, or the fields of a time series, go through
+// one launch instead of one each).  Spacings are in elements.
 struct R2CPtrs {
-    const float* in[3];
-    c32* out[3];
+    const float* in;
+    int64_t is;
+    c32* out;
+    int64_t os;
 };
 struct C2RPtrs {
-    const c32* in[3];
-    float* out[3];
-    const float* add[3];
+    const c32* in;
+    int64_t is;
+    float* out;
+    int64_t os;
+    const float* add;
+    int64_t as;
 };
-struct ColPtrs {
-    const c32* in[3];
-    c32* out[3];
+struct ColPtrs {  // in place
+    c32* data;
+    int64_t ds;
 };
 
 template <int N>
 __global__ __launch_bounds__(Geo<N>::THREADS) void k_row_r2c(R2CPtrs ptr, int64_t nrows, const c32* __restrict__ tw) {
-    const float* __restrict__ in = ptr.in[blockIdx.y];
-    c32* __restrict__ out = ptr.out[blockIdx.y];
+    const float* __restrict__ in = ptr.in + blockIdx.y * ptr.is;
+    c32* __restrict__ out = ptr.out + blockIdx.y * ptr.os;
     using G = Geo<N>;
     __shared__ c32 s[G::LDS_ELEMS];
     constexpr int V = G::V, T = G::T, R0 = First<typename Plan<N>::Fwd>::value,
@@ -420,9 +426,9 @@ __device__ __forceinline__ void flat_copy(int n, Load&& load, Use&& use) {
 template <int N, bool ADD>
 __global__ __launch_bounds__(Geo<N>::THREADS) void k_row_c2r(C2RPtrs ptr, int64_t nrows, const c32* __restrict__ tw,
                                                              float alpha, float beta) {
-    const c32* __restrict__ in = ptr.in[blockIdx.y];
-    float* __restrict__ out = ptr.out[blockIdx.y];
-    const float* __restrict__ add = ADD ? ptr.add[blockIdx.y] : nullptr;
+    const c32* __restrict__ in = ptr.in + blockIdx.y * ptr.is;
+    float* __restrict__ out = ptr.out + blockIdx.y * ptr.os;
+    const float* __restrict__ add = ADD ? ptr.add + blockIdx.y * ptr.as : nullptr;
     using G = Geo<N>;
     __shared__ c32 s[G::LDS_ELEMS];
     constexpr int V = G::V, T = G::T, R0 = First<typename Plan<N>::Inv>::value,
@@ -601,8 +607,7 @@ __device__ __forceinline__ void bstore_c(spec_rsrc_t r, c32 v, uint32_t voff, ui
 
 template <int N, int DIR>
 __global__ __launch_bounds__(ColGeo<N>::THREADS) void k_col(ColPtrs ptr, ColGeom geo, const c32* __restrict__ tw) {
-    const c32* in = ptr.in[blockIdx.y];  // may equal out (in place): no __restrict__
-    c32* out = ptr.out[blockIdx.y];
+    c32* data = ptr.data + blockIdx.y * ptr.ds;  // in place
     using G = ColGeo<N>;
     __shared__ c32 s[G::LDS_ELEMS];
     using L = typename std::conditional<(DIR < 0), typename Plan<N>::Fwd, typename Plan<N>::Inv>::type;
@@ -618,14 +623,14 @@ __global__ __launch_bounds__(ColGeo<N>::THREADS) void k_col(ColPtrs ptr, ColGeom
     const bool valid = cg < geo.ncols;
     const int64_t base = valid ? col_base<N>(geo, cg) : 0;
     c32 v[V];
-    const spec_rsrc_t rin = spec_rsrc(in, geo.ncols * N), rout = spec_rsrc(out, geo.ncols * N);
+    const spec_rsrc_t rio = spec_rsrc(data, geo.ncols * N);
     const uint32_t es8 = static_cast<uint32_t>(geo.estride) * 8u;
     const uint32_t lane = static_cast<uint32_t>(base) * 8u + static_cast<uint32_t>(t) * es8;
 #pragma unroll
     for (int q = 0; q < V / R0; ++q)
 #pragma unroll
         for (int r = 0; r < R0; ++r) {
-            const c32 x = bload_c(rin, lane, static_cast<uint32_t>(T * q + r * (N / R0)) * es8);
+            const c32 x = bload_c(rio, lane, static_cast<uint32_t>(T * q + r * (N / R0)) * es8);
             v[q * R0 + r] = valid ? x : c32{0.f, 0.f};
         }
     fft_regs<N, DIR>(v, s, ColLayout{G::LD}, c, t, tw);
@@ -634,7 +639,7 @@ __global__ __launch_bounds__(ColGeo<N>::THREADS) void k_col(ColPtrs ptr, ColGeom
         for (int q = 0; q < V / RL; ++q)
 #pragma unroll
             for (int r = 0; r < RL; ++r)
-                bstore_c(rout, v[q * RL + r], lane, static_cast<uint32_t>(T * q + r * (N / RL)) * es8);
+                bstore_c(rio, v[q * RL + r], lane, static_cast<uint32_t>(T * q + r * (N / RL)) * es8);
     }
 }
 
@@ -669,13 +674,19 @@ __device__ __forceinline__ float proj_factor(const SpecParams& p, int k1, int k2
     return opik * lapinvik;
 }
 
-struct Ptr3 {
-    const c32* in[3];
-    c32* out[3];
+// Field f of a pass at in + f·is and out + f·os; in grad mode field f's three
+// components go to out + f·os + d·oc, in div mode the components come from
+// in + d·is.
+struct X1Ptrs {
+    const c32* in;
+    int64_t is;
+    c32* out;
+    int64_t os;
+    int64_t oc;
 };
 
 template <int N, int MODE>
-__global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(Ptr3 ptr, ColGeom geo, const c32* __restrict__ tw,
+__global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(X1Ptrs ptr, ColGeom geo, const c32* __restrict__ tw,
                                                               SpecParams sp, int n2, int n3, int nh) {
     using G = Geo<N>;
     __shared__ c32 s[G::LDS_ELEMS];
@@ -719,9 +730,8 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(Ptr3 ptr, ColGeom 
     };
 
     if constexpr (MODE == kFuseMult) {
-        const int d = blockIdx.y;
         c32 v[V];
-        load_fwd(ptr.in[d], v);
+        load_fwd(ptr.in + blockIdx.y * ptr.is, v);
 #pragma unroll
         for (int q = 0; q < V / RL; ++q) {
             const int j = t + T * q;
@@ -732,10 +742,10 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(Ptr3 ptr, ColGeom 
                 v[q * RL + r] = {v[q * RL + r].x * m, v[q * RL + r].y * m};
             }
         }
-        inv_store(v, ptr.out[d]);
+        inv_store(v, ptr.out + blockIdx.y * ptr.os);
     } else if constexpr (MODE == kFuseGrad) {
         c32 x[V];
-        load_fwd(ptr.in[0], x);
+        load_fwd(ptr.in + blockIdx.y * ptr.is, x);
         const float sc = sp.scale;
 #pragma unroll 1
         for (int d = 0; d < 3; ++d) {
@@ -751,7 +761,7 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(Ptr3 ptr, ColGeom 
                     v[q * RL + r] = {-wd * a.y * sc, wd * a.x * sc};
                 }
             }
-            inv_store(v, ptr.out[d]);
+            inv_store(v, ptr.out + blockIdx.y * ptr.os + d * ptr.oc);
         }
     } else if constexpr (MODE == kFuseDiv) {
         c32 acc[V];
@@ -760,7 +770,7 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(Ptr3 ptr, ColGeom 
 #pragma unroll 1
         for (int d = 0; d < 3; ++d) {
             c32 v[V];
-            load_fwd(ptr.in[d], v);
+            load_fwd(ptr.in + d * ptr.is, v);
 #pragma unroll
             for (int q = 0; q < V / RL; ++q) {
                 const int j = t + T * q;
@@ -778,13 +788,13 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(Ptr3 ptr, ColGeom 
         const float sc = sp.scale;
 #pragma unroll
         for (int i = 0; i < V; ++i) acc[i] = {acc[i].x * sc, acc[i].y * sc};
-        inv_store(acc, ptr.out[0]);
+        inv_store(acc, ptr.out);
     } else {
         // projection of a vector field: all three components at every mode
         c32 a[V], b[V], e[V];
-        load_fwd(ptr.in[0], a);
-        load_fwd(ptr.in[1], b);
-        load_fwd(ptr.in[2], e);
+        load_fwd(ptr.in, a);
+        load_fwd(ptr.in + ptr.is, b);
+        load_fwd(ptr.in + 2 * ptr.is, e);
         const float sc = sp.scale;
         const float g2 = static_cast<float>(w2), g3 = static_cast<float>(w3);
 #pragma unroll
@@ -805,9 +815,9 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(Ptr3 ptr, ColGeom 
                 a[i] = {cre * -g1, cim * g1};
             }
         }
-        inv_store(a, ptr.out[0]);
-        inv_store(b, ptr.out[1]);
-        inv_store(e, ptr.out[2]);
+        inv_store(a, ptr.out);
+        inv_store(b, ptr.out + ptr.os);
+        inv_store(e, ptr.out + 2 * ptr.os);
     }
 }
 
@@ -834,7 +844,7 @@ __device__ __forceinline__ double norm_factor(const SpecParams& p, double k2) {
 }
 
 template <int N>
-__global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_norm(Ptr3 ptr, ColGeom geo, const c32* __restrict__ tw,
+__global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_norm(X1Ptrs ptr, ColGeom geo, const c32* __restrict__ tw,
                                                              SpecParams sp, int n2, int n3, int nh,
                                                              double* __restrict__ partial) {
     using G = Geo<N>;
@@ -851,7 +861,7 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_norm(Ptr3 ptr, ColGeom g
     const int w2 = wavenum(k2, n2), w3 = wavenum(k3, n3);
     const uint32_t es8 = static_cast<uint32_t>(geo.estride) * 8u;
     const uint32_t lane = static_cast<uint32_t>(base) * 8u + static_cast<uint32_t>(t) * es8;
-    const spec_rsrc_t r_in = spec_rsrc(ptr.in[blockIdx.y], geo.ncols * N);
+    const spec_rsrc_t r_in = spec_rsrc(ptr.in + blockIdx.y * ptr.is, geo.ncols * N);
     c32 v[V];
 #pragma unroll
     for (int q = 0; q < V / R0; ++q)
@@ -927,7 +937,7 @@ struct RowC2R {
         const int64_t npairs = (nrows + 1) / 2;
         const int64_t blocks = (npairs + G::B - 1) / G::B;
         const dim3 grid(static_cast<unsigned>(blocks), ncomp);
-        if (p.add[0] || p.add[1] || p.add[2])
+        if (p.add)
             hipLaunchKernelGGL((k_row_c2r<N, true>), grid, dim3(G::THREADS), 0, st, p, nrows, tw, alpha, beta);
         else
             hipLaunchKernelGGL((k_row_c2r<N, false>), grid, dim3(G::THREADS), 0, st, p, nrows, tw, alpha, beta);
@@ -948,22 +958,15 @@ struct ColPass {
     }
 };
 
-ColPtrs col_ptrs(c32* const data[], int ncomp) {
-    CLR_REQUIRE(ncomp >= 1 && ncomp <= 3, kErrInvalidArgument, "1 to 3 fields per FFT pass");
-    ColPtrs p{};
-    for (int c = 0; c < ncomp; ++c) p.in[c] = p.out[c] = data[c];
-    return p;
-}
-
 template <int N>
 struct X1Fused {
-    static void go(int mode, Ptr3 p, ColGeom geo, const c32* tw, SpecParams sp, int n2, int n3, int nh, int ncomp,
+    static void go(int mode, X1Ptrs p, ColGeom geo, const c32* tw, SpecParams sp, int n2, int n3, int nh, int nfields,
                    hipStream_t st) {
         using G = Geo<N>;
         CLR_REQUIRE(geo.ncols * N * 8 < (int64_t(1) << 31), kErrInvalidArgument,
                     "spectrum field too large for 32-bit buffer offsets");
         const int64_t blocks = (geo.ncols + G::B - 1) / G::B;
-        dim3 grid(static_cast<unsigned>(blocks), mode == kFuseMult ? ncomp : 1);
+        dim3 grid(static_cast<unsigned>(blocks), mode == kFuseMult || mode == kFuseGrad ? nfields : 1);
         switch (mode) {
             case kFuseMult:
                 hipLaunchKernelGGL((k_x1_fused<N, kFuseMult>), grid, dim3(G::THREADS), 0, st, p, geo, tw, sp, n2, n3, nh);
@@ -989,7 +992,7 @@ struct X1Blocks {
 
 template <int N>
 struct X1Norm {
-    static void go(Ptr3 p, ColGeom geo, const c32* tw, SpecParams sp, int n2, int n3, int nh, int ncomp, double* partial,
+    static void go(X1Ptrs p, ColGeom geo, const c32* tw, SpecParams sp, int n2, int n3, int nh, int ncomp, double* partial,
                    hipStream_t st) {
         using G = Geo<N>;
         CLR_REQUIRE(geo.ncols * N * 8 < (int64_t(1) << 31), kErrInvalidArgument,
@@ -1056,71 +1059,31 @@ FFTPlan3D::~FFTPlan3D() {
         if (tw[a]) (void)hipFree(tw[a]);
 }
 
-void FFTPlan3D::r2c(const float* in, c32* out, hipStream_t st) const {
-    x3_r2c(in, out, st);
-    x2(out, -1, st);
-    x1(out, -1, st);
+void FFTPlan3D::x3_r2c(const float* in, int64_t is, c32* out, int64_t os, int n, hipStream_t st) const {
+    CLR_REQUIRE(n >= 1 && n <= 65535, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
+    const R2CPtrs p{in, is, out, os};
+    dispatch_n<RowR2C>(dims.n[2], p, n, static_cast<int64_t>(dims.n[0]) * dims.n[1], tw[2], st);
 }
-
-void FFTPlan3D::c2r(c32* in, float* out, hipStream_t st, float alpha, const float* add, float beta) const {
-    x1(in, +1, st);
-    x2(in, +1, st);
-    x3_c2r(in, out, st, alpha, add, beta);
+void FFTPlan3D::x3_c2r(const c32* in, int64_t is, float* out, int64_t os, int n, hipStream_t st, float alpha,
+                       const float* add, int64_t as, float beta) const {
+    CLR_REQUIRE(n >= 1 && n <= 65535, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
+    const C2RPtrs p{in, is, out, os, add, as};
+    dispatch_n<RowC2R>(dims.n[2], p, n, static_cast<int64_t>(dims.n[0]) * dims.n[1], tw[2], alpha, beta, st);
 }
-
-void FFTPlan3D::x3_r2c_n(const float* const in[], c32* const out[], int ncomp, hipStream_t st) const {
-    CLR_REQUIRE(ncomp >= 1 && ncomp <= 3, kErrInvalidArgument, "1 to 3 fields per FFT pass");
-    R2CPtrs p{};
-    for (int c = 0; c < ncomp; ++c) {
-        p.in[c] = in[c];
-        p.out[c] = out[c];
-    }
-    dispatch_n<RowR2C>(dims.n[2], p, ncomp, static_cast<int64_t>(dims.n[0]) * dims.n[1], tw[2], st);
-}
-void FFTPlan3D::x3_c2r_n(const c32* const in[], float* const out[], int ncomp, hipStream_t st, float alpha,
-                         const float* const add[], float beta) const {
-    CLR_REQUIRE(ncomp >= 1 && ncomp <= 3, kErrInvalidArgument, "1 to 3 fields per FFT pass");
-    C2RPtrs p{};
-    for (int c = 0; c < ncomp; ++c) {
-        p.in[c] = in[c];
-        p.out[c] = out[c];
-        p.add[c] = add ? add[c] : nullptr;
-    }
-    dispatch_n<RowC2R>(dims.n[2], p, ncomp, static_cast<int64_t>(dims.n[0]) * dims.n[1], tw[2], alpha, beta, st);
-}
-void FFTPlan3D::x2_n(c32* const data[], int ncomp, int dir, hipStream_t st) const {
-    dispatch_n<ColPass>(dims.n[1], col_ptrs(data, ncomp), ncomp, geom_x2(dims), dir, tw[1], st);
-}
-
-void FFTPlan3D::x3_r2c(const float* in, c32* out, hipStream_t st) const {
-    const float* i[1] = {in};
-    c32* o[1] = {out};
-    x3_r2c_n(i, o, 1, st);
-}
-void FFTPlan3D::x3_c2r(const c32* in, float* out, hipStream_t st, float alpha, const float* add, float beta) const {
-    const c32* i[1] = {in};
-    float* o[1] = {out};
-    const float* a[1] = {add};
-    x3_c2r_n(i, o, 1, st, alpha, a, beta);
-}
-void FFTPlan3D::x2(c32* data, int dir, hipStream_t st) const {
-    c32* d[1] = {data};
-    x2_n(d, 1, dir, st);
+void FFTPlan3D::x2(c32* data, int64_t ds, int n, int dir, hipStream_t st) const {
+    CLR_REQUIRE(n >= 1 && n <= 65535, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
+    const ColPtrs p{data, ds};
+    dispatch_n<ColPass>(dims.n[1], p, n, geom_x2(dims), dir, tw[1], st);
 }
 void FFTPlan3D::x1(c32* data, int dir, hipStream_t st) const {
-    c32* d[1] = {data};
-    dispatch_n<ColPass>(dims.n[0], col_ptrs(d, 1), 1, geom_x1(dims), dir, tw[0], st);
+    const ColPtrs p{data, 0};
+    dispatch_n<ColPass>(dims.n[0], p, 1, geom_x1(dims), dir, tw[0], st);
 }
 
-void FFTPlan3D::x1_multiplier(const c32* const in[3], c32* const out[3], int ncomp, const SpecParams& sp,
-                              hipStream_t st) const {
-    Ptr3 p{};
-    for (int d = 0; d < ncomp; ++d) {
-        p.in[d] = in[d];
-        p.out[d] = out[d];
-    }
+void FFTPlan3D::x1_multiplier(c32* data, int64_t ds, int n, const SpecParams& sp, hipStream_t st) const {
+    const X1Ptrs p{data, ds, data, ds, 0};
     dispatch_n<X1Fused>(dims.n[0], static_cast<int>(kFuseMult), p, geom_x1(dims), tw[0], sp, dims.n[1], dims.n[2],
-                        dims.nh, ncomp, st);
+                        dims.nh, n, st);
 }
 
 int64_t FFTPlan3D::x1_norm_partials(int ncomp) const {
@@ -1129,40 +1092,34 @@ int64_t FFTPlan3D::x1_norm_partials(int ncomp) const {
     return blocks * ncomp;
 }
 
-void FFTPlan3D::x1_norm(const c32* const in[3], int ncomp, const SpecParams& sp, double* partial,
+void FFTPlan3D::x1_norm(const c32* in, int64_t is, int n, const SpecParams& sp, double* partial,
                         hipStream_t st) const {
-    CLR_REQUIRE(ncomp >= 1 && ncomp <= 3, kErrInvalidArgument, "1 to 3 fields per FFT pass");
-    Ptr3 p{};
-    for (int d = 0; d < ncomp; ++d) p.in[d] = in[d];
-    dispatch_n<X1Norm>(dims.n[0], p, geom_x1(dims), tw[0], sp, dims.n[1], dims.n[2], dims.nh, ncomp, partial, st);
+    const X1Ptrs p{in, is, nullptr, 0, 0};
+    dispatch_n<X1Norm>(dims.n[0], p, geom_x1(dims), tw[0], sp, dims.n[1], dims.n[2], dims.nh, n, partial, st);
 }
 
-void FFTPlan3D::x1_grad(const c32* in, c32* const out[3], hipStream_t st) const {
-    Ptr3 p{};
-    p.in[0] = in;
-    for (int d = 0; d < 3; ++d) p.out[d] = out[d];
+void FFTPlan3D::x1_grad(const c32* in, int64_t is, c32* out, int64_t os, int64_t oc, int n, hipStream_t st) const {
+    CLR_REQUIRE(n >= 1 && n <= 65535, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
+    const X1Ptrs p{in, is, out, os, oc};
     SpecParams sp{};
     sp.scale = dims.scale;
     dispatch_n<X1Fused>(dims.n[0], static_cast<int>(kFuseGrad), p, geom_x1(dims), tw[0], sp, dims.n[1], dims.n[2],
-                        dims.nh, 3, st);
+                        dims.nh, n, st);
 }
 
-void FFTPlan3D::x1_project(c32* const data[3], const SpecParams& sp, hipStream_t st) const {
+void FFTPlan3D::x1_project(c32* data, int64_t ds, const SpecParams& sp, hipStream_t st) const {
     CLR_REQUIRE(sp.op == kOpProjStokes || sp.op == kOpProjRelaxed, kErrInvalidArgument, "not a projection");
-    Ptr3 p{};
-    for (int d = 0; d < 3; ++d) p.in[d] = p.out[d] = data[d];
+    const X1Ptrs p{data, ds, data, ds, 0};
     dispatch_n<X1Fused>(dims.n[0], static_cast<int>(kFuseProject), p, geom_x1(dims), tw[0], sp, dims.n[1], dims.n[2],
-                        dims.nh, 3, st);
+                        dims.nh, 1, st);
 }
 
-void FFTPlan3D::x1_div(const c32* const in[3], c32* out, hipStream_t st) const {
-    Ptr3 p{};
-    for (int d = 0; d < 3; ++d) p.in[d] = in[d];
-    p.out[0] = out;
+void FFTPlan3D::x1_div(const c32* in, int64_t is, c32* out, hipStream_t st) const {
+    const X1Ptrs p{in, is, out, 0, 0};
     SpecParams sp{};
     sp.scale = dims.scale;
     dispatch_n<X1Fused>(dims.n[0], static_cast<int>(kFuseDiv), p, geom_x1(dims), tw[0], sp, dims.n[1], dims.n[2],
-                        dims.nh, 3, st);
+                        dims.nh, 1, st);
 }
 
 }  // namespace claire_amd

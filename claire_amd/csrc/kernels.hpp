@@ -28,36 +28,30 @@ class FFTPlan3D {
     FFTPlan3D(const FFTPlan3D&) = delete;
     FFTPlan3D& operator=(const FFTPlan3D&) = delete;
 
-    // Full transforms (unnormalized).  c2r overwrites its input.
-    // c2r epilogue: out = alpha·F⁻¹(in) + beta·add (add may be null).
-    void r2c(const float* in, c32* out, hipStream_t st) const;
-    void c2r(c32* in, float* out, hipStream_t st, float alpha = 1.f, const float* add = nullptr, float beta = 0.f) const;
-
-    // Individual passes.
-    void x3_r2c(const float* in, c32* out, hipStream_t st) const;
-    void x3_c2r(const c32* in, float* out, hipStream_t st, float alpha = 1.f, const float* add = nullptr,
-                float beta = 0.f) const;
-    void x2(c32* data, int dir, hipStream_t st) const;
+    // Individual passes over n fields in one launch, field f at in + f·is (and
+    // out + f·os, add + f·as): a vector field's components or a time series.
+    void x3_r2c(const float* in, int64_t is, c32* out, int64_t os, int n, hipStream_t st) const;
+    // out = alpha·x + beta·add (add may be null, or equal out with as = os)
+    void x3_c2r(const c32* in, int64_t is, float* out, int64_t os, int n, hipStream_t st, float alpha = 1.f,
+                const float* add = nullptr, int64_t as = 0, float beta = 0.f) const;
+    void x2(c32* data, int64_t ds, int n, int dir, hipStream_t st) const;
     void x1(c32* data, int dir, hipStream_t st) const;
-    // The same passes over 1 to 3 fields in one launch (add may be null;
-    // add[c] may equal out[c] but no other field's out).
-    void x3_r2c_n(const float* const in[], c32* const out[], int ncomp, hipStream_t st) const;
-    void x3_c2r_n(const c32* const in[], float* const out[], int ncomp, hipStream_t st, float alpha = 1.f,
-                  const float* const add[] = nullptr, float beta = 0.f) const;
-    void x2_n(c32* const data[], int ncomp, int dir, hipStream_t st) const;
     // Fused x1 passes (forward x1, k-space operator, inverse x1).
-    void x1_multiplier(const c32* const in[3], c32* const out[3], int ncomp, const SpecParams& sp, hipStream_t st) const;
-    void x1_grad(const c32* in, c32* const out[3], hipStream_t st) const;
-    void x1_div(const c32* const in[3], c32* out, hipStream_t st) const;
+    void x1_multiplier(c32* data, int64_t ds, int n, const SpecParams& sp, hipStream_t st) const;
+    // component d of field f's gradient at out + f·os + d·oc; in + f·is may be
+    // one of the three
+    void x1_grad(const c32* in, int64_t is, c32* out, int64_t os, int64_t oc, int n, hipStream_t st) const;
+    // out (may equal in) = divergence of the field with components in + d·is
+    void x1_div(const c32* in, int64_t is, c32* out, hipStream_t st) const;
     // Forward x1 pass that ends in a sum: per block Σ c(k3)·m(k)²·|x̂(k)|² over
     // its columns, m² the regularization norm's (sp.norm; sp.beta1 = β1 for H1,
-    // √β1 for H2), so that the sum of all x1_norm_partials(ncomp) values over N
-    // is Σ_x |M x|² of the ncomp fields.
-    void x1_norm(const c32* const in[3], int ncomp, const SpecParams& sp, double* partial, hipStream_t st) const;
-    int64_t x1_norm_partials(int ncomp) const;
+    // √β1 for H2), so that the sum of all x1_norm_partials(n) values over N
+    // is Σ_x |M x|² of the n fields.
+    void x1_norm(const c32* in, int64_t is, int n, const SpecParams& sp, double* partial, hipStream_t st) const;
+    int64_t x1_norm_partials(int n) const;
     // Projection of a vector field (sp.op kOpProjStokes or kOpProjRelaxed):
-    // x̂_i = g_i·scale·m·(g·b̂) in place of the three spectra.
-    void x1_project(c32* const data[3], const SpecParams& sp, hipStream_t st) const;
+    // x̂_i = g_i·scale·m·(g·b̂) in place of the three spectra data + d·ds.
+    void x1_project(c32* data, int64_t ds, const SpecParams& sp, hipStream_t st) const;
 
     Dims dims;
 

@@ -96,18 +96,15 @@ void grad_noalloc(const int nx[3], const float* f, float* g, hipStream_t st) {
     c32* tw_base = reinterpret_cast<c32*>(base);
     c32* const tw[3] = {tw_base + twiddle_offset(nx[0]), tw_base + twiddle_offset(nx[1]),
                         tw_base + twiddle_offset(nx[2])};
-    const size_t spec_bytes = round_up(static_cast<size_t>(d.nlc) * sizeof(c32), kSpectrumAlign);
-    c32* s[3];
-    for (int i = 0; i < 3; ++i) s[i] = reinterpret_cast<c32*>(base + kTwiddleBytes + i * spec_bytes);
+    const int64_t ss = static_cast<int64_t>(round_up(static_cast<size_t>(d.nlc) * sizeof(c32), kSpectrumAlign) / sizeof(c32));
+    c32* spec = reinterpret_cast<c32*>(base + kTwiddleBytes);
     const FFTPlan3D plan(d, tw);
     // the launches of SpectralOps::Grad, in the same order
-    const int64_t nl = d.nl;
-    float* out[3] = {g, g + nl, g + 2 * nl};
-    plan.x3_r2c(f, s[0], st);
-    plan.x2(s[0], -1, st);
-    plan.x1_grad(s[0], s, st);
-    plan.x2_n(s, 3, +1, st);
-    plan.x3_c2r_n(s, out, 3, st);
+    plan.x3_r2c(f, 0, spec, 0, 1, st);
+    plan.x2(spec, 0, 1, -1, st);
+    plan.x1_grad(spec, 0, spec, 0, ss, 1, st);
+    plan.x2(spec, ss, 3, +1, st);
+    plan.x3_c2r(spec, ss, g, d.nl, 3, st);
 }
 
 }  // namespace claire_amd
