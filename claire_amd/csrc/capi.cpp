@@ -556,7 +556,7 @@ int clr_interp_points(clr_ctx* ctx, const float* f, const float* X, float* out) 
         CLR_REQUIRE(out != f, claire_amd::kErrInvalidArgument, "interpolation output must not alias the field");
         reg::CLAIRE& c = C(ctx);
         reg::KernelScope k(c.Opt().prof, "gather_scalar", 20.0 * c.Opt().domain.nl);
-        claire_amd::launch_gather1(claire_amd::gather_dims(c.Opt().domain), f, X, out, c.Opt().stream);
+        claire_amd::launch_points_gather(claire_amd::gather_dims(c.Opt().domain), f, X, out, c.Opt().stream);
         check_hip_launch();
     });
 }

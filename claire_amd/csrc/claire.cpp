@@ -500,9 +500,8 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
     const float* vc[3] = {v->m_X1, v->m_X2, v->m_X3};
     const float sigma = w == 0 ? 1.0f : -1.0f;
     const float ht = m_Opt->GetTimeStepSize();
-    const int dmax = lds_gather_max_displacement();
     int db = m_PredBound[w];
-    if (db <= dmax && !(w == 0 && m_PredInPlan)) {
+    if (plan_gather_lds(g, db, 3) && !(w == 0 && m_PredInPlan)) {
         // bytes: v read (12) + plan written (12) per point
         KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 24.0 * nl);
         launch_predictor_plan(m_Opt->domain, vc, sigma, PredictorStep(), P, m_Opt->stream);
@@ -513,7 +512,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
         m_F2.resize(n);
         float* const fbuf[4] = {nullptr, m_F.get(), m_F2.get(), nullptr};
         for (int stage = 1; stage <= 3; ++stage) {
-            if (db <= dmax) {
+            if (plan_gather_lds(g, db, 3)) {
                 {
                     // 3 × (plan 12 + gathered v 4 + aux 4 + next point 4 (+ f 4)) per point
                     KernelScope k(m_Opt->prof, "gather_traj_rk4", (stage < 3 ? 84.0 : 72.0) * nl);
@@ -525,14 +524,14 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
                 KernelScope k(m_Opt->prof, "gather_plan", 24.0 * nl);
                 db = launch_make_plan(g, X, P, m_PlanMax.get(), m_Opt->stream);
             } else {
-                // this stage's point is out of the LDS window, and so, nearly
+                // this stage's point is not for the LDS gathers, and so, nearly
                 // always, are the later stages' (their plans are not formed)
                 KernelScope k(m_Opt->prof, "gather_traj_rk4", 48.0 * nl);
                 launch_trajectory_rk4_stage(stage, m_Opt->domain, vc, sigma, ht, X, fbuf[stage - 1], fbuf[stage],
                                             m_Opt->stream);
             }
         }
-    } else if (db <= dmax) {
+    } else if (plan_gather_lds(g, db, 3)) {
         // 3 × (plan 12 + gathered v 4 + v at the point 4 + X component 4) per point
         KernelScope k(m_Opt->prof, "gather_traj_rk2", 72.0 * nl);
         launch_lds_traj_rk2_corrector(m_Opt->domain, P, db, vc, sigma, ht, X, m_Opt->stream);

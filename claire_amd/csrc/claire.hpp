@@ -338,8 +338,7 @@ class SemiLagrangian {
     // Interpolation plan of the trajectory (Interp3_Plan after scatter):
     // packed foot points (3 words per point), the raw foot points and the
     // per-axis stencil displacement bound in cells.  Gathers along it use the
-    // LDS-staged kernels when the bound is at most
-    // lds_gather_max_displacement(), else the direct kernels.
+    // LDS-staged kernels where plan_gather_lds says so, else the direct kernels.
     claire_amd::TrajectoryPlan Plan(const std::string& flag) const;
     bool HasTrajectory(const std::string& flag) const;
     int DisplacementBound(const std::string& flag) const { return m_D[Which(flag)]; }

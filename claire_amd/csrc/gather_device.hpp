@@ -112,6 +112,12 @@ __device__ __forceinline__ void setup_stencil_u(const float u[3], const GatherDi
     setup_axis_u(u[2], g.n3, S.a3);
 }
 
+// Σ_c w[c]·f_c with the FMA chain starting at node 1: the order of every
+// contraction but that of the pair-layout gather within its window.
+__device__ __forceinline__ float row_sum(const float w[4], float f0, float f1, float f2, float f3) {
+    return fmaf(w[3], f3, fmaf(w[2], f2, fmaf(w[0], f0, w[1] * f1)));
+}
+
 // Σ_a w1[a] Σ_b w2[b] Σ_c w3[c] f[i1_a, i2_b, i3_c] for ND fields sharing the
 // stencil, read straight from global memory.
 template <int ND>
@@ -133,11 +139,10 @@ __device__ __forceinline__ void eval_stencil(const float* const f[ND], const Ste
                 float r;
                 if (contig) {
                     const f4u q = *reinterpret_cast<const f4u*>(f[d] + off + S.a3.idx[0]);
-                    r = S.a3.w[0] * q.x + S.a3.w[1] * q.y + S.a3.w[2] * q.z + S.a3.w[3] * q.w;
+                    r = row_sum(S.a3.w, q.x, q.y, q.z, q.w);
                 } else {
                     const float* row = f[d] + off;
-                    r = S.a3.w[0] * row[S.a3.idx[0]] + S.a3.w[1] * row[S.a3.idx[1]] + S.a3.w[2] * row[S.a3.idx[2]] +
-                        S.a3.w[3] * row[S.a3.idx[3]];
+                    r = row_sum(S.a3.w, row[S.a3.idx[0]], row[S.a3.idx[1]], row[S.a3.idx[2]], row[S.a3.idx[3]]);
                 }
                 sa[d] += S.a2.w[b] * r;
             }
@@ -175,6 +180,25 @@ struct __attribute__((packed, aligned(4))) PlanPt {
 
 __device__ __forceinline__ float plan_t(uint32_t w) { return __uint_as_float((w & 0x7FFFFFu) | 0x3F800000u); }
 __device__ __forceinline__ int plan_off(uint32_t w) { return static_cast<int>(w) >> 23; }
+
+// Stencil of the point (i1, i2, i3) from its plan words.
+__device__ __forceinline__ void plan_axis(uint32_t w, int i, int n, Axis& A) {
+    lagrange_weights(plan_t(w), A.w);
+    int k = i + plan_off(w);  // in [−n/2, 3n/2)
+    k += (k < 0) ? n : 0;
+    k -= (k >= n) ? n : 0;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        A.idx[a] = k;
+        k = (k + 1 == n) ? 0 : k + 1;
+    }
+}
+__device__ __forceinline__ void plan_stencil(const uint32_t w[3], int i1, int i2, int i3, const GatherDims& g,
+                                             Stencil& S) {
+    plan_axis(w[0], i1, g.n1, S.a1);
+    plan_axis(w[1], i2, g.n2, S.a2);
+    plan_axis(w[2], i3, g.n3, S.a3);
+}
 
 // Encodes one axis; returns false when u is not a finite, wrapped coordinate.
 __device__ __forceinline__ bool plan_encode(float u, int idx, int n, uint32_t& w, int& off) {
@@ -293,6 +317,7 @@ struct EpiTrajRk2 {
     int64_t zstride;
     float hx0, hx1, hx2;  // grid spacings
     float shth;  // σ·ht/2
+    bool far;    // bound above kNearBound: x rounded first, the order of k_traj_rk2
     int z;
     float hz;  // spacing of axis z, set by select
     __device__ void select(int zz) {
@@ -307,8 +332,8 @@ struct EpiTrajRk2 {
     __device__ float* outp() const { return out; }
     __device__ float apply_at(float vx, float vl, int i1, int i2, int i3) const {
         const int idx = z == 0 ? i1 : (z == 1 ? i2 : i3);
-        const float x = hz * static_cast<float>(idx);
-        const float t = x - shth * (vx + vl);
+        const float i = static_cast<float>(idx), u = vx + vl;
+        const float t = far ? fmaf(-shth, u, hz * i) : fmaf(hz, i, -(shth * u));
         return static_cast<float>(over_2pi(static_cast<double>(t)));
     }
 };
@@ -334,6 +359,7 @@ struct EpiTrajRk4 {
     float hx0, hx1, hx2;  // grid spacings
     float step;  // σ·ht/2 (stage 1), σ·ht (stage 2)
     double s6;   // σ·(ht/6) (stage 3)
+    bool far;    // stage 1 as in EpiTrajRk2
     int z;
     float hz;  // spacing of axis z, set by select
     __device__ void select(int zz) {
@@ -350,12 +376,12 @@ struct EpiTrajRk4 {
     __device__ float* outp2() const { return f; }
     __device__ float apply_at(float vx, float av, int i1, int i2, int i3) const {
         const int idx = z == 0 ? i1 : (z == 1 ? i2 : i3);
-        const float x = hz * static_cast<float>(idx);
+        const float i = static_cast<float>(idx);
         if constexpr (STAGE < 3) {
-            const float t = x - step * vx;
+            const float t = STAGE == 1 && far ? fmaf(-step, vx, hz * i) : fmaf(hz, i, -(step * vx));
             return static_cast<float>(over_2pi(static_cast<double>(t)));
         } else {
-            const float fs = av + vx;
+            const float x = hz * i, fs = av + vx;
             return static_cast<float>(over_2pi(static_cast<double>(x) - s6 * static_cast<double>(fs)));
         }
     }

@@ -12,7 +12,9 @@
 //   * LDS holds a ring of input planes, each the tile plus a halo of D+1
 //     (low side) and D+2 (high side) cells in x2 and x3, where D is the exact
 //     per-axis stencil displacement bound of the plan (D <= 2 covers CFL 2),
-//     so every stencil of the tile lies inside the ring by construction;
+//     so every stencil of the tile lies inside the ring by construction; larger
+//     displacements, and raw query points, take windows centred per block, with
+//     the few points outside them read from global memory (see PointMode);
 //   * the ring has one spare slot: while the block evaluates plane x1 the
 //     global loads of plane x1+D+3 and of the next plane's query points are
 //     in flight and land in the spare slot / registers afterwards, so each
@@ -41,11 +43,11 @@ using namespace gather;
 constexpr int kLT2 = 16;        // tile extent in x2
 constexpr int kLThreads = 512;  // 8 waves; wave w covers tile rows 2w and 2w+1
 
-// LDS plane geometry for displacement bound D.  A plane holds E2 rows of E3
-// valid columns at a row pitch that is a multiple of 32 dwords: a wave reads
-// two tile rows of 32 points each (one row per half-wave), so lanes whose
-// stencils start on different rows or planes still hit different banks
-// unless their columns collide mod 32.
+// LDS plane geometry of the one-value layout for displacement bound D.  A plane
+// holds E2 rows of E3 valid columns at a row pitch that is a multiple of 32
+// dwords: a wave reads two tile rows of 32 points each (one row per half-wave),
+// so lanes whose stencils start on different rows or planes still hit different
+// banks unless their columns collide mod 32.
 //   D <= 2: a 16 × 32 tile, one point per thread, 53 KB of LDS -- three
 //           blocks (24 waves) per CU;
 //   D <= 4: a 16 × 64 tile, two points per thread 32 columns apart, 135 KB.
@@ -123,6 +125,7 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
     GatherDims g, const PlanPt* __restrict__ plan, const float* __restrict__ fbase, int64_t fzstride, Epi epi,
     int nblocks, int chunk) {
     using G = LdsGeo<D>;
+    constexpr int PTS = G::PTS;
     __shared__ float lds[G::W * G::P];
     const int tid = threadIdx.x;
     const int nt3 = (g.n3 + G::LT3 - 1) / G::LT3;
@@ -172,12 +175,12 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
     const int lane = tid & 63;
     const int lx2 = 2 * (tid >> 6) + (lane >> 5);
     const int x2 = t2 * kLT2 + lx2;
-    uint32_t off[G::PTS];
-    int rc4[G::PTS];
-    bool valid[G::PTS];
-    int x3s[G::PTS];
+    uint32_t off[PTS];
+    int rc4[PTS];
+    bool valid[PTS];
+    int x3s[PTS];
 #pragma unroll
-    for (int k = 0; k < G::PTS; ++k) {
+    for (int k = 0; k < PTS; ++k) {
         const int lx3 = (lane & 31) + 32 * k;
         const int x3 = t3 * G::LT3 + lx3;
         x3s[k] = x3;
@@ -211,12 +214,12 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
     // Query points of plane x1 live in (qa, aa) or (qb, ab); the loop below
     // alternates the two so that the prefetch of the next plane's points
     // needs no register copies.
-    PlanPt qa[G::PTS], qb[G::PTS];
-    float aa[G::PTS], ab[G::PTS];
+    PlanPt qa[PTS], qb[PTS];
+    float aa[PTS], ab[PTS];
     {
         const uint32_t pb = static_cast<uint32_t>(x1s) * plane4;
 #pragma unroll
-        for (int k = 0; k < G::PTS; ++k) {
+        for (int k = 0; k < PTS; ++k) {
             qa[k] = bload_plan(rp, 3u * off[k], 3u * pb);
             aa[k] = Epi::kHasAux ? bload_once(ra, off[k], pb) : 0.0f;
         }
@@ -238,8 +241,8 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
     // periodic index of plane x1 + HHI + 2, advanced by one per step (a
     // scalar modulo per step costs about 20 scalar instructions)
     int xf = pmod(x1s + G::HHI + 2, g.n1);
-    auto step = [&](int x1, const PlanPt (&cur)[G::PTS], const float (&caux)[G::PTS], PlanPt (&nxt)[G::PTS],
-                    float (&naux)[G::PTS], const float (&pre)[G::FILL], float (&pnext)[G::FILL]) {
+    auto step = [&](int x1, const PlanPt (&cur)[PTS], const float (&caux)[PTS], PlanPt (&nxt)[PTS],
+                    float (&naux)[PTS], const float (&pre)[G::FILL], float (&pnext)[G::FILL]) {
         // Prefetch for the next steps, unconditionally (past the chunk end it
         // reloads a plane of this chunk; the values are never used).
         const int xn = (x1 + 1 < x1e) ? x1 + 1 : x1;
@@ -252,7 +255,7 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
         {
             const uint32_t pb = static_cast<uint32_t>(xn) * plane4;
 #pragma unroll
-            for (int k = 0; k < G::PTS; ++k) {
+            for (int k = 0; k < PTS; ++k) {
                 nxt[k] = bload_plan(rp, 3u * off[k], 3u * pb);
                 naux[k] = Epi::kHasAux ? bload_once(ra, off[k], pb) : 0.0f;
             }
@@ -262,10 +265,10 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
         // four planes of each point.  The plan's bound keeps every offset
         // within the ring; the clamps only pin LDS addresses inside the
         // allocation.
-        float w1[G::PTS][4], w2[G::PTS][4], w3[G::PTS][4];
-        int base[G::PTS][4], base3[G::PTS][4];
+        float w1[PTS][4], w2[PTS][4], w3[PTS][4];
+        int base[PTS][4], base3[PTS][4];
 #pragma unroll
-        for (int k = 0; k < G::PTS; ++k) {
+        for (int k = 0; k < PTS; ++k) {
             lagrange_weights(plan_t(cur[k].w[0]), w1[k]);
             lagrange_weights(plan_t(cur[k].w[1]), w2[k]);
             lagrange_weights(plan_t(cur[k].w[2]), w3[k]);
@@ -281,18 +284,18 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
 #pragma unroll
             for (int a = 0; a < 4; ++a) base3[k][a] = opaque(base[k][a] + 3 * 4 * G::PITCH);
         }
-        float v[G::PTS];
+        float v[PTS];
 #pragma unroll
-        for (int k = 0; k < G::PTS; ++k) v[k] = 0.f;
+        for (int k = 0; k < PTS; ++k) v[k] = 0.f;
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
-            float sa[G::PTS];
+            float sa[PTS];
 #pragma unroll
-            for (int k = 0; k < G::PTS; ++k) sa[k] = 0.f;
+            for (int k = 0; k < PTS; ++k) sa[k] = 0.f;
 #pragma unroll
             for (int b = 0; b < 4; ++b) {
 #pragma unroll
-                for (int k = 0; k < G::PTS; ++k) {
+                for (int k = 0; k < PTS; ++k) {
                     const float* p = (b < 3) ? reinterpret_cast<const float*>(ldsb + base[k][a]) + b * G::PITCH
                                              : reinterpret_cast<const float*>(ldsb + base3[k][a]);
                     const float r = w3[k][0] * p[0] + w3[k][1] * p[1] + w3[k][2] * p[2] + w3[k][3] * p[3];
@@ -300,12 +303,12 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
                 }
             }
 #pragma unroll
-            for (int k = 0; k < G::PTS; ++k) v[k] += w1[k][a] * sa[k];
+            for (int k = 0; k < PTS; ++k) v[k] += w1[k][a] * sa[k];
         }
         {
             const uint32_t pb = static_cast<uint32_t>(x1) * plane4;
 #pragma unroll
-            for (int k = 0; k < G::PTS; ++k) {
+            for (int k = 0; k < PTS; ++k) {
                 if (!valid[k]) continue;
                 if constexpr (Epi::kCoord)
                     bstore(ro, epi.apply_at(v[k], caux[k], x1, x2, x3s[k]), off[k], pb);
@@ -333,7 +336,7 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
     if (x1 < x1e) step(x1, qa, aa, qb, ab, pa, pb2);
 }
 
-// Pair layout for D <= 2.  Entry c of an LDS row holds the two consecutive
+// Pair layout, D = 2 around a centre.  Entry c of an LDS row holds the two consecutive
 // values (f[c], f[c+1]) of the tile row, so the four values of a stencil row
 // starting at column c are the 8-byte entries c and c + 2: one ds_read2_b64
 // per stencil row instead of two ds_read2_b32, with no alignment condition
@@ -370,10 +373,26 @@ struct PairGeo {
     static_assert(2 * W * P * 4 <= 160 * 1024, "ring too large for two blocks per CU");
 };
 
-template <class Epi>
+// Which points a launch takes:
+//   kPtsNear  plan words with a bound D <= 2: every stencil lies in the window;
+//   kPtsPlan  plan words of any displacement;
+//   kPtsRaw   raw query points (3 floats per point over 2π, any value), turned
+//             into plan words as they are used.
+// For the last two the window of a block is centred on the mean offset of a
+// sample of its points (a smooth deformation is nearly rigid over a tile), and a
+// point whose stencil is not inside reads it from global memory, in the
+// arithmetic of the direct kernels.  A block whose sample lies mostly outside
+// (scattered points) stages nothing and takes the direct way throughout.
+enum PointMode { kPtsNear = 0, kPtsPlan = 1, kPtsRaw = 2 };
+// most planes per block of the last two (one bit of a mask each; raw points keep
+// to 32 bits and to input planes one step ahead, or the kernel runs out of
+// registers)
+constexpr int far_chunk(int mode) { return mode == kPtsRaw ? 32 : 64; }
+
+template <class Epi, int MODE>
 __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(PairGeo::WAVES_PER_EU))) void
-k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __restrict__ fbase, int64_t fzstride,
-                  Epi epi, int nblocks, int chunk) {
+k_gather_lds_pair(GatherDims g, HH hh, const PlanPt* __restrict__ plan, const float* __restrict__ fbase,
+                  int64_t fzstride, Epi epi, int nblocks, int chunk) {
     using G = PairGeo;
     __shared__ __align__(16) float lds[G::W * G::P];
     const int tid = threadIdx.x;
@@ -401,8 +420,128 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
     const uint32_t plane4 = static_cast<uint32_t>(g.n2) * static_cast<uint32_t>(g.n3) * 4u;
     const int x1s = ch * chunk;
     const int x1e = min(x1s + chunk, g.n1);
-    const int r2 = t2 * kLT2 - G::HLO;
-    const int r3 = t3 * G::LT3 - G::HLO;
+    // Wave w covers tile rows 2w and 2w + 1, 32 columns each.
+    struct Column {
+        int lx2, lx3, x2, x3;
+        bool valid;
+        uint32_t off;  // bytes of a float within a plane (0 where not valid)
+    };
+    auto column = [&](int t) {
+        Column c;
+        c.lx2 = 2 * (t >> 6) + ((t & 63) >> 5);
+        c.lx3 = t & 31;
+        c.x2 = t2 * kLT2 + c.lx2;
+        c.x3 = t3 * G::LT3 + c.lx3;
+        c.valid = c.x2 < g.n2 && c.x3 < g.n3;
+        c.off = c.valid ? 4u * static_cast<uint32_t>(c.x2 * g.n3 + c.x3) : 0u;
+        return c;
+    };
+    const int lane = tid & 63;
+    const Column me = column(tid);
+
+    // Plan words of a loaded point of plane x1; false when a raw point has none
+    // (a coordinate that is not finite).
+    auto decode = [&](const PlanPt& p, int x1, const Column& c, uint32_t (&w)[3]) {
+        if constexpr (MODE != kPtsRaw) {
+            w[0] = p.w[0];
+            w[1] = p.w[1];
+            w[2] = p.w[2];
+            return true;
+        } else {
+            int o;
+            w[0] = w[1] = w[2] = 0u;
+            const bool a = plan_encode(index_coord(__uint_as_float(p.w[0]), g.n1, hh.h[0]), x1, g.n1, w[0], o);
+            const bool b = plan_encode(index_coord(__uint_as_float(p.w[1]), g.n2, hh.h[1]), c.x2, g.n2, w[1], o);
+            const bool e = plan_encode(index_coord(__uint_as_float(p.w[2]), g.n3, hh.h[2]), c.x3, g.n3, w[2], o);
+            return a && b && e;
+        }
+    };
+    auto store_point = [&](int x1, const Column& c, float v, float a) {
+        const uint32_t pb = static_cast<uint32_t>(x1) * plane4;
+        if constexpr (Epi::kCoord)
+            bstore(ro, epi.apply_at(v, a, x1, c.x2, c.x3), c.off, pb);
+        else
+            bstore(ro, epi.apply(v, a), c.off, pb);
+        if constexpr (Epi::kOut2) bstore(ro2, epi.apply2(v, a), c.off, pb);
+    };
+    // a point of plane x1 read straight from global memory, and stored
+    auto direct_point = [&](int x1, const Column& c) {
+        const uint32_t pb = static_cast<uint32_t>(x1) * plane4;
+        const PlanPt p = bload_plan(rp, 3u * c.off, 3u * pb);
+        const float a = Epi::kHasAux ? bload_once(ra, c.off, pb) : 0.0f;
+        Stencil st;
+        if constexpr (MODE == kPtsRaw) {
+            const float q[3] = {__uint_as_float(p.w[0]), __uint_as_float(p.w[1]), __uint_as_float(p.w[2])};
+            setup_stencil(q, g, hh.h, st);
+        } else {
+            plan_stencil(p.w, x1, c.x2, c.x3, g, st);
+        }
+        const float* fs[1] = {f};
+        float r[1];
+        eval_stencil<1>(fs, st, g, r);
+        store_point(x1, c, r[0], a);
+    };
+    // Window: stencil offsets o with o − c in [−D − 1, D − 1] on every axis.
+    int c1 = 0, c2 = 0, c3 = 0;
+    auto in_window = [&](const uint32_t (&w)[3]) {
+        return static_cast<uint32_t>(plan_off(w[0]) - c1 + G::D + 1) <= 2u * G::D &&
+               static_cast<uint32_t>(plan_off(w[1]) - c2 + G::D + 1) <= 2u * G::D &&
+               static_cast<uint32_t>(plan_off(w[2]) - c3 + G::D + 1) <= 2u * G::D;
+    };
+    if constexpr (MODE != kPtsNear) {
+        // sample: this thread's column at a quarter and three quarters of the chunk
+        uint32_t w[2][3];
+        bool ok[2];
+        PlanPt p[2];
+        const int xs[2] = {x1s + (x1e - x1s) / 4, x1s + 3 * (x1e - x1s) / 4};
+#pragma unroll
+        for (int k = 0; k < 2; ++k) p[k] = bload_plan(rp, 3u * me.off, 3u * (static_cast<uint32_t>(xs[k]) * plane4));
+        int m[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            ok[k] = decode(p[k], xs[k], me, w[k]) && me.valid;
+            if (ok[k]) {
+                m[0] += plan_off(w[k][0]);
+                m[1] += plan_off(w[k][1]);
+                m[2] += plan_off(w[k][2]);
+                m[3] += 1;
+            }
+        }
+        int* sh = reinterpret_cast<int*>(lds);
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) m[a] += __shfl_xor(m[a], o, 64);
+            if (lane == 0) sh[4 * (tid >> 6) + a] = m[a];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            m[a] = 0;
+#pragma unroll
+            for (int k = 0; k < kLThreads / 64; ++k) m[a] += sh[4 * k + a];
+        }
+        const float inv = 1.0f / static_cast<float>(max(m[3], 1));
+        // offsets of −1 (a point on its own node's cell) sit at the window's middle
+        c1 = __builtin_amdgcn_readfirstlane(__float2int_rn(static_cast<float>(m[0]) * inv)) + 1;
+        c2 = __builtin_amdgcn_readfirstlane(__float2int_rn(static_cast<float>(m[1]) * inv)) + 1;
+        c3 = __builtin_amdgcn_readfirstlane(__float2int_rn(static_cast<float>(m[2]) * inv)) + 1;
+        const int mine = __popcll(__ballot(ok[0] && in_window(w[0]))) + __popcll(__ballot(ok[1] && in_window(w[1])));
+        if (lane == 0) sh[64 + (tid >> 6)] = mine;
+        __syncthreads();
+        int inside = 0;
+#pragma unroll
+        for (int k = 0; k < kLThreads / 64; ++k) inside += sh[64 + k];
+        __syncthreads();  // the staging below reuses sh
+        if (2 * __builtin_amdgcn_readfirstlane(inside) < __builtin_amdgcn_readfirstlane(m[3])) {
+            if (me.valid)
+                for (int x = x1s; x < x1e; ++x) direct_point(x, me);
+            return;
+        }
+    }
+    const int r2 = t2 * kLT2 - G::HLO + c2;
+    const int r3 = t3 * G::LT3 - G::HLO + c3;
+    const int xw0 = x1s - G::HLO + c1;  // the first input plane
 
     // Entries this thread fills: the byte offsets (within a global plane) of
     // the entry's two values and the entry's dword offset in an LDS plane.
@@ -420,15 +559,9 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
         loff[k] = e2 * G::PITCH + 2 * e3;
     }
 
-    const int lane = tid & 63;
-    const int lx2 = 2 * (tid >> 6) + (lane >> 5);
-    const int x2 = t2 * kLT2 + lx2;
-    const int lx3 = lane & 31;
-    const int x3 = t3 * G::LT3 + lx3;
-    const bool valid = x2 < g.n2 && x3 < g.n3;
-    const uint32_t off = valid ? 4u * static_cast<uint32_t>(x2 * g.n3 + x3) : 0u;
-    // byte offset of the point's own cell (its entry) in an LDS plane
-    const int rc = 4 * ((lx2 + G::HLO) * G::PITCH + 2 * (lx3 + G::HLO));
+    // byte offset of the point's own cell (its entry) in an LDS plane, less the
+    // window's centre
+    const int rc = 4 * ((me.lx2 + G::HLO - c2) * G::PITCH + 2 * (me.lx3 + G::HLO - c3));
 
     auto store2 = [&](float* dst, int q, float a, float b) {
         *reinterpret_cast<float2*>(dst + loff[q]) = make_float2(a, b);
@@ -442,7 +575,7 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
     // from 104.5 to 103.7 µs for 8 more VGPRs (123); plan words three steps
     // ahead instead of two are slower (105 µs).
     constexpr int LA_PT = 2;  // steps between a plan word load and its use
-    constexpr int LA_PL = 2;  // steps between an input plane load and its landing
+    constexpr int LA_PL = MODE == kPtsRaw ? 1 : 2;  // steps between an input plane load and its landing
     constexpr int NPRE = (LA_PL == 1) ? 2 : 4;
     PlanPt Q[4];
     float A[4];
@@ -450,8 +583,8 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
     auto load_point = [&](int x, PlanPt& q, float& a) {
         const int xc = min(x, x1e - 1);  // past the chunk end: a plane of this chunk, never used
         const uint32_t pb = static_cast<uint32_t>(xc) * plane4;
-        q = bload_plan(rp, 3u * off, 3u * pb);
-        a = Epi::kHasAux ? bload_once(ra, off, pb) : 0.0f;
+        q = bload_plan(rp, 3u * me.off, 3u * pb);
+        a = Epi::kHasAux ? bload_once(ra, me.off, pb) : 0.0f;
     };
     auto load_plane = [&](int xw, float (&pre)[G::FILL][2]) {  // xw: plane index in [0, n1)
         const uint32_t src = static_cast<uint32_t>(xw) * plane4;
@@ -471,7 +604,7 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
     {
         constexpr int NPRO = G::WIN + G::PERIOD - 1;
         float pro[NPRO][G::FILL][2];
-        int xw = pmod(x1s - G::HLO, g.n1);
+        int xw = pmod(xw0, g.n1);
 #pragma unroll
         for (int k = 0; k < NPRO; ++k) {
             load_plane(xw, pro[k]);
@@ -484,10 +617,10 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
                 if (tid + kLThreads * q < G::NV) store2(lds + k * G::P, q, pro[k][q][0], pro[k][q][1]);
     }
     for (int k = 0; k < LA_PT; ++k) load_point(x1s + k, Q[k], A[k]);
-    for (int k = 0; k < LA_PL; ++k) load_plane(pmod(x1s + G::HHI + G::PERIOD + k, g.n1), PRE[k]);
+    for (int k = 0; k < LA_PL; ++k) load_plane(pmod(xw0 + G::HLO + G::HHI + G::PERIOD + k, g.n1), PRE[k]);
     // periodic index of the input plane the next step loads, advanced by one
     // per step (a scalar modulo per step costs about 20 scalar instructions)
-    int xf = pmod(x1s + G::HHI + G::PERIOD + LA_PL, g.n1);
+    int xf = pmod(xw0 + G::HLO + G::HHI + G::PERIOD + LA_PL, g.n1);
     __syncthreads();
 
     constexpr int P4 = 4 * G::P;
@@ -506,9 +639,12 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
     // those of the LDS reads, so results are unchanged bit for bit.
     float2 S[4][4][2];
     int prev_key = std::numeric_limits<int>::min();
+    // planes of the chunk whose point of this thread is outside the window
+    using Mask = typename std::conditional<(far_chunk(MODE) > 32), uint64_t, uint32_t>::type;
+    Mask outside = 0;
     auto step = [&](auto kconst, int x1) {
         constexpr int K = decltype(kconst)::value;
-        const PlanPt& cur = Q[K & 3];
+        const PlanPt cur = Q[K & 3];
         const float caux = A[K & 3];
         load_point(x1 + LA_PT, Q[(K + LA_PT) & 3], A[(K + LA_PT) & 3]);
         load_plane(xf, PRE[(K + LA_PL) % NPRE]);  // plane x1 + HHI + PERIOD + LA_PL
@@ -527,14 +663,18 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
 #pragma unroll
         for (int q = 0; q < G::FILL; ++q)
             if (tid + kLThreads * q < G::NV) store2(dst, q, PRE[K % NPRE][q][0], PRE[K % NPRE][q][1]);
+        uint32_t word[3];
+        bool inside = decode(cur, x1, me, word);
+        if constexpr (MODE != kPtsNear) inside = inside && in_window(word);
         float w1[4], w2[4], w3[4];
-        lagrange_weights(plan_t(cur.w[0]), w1);
-        lagrange_weights(plan_t(cur.w[1]), w2);
-        lagrange_weights(plan_t(cur.w[2]), w3);
+        lagrange_weights(plan_t(word[0]), w1);
+        lagrange_weights(plan_t(word[1]), w2);
+        lagrange_weights(plan_t(word[2]), w3);
         // Byte address of the stencil's first row, counted from the ring slot
         // of plane x1 - HLO as if the ring did not end: o1·P4 plus the cell's
         // address within a plane (below P4, so equal keys are equal offsets).
-        const int key = plan_off(cur.w[0]) * P4 + (rc + plan_off(cur.w[1]) * (4 * G::PITCH) + 8 * plan_off(cur.w[2]));
+        const int key = (plan_off(word[0]) - c1) * P4 +
+                        (rc + plan_off(word[1]) * (4 * G::PITCH) + 8 * plan_off(word[2]));
         const bool reuse = key == prev_key;  // never on a chunk's first plane
         prev_key = key;
         // Stencil plane a starts at x = key + (slot + a)·P4, less the ring's
@@ -582,19 +722,19 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
             for (int b = 0; b < 4; ++b) {
                 const float2 lo = S[(K + a) & 3][b][0];
                 const float2 hi = S[(K + a) & 3][b][1];
-                const float r01 = Epi::kRowFrom1 ? fmaf(w3[0], lo.x, w3[1] * lo.y) : fmaf(w3[1], lo.y, w3[0] * lo.x);
-                const float r = fmaf(w3[3], hi.y, fmaf(w3[2], hi.x, r01));
-                sa += w2[b] * r;
+                if constexpr (MODE != kPtsNear || Epi::kRowFrom1)
+                    sa += w2[b] * row_sum(w3, lo.x, lo.y, hi.x, hi.y);
+                else
+                    sa += w2[b] * fmaf(w3[3], hi.y, fmaf(w3[2], hi.x, fmaf(w3[1], lo.y, w3[0] * lo.x)));
             }
             v += w1[a] * sa;
         }
-        if (valid) {
-            const uint32_t pb = static_cast<uint32_t>(x1) * plane4;
-            if constexpr (Epi::kCoord)
-                bstore(ro, epi.apply_at(v, caux, x1, x2, x3), off, pb);
-            else
-                bstore(ro, epi.apply(v, caux), off, pb);
-            if constexpr (Epi::kOut2) bstore(ro2, epi.apply2(v, caux), off, pb);
+        if constexpr (MODE == kPtsNear) {
+            if (me.valid) store_point(x1, me, v, caux);
+        } else {
+            if (me.valid && inside) store_point(x1, me, v, caux);
+            if (__ballot(me.valid && !inside))
+                outside |= static_cast<Mask>(me.valid && !inside) << (x1 - x1s);
         }
         cs4 = (cs4 == (G::W - 1 + G::HLO) * P4) ? G::HLO * P4 : cs4 + P4;
         if constexpr (K % G::PERIOD == G::PERIOD - 1) __syncthreads();
@@ -616,6 +756,31 @@ k_gather_lds_pair(GatherDims g, const PlanPt* __restrict__ plan, const float* __
     if (x1 < x1e) step(K0{}, x1);
     if (x1 + 1 < x1e) step(K1{}, x1 + 1);
     if (x1 + 2 < x1e) step(K2{}, x1 + 2);
+    // The points outside the window, of all threads, listed in the ring's memory
+    // and shared out evenly: they lie together, so a few waves would have most
+    // of them, one memory round trip each.  (Within the steps, the global
+    // stencil beside the rows kept for the next plane spills registers.)
+    if constexpr (MODE != kPtsNear) {
+        constexpr int kList = 8192;
+        static_assert((kList + 1) * 4 <= G::W * G::P * 4, "list exceeds the ring");
+        static_assert(far_chunk(MODE) <= 8 * static_cast<int>(sizeof(Mask)), "one bit per plane");
+        int* count = reinterpret_cast<int*>(lds);
+        int* list = count + 1;
+        __syncthreads();  // the ring is no longer read
+        if (tid == 0) *count = 0;
+        __syncthreads();
+        for (; outside; outside &= outside - 1) {
+            const int k = __builtin_ctzll(outside);
+            const int at = atomicAdd(count, 1);
+            if (at < kList)
+                list[at] = k * kLThreads + tid;
+            else
+                direct_point(x1s + k, me);
+        }
+        __syncthreads();
+        const int n = min(*count, kList);
+        for (int e = tid; e < n; e += kLThreads) direct_point(x1s + list[e] / kLThreads, column(list[e] % kLThreads));
+    }
 }
 
 // Incremental state right-hand sides, streamed with 16-byte accesses:
@@ -861,14 +1026,14 @@ bool pair_layout() {
 constexpr int kMaxChunk = 128;
 constexpr int kCandidates = 6;
 
-std::vector<int> chunk_candidates(int n1, int64_t tiles, int per_cu) {
+std::vector<int> chunk_candidates(int n1, int64_t tiles, int per_cu, int most) {
     static const double share[4][4] = {
         {0, 0, 0, 0}, {0, 1.0, 0, 0}, {0, 0.68, 1.0, 0}, {0, 0.43, 0.72, 1.0}};
     constexpr double kPrologue = 3.0;
     std::vector<std::pair<double, int>> cost;
     for (int nch = 1; nch <= n1; ++nch) {
         const int chunk = (n1 + nch - 1) / nch;
-        if (chunk > kMaxChunk || (!cost.empty() && cost.back().second == chunk)) continue;
+        if (chunk > most || (!cost.empty() && cost.back().second == chunk)) continue;
         const int64_t blocks = tiles * ((n1 + chunk - 1) / chunk);
         const int64_t k = (blocks + num_cus() - 1) / num_cus();
         const double rounds = static_cast<double>(k / per_cu) + share[per_cu][k % per_cu];
@@ -912,14 +1077,14 @@ bool tuning_enabled() {
 // Launches through `launch(chunk)` with the tuned chunk length of `key`,
 // tuning it on the first launch of that shape (see ShapeKey).
 template <class Launch>
-void tuned_launch(const ShapeKey& key, int64_t tiles, int per_cu, hipStream_t st, Launch&& launch) {
-    if (chunk_override() >= 1) return launch(std::min(chunk_override(), key.n1));
+void tuned_launch(const ShapeKey& key, int64_t tiles, int per_cu, int most, hipStream_t st, Launch&& launch) {
+    if (chunk_override() >= 1) return launch(std::min({chunk_override(), key.n1, most}));
     {
         std::lock_guard<std::mutex> lock(g_tune_mu);
         const auto it = g_tuned.find(key);
         if (it != g_tuned.end()) return launch(it->second);
     }
-    const std::vector<int> cand = chunk_candidates(key.n1, tiles, per_cu);
+    const std::vector<int> cand = chunk_candidates(key.n1, tiles, per_cu, most);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (!tuning_enabled() || hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone)
         return launch(cand[0]);
@@ -950,32 +1115,54 @@ void tuned_launch(const ShapeKey& key, int64_t tiles, int per_cu, hipStream_t st
     g_tuned[key] = best;
 }
 
-template <int D, bool PAIR, class Epi>
-void launch_lds(const GatherDims& g, const uint32_t* P, const float* f, int64_t fzstride, int nz, const Epi& epi,
+// One-value layout for bound −MODE (MODE < 0) or pair layout with the points of
+// MODE.
+template <int MODE, class Epi>
+void launch_lds(const GatherDims& g, const void* pts, const float* f, int64_t fzstride, int nz, const Epi& epi,
                 hipStream_t st) {
-    static_assert(!PAIR || D == 2, "the pair layout is for D <= 2");
+    constexpr bool kPair = MODE >= 0;
+    constexpr int D = kPair ? PairGeo::D : -MODE;
     const int nt3 = (g.n3 + LdsGeo<D>::LT3 - 1) / LdsGeo<D>::LT3;
     const int nt2 = (g.n2 + kLT2 - 1) / kLT2;
+    const PlanPt* P = static_cast<const PlanPt*>(pts);
     auto launch = [&](int chunk) {
         const int nch = (g.n1 + chunk - 1) / chunk;
         const int nb = nt3 * nt2 * nch;
-        if constexpr (PAIR)
-            hipLaunchKernelGGL((k_gather_lds_pair<Epi>), dim3(nb * nz), dim3(kLThreads), 0, st, g,
-                               reinterpret_cast<const PlanPt*>(P), f, fzstride, epi, nb, chunk);
+        if constexpr (kPair)
+            hipLaunchKernelGGL((k_gather_lds_pair<Epi, MODE>), dim3(nb * nz), dim3(kLThreads), 0, st, g, make_hh(g), P,
+                               f, fzstride, epi, nb, chunk);
         else
-            hipLaunchKernelGGL((k_gather_lds<D, Epi>), dim3(nb * nz), dim3(kLThreads), 0, st, g,
-                               reinterpret_cast<const PlanPt*>(P), f, fzstride, epi, nb, chunk);
+            hipLaunchKernelGGL((k_gather_lds<D, Epi>), dim3(nb * nz), dim3(kLThreads), 0, st, g, P, f, fzstride, epi,
+                               nb, chunk);
     };
-    const ShapeKey key{PAIR ? 100 + D : D, g.n1, g.n2, g.n3, nz};
-    tuned_launch(key, static_cast<int64_t>(nt3) * nt2 * nz, PAIR ? 2 : (D <= 2 ? 3 : 1), st, launch);
+    const ShapeKey key{MODE, g.n1, g.n2, g.n3, nz};
+    tuned_launch(key, static_cast<int64_t>(nt3) * nt2 * nz, kPair ? 2 : (D <= 2 ? 3 : 1),
+                 MODE > kPtsNear ? far_chunk(MODE) : kMaxChunk, st, launch);
 }
+
+void check_lds_dims(const GatherDims& g) {
+    CLR_REQUIRE(g.n1 >= 4 && g.n2 >= 4 && g.n3 >= 4, kErrInvalidArgument, "gather needs n >= 4 per axis");
+    CLR_REQUIRE(g.nl < (int64_t(1) << 28), kErrInvalidArgument, "grid too large for 32-bit buffer byte offsets");
+}
+
+// Points of a launch from which bounds above 2 take centred windows (kPtsPlan).
+// Finding the centres costs a block about 2 µs, which small launches, one block
+// per CU, do not hide.  Centred windows against the D <= 4 kernel at CFL 4.5 and
+// the direct kernels at CFL 9, one field: 64³ 8.5 : 6.8 µs (CFL 4.5); 96³
+// 14.2 : 15.8 and 18.4 : 22.0; 128³ 21.0 : 22.9 and 25.8 : 45.3; 256³ 93 : 140
+// and 145 : 360.  Three fields: 64³ 13.7 : 13.7 and 18.6 : 25.1; 96³ 27.2 : 36.8
+// and 34.7 : 58.2; 256³ 271 : 392.
+constexpr int64_t kFarPoints = int64_t(1) << 19;
 
 template <class Epi>
 void dispatch(int dbound, const GatherDims& g, const uint32_t* P, const float* f, int64_t fzstride, int nz,
               const Epi& epi, hipStream_t st) {
-    CLR_REQUIRE(g.n1 >= 4 && g.n2 >= 4 && g.n3 >= 4, kErrInvalidArgument, "gather needs n >= 4 per axis");
-    CLR_REQUIRE(g.nl < (int64_t(1) << 28), kErrInvalidArgument, "grid too large for 32-bit buffer byte offsets");
-    CLR_REQUIRE(dbound >= 0 && dbound <= 4, kErrInvalidArgument, "displacement bound too large for the LDS gather");
+    check_lds_dims(g);
+    CLR_REQUIRE(plan_gather_lds(g, dbound, nz), kErrInvalidArgument, "displacement bound too large for the LDS gather");
+    if (dbound > 2) {
+        if (g.nl * nz >= kFarPoints) return launch_lds<kPtsPlan>(g, P, f, fzstride, nz, epi, st);
+        return launch_lds<-4>(g, P, f, fzstride, nz, epi, st);
+    }
     // The pair layout (two blocks per CU) is faster than the one-value layout
     // (three) for one field per launch (the solves' steps: 110 µs against 115
     // at 256³, before later changes to both kernels), for plain three-field
@@ -985,23 +1172,34 @@ void dispatch(int dbound, const GatherDims& g, const uint32_t* P, const float* f
     // third resident block counts for more: 58.6 against 56.9 µs at 64³.
     constexpr bool kPlain = std::is_same<Epi, EpiPlain>::value;
     constexpr int64_t kPairStagePoints = int64_t(1) << 19;
-    if (dbound <= 2 && (nz == 1 || kPlain || g.nl >= kPairStagePoints) && pair_layout())
-        launch_lds<2, true>(g, P, f, fzstride, nz, epi, st);
-    else if (dbound <= 2)
-        launch_lds<2, false>(g, P, f, fzstride, nz, epi, st);
+    if ((nz == 1 || kPlain || g.nl >= kPairStagePoints) && pair_layout())
+        launch_lds<kPtsNear>(g, P, f, fzstride, nz, epi, st);
     else
-        launch_lds<4, false>(g, P, f, fzstride, nz, epi, st);
+        launch_lds<-2>(g, P, f, fzstride, nz, epi, st);
 }
 
-bool use_lds(const TrajectoryPlan& tp) { return tp.dbound >= 0 && tp.dbound <= lds_gather_max_displacement(); }
+bool use_lds(const TrajectoryPlan& tp, const GatherDims& g, int nz) { return plan_gather_lds(g, tp.dbound, nz); }
 
 }  // namespace
 
-int lds_gather_max_displacement() { return 4; }
+bool plan_gather_lds(const GatherDims& g, int dbound, int nz) {
+    if (dbound < 0 || dbound > kPlanMaxN) return false;  // no plan: a point is not finite
+    return dbound <= kNearBound || g.nl * nz >= kFarPoints;
+}
+
+void launch_points_gather(const GatherDims& g, const float* f, const float* X, float* out, hipStream_t st) {
+    // Raw points cost the centred windows their encoding too: image warps by
+    // smooth maps of CFL 2 to 9 at 128³ take 25-38 µs against 44-47 directly, at
+    // 192×150×256 and CFL 6 69 : 125, at 256³ and CFL 3 121 : 357; at 96³ 17.5 :
+    // 19.3 (CFL 2) and 22.5 : 20.9 (CFL 6), at 64³ 10.2 : 7.8.
+    if (g.nl < (int64_t(1) << 20)) return launch_gather1(g, f, X, out, st);
+    check_lds_dims(g);
+    launch_lds<kPtsRaw>(g, X, f, 0, 1, EpiPlain{out, 0}, st);
+}
 
 void launch_plan_gather(const TrajectoryPlan& tp, const GatherDims& g, const float* const f[], int nf,
                         float* const out[], hipStream_t st) {
-    if (!use_lds(tp)) return launch_direct_gather(g, tp.X, f, nf, out, st);
+    if (!use_lds(tp, g, nf)) return launch_direct_gather(g, tp.X, f, nf, out, st);
     const int64_t fz = nf > 1 ? (f[1] - f[0]) : 0;
     const int64_t oz = nf > 1 ? (out[1] - out[0]) : 0;
     for (int d = 2; d < nf; ++d)
@@ -1012,21 +1210,21 @@ void launch_plan_gather(const TrajectoryPlan& tp, const GatherDims& g, const flo
 
 void launch_plan_inc_state_step(const TrajectoryPlan& tp, const GatherDims& g, const float* mt, const float* sj,
                                 float* out, int negate, hipStream_t st) {
-    if (!use_lds(tp)) return launch_direct_inc_state_step(g, tp.X, mt, sj, out, negate, st);
+    if (!use_lds(tp, g, 1)) return launch_direct_inc_state_step(g, tp.X, mt, sj, out, negate, st);
     CLR_REQUIRE(mt != out, kErrInvalidArgument, "semi-Lagrangian step cannot run in place");
     dispatch(tp.dbound, g, tp.P, mt, 0, 1, EpiIncStep{sj, out, negate ? -1.0f : 1.0f}, st);
 }
 
 void launch_plan_adjoint_step(const TrajectoryPlan& tp, const GatherDims& g, const float* C, const float* lam,
                               float* out, hipStream_t st) {
-    if (!use_lds(tp)) return launch_direct_adjoint_step(g, tp.X, C, lam, out, st);
+    if (!use_lds(tp, g, 1)) return launch_direct_adjoint_step(g, tp.X, C, lam, out, st);
     CLR_REQUIRE(lam != out, kErrInvalidArgument, "semi-Lagrangian step cannot run in place");
     dispatch(tp.dbound, g, tp.P, lam, 0, 1, EpiAdjStep{C, out}, st);
 }
 
 void launch_plan_adjoint_coeff(const TrajectoryPlan& tp, const GatherDims& g, const float* divv, float ht, float alpha,
                                float* C, hipStream_t st) {
-    if (!use_lds(tp)) return launch_adjoint_coeff(g, tp.X, divv, ht, alpha, C, st);
+    if (!use_lds(tp, g, 1)) return launch_adjoint_coeff(g, tp.X, divv, ht, alpha, C, st);
     CLR_REQUIRE(divv != C, kErrInvalidArgument, "coefficient cannot overwrite ∇·v");
     dispatch(tp.dbound, g, tp.P, divv, 0, 1, EpiAdjCoeff{divv, C, ht, alpha}, st);
 }
@@ -1036,7 +1234,7 @@ void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, int dbound,
     const GatherDims g = gather_dims(d);
     const int64_t vz = v[1] - v[0];
     CLR_REQUIRE(v[2] - v[1] == vz && vz == g.nl, kErrInvalidArgument, "velocity components must be contiguous");
-    EpiTrajRk2 e{v[0], X, g.nl, d.hx[0], d.hx[1], d.hx[2], sigma * (0.5f * ht), 0};
+    EpiTrajRk2 e{v[0], X, g.nl, d.hx[0], d.hx[1], d.hx[2], sigma * (0.5f * ht), dbound > kNearBound, 0};
     dispatch(dbound, g, P, v[0], vz, 3, e, st);
 }
 
@@ -1054,15 +1252,15 @@ void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, int 
     const double s6 = static_cast<double>(sigma) * (static_cast<double>(ht) / 6.0);
     switch (stage) {
         case 1: {
-            EpiTrajRk4<1> e{v[0], X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * hthalf, s6, 0};
+            EpiTrajRk4<1> e{v[0], X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * hthalf, s6, dbound > kNearBound, 0};
             return dispatch(dbound, g, P, v[0], vz, 3, e, st);
         }
         case 2: {
-            EpiTrajRk4<2> e{Fin, X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * ht, s6, 0};
+            EpiTrajRk4<2> e{Fin, X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * ht, s6, false, 0};
             return dispatch(dbound, g, P, v[0], vz, 3, e, st);
         }
         case 3: {
-            EpiTrajRk4<3> e{Fin, X, X, g.nl, hx[0], hx[1], hx[2], 0.0f, s6, 0};  // no second output
+            EpiTrajRk4<3> e{Fin, X, X, g.nl, hx[0], hx[1], hx[2], 0.0f, s6, false, 0};  // no second output
             return dispatch(dbound, g, P, v[0], vz, 3, e, st);
         }
         default:

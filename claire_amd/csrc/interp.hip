@@ -9,8 +9,9 @@
 //     together with the exact per-axis displacement bound that decides
 //     whether the LDS-staged gathers can be used;
 //   * direct gathers (one thread per point, stencil rows read from global
-//     memory as unaligned 16-byte loads) for arbitrary query points and for
-//     trajectories whose displacement exceeds the LDS window.
+//     memory as unaligned 16-byte loads) for what the LDS-staged gathers do not
+//     take: small grids with query points anywhere or displacements beyond their
+//     windows, and trajectories with points that are not finite.
 #include <algorithm>
 
 #include "gather_device.hpp"

@@ -74,7 +74,8 @@ void grad_noalloc(const int nx[3], const float* f, float* g, hipStream_t st);
 // ---------------------------------------------------------------------------
 // Semi-Lagrangian gathers (interp.hip, gather_lds.hip).  X: foot points over
 // 2π, one component per field (component d of point i at X[d·nl + i]), except
-// for launch_gather1, whose query points are interleaved xyz.
+// for launch_gather1 and launch_points_gather, whose query points are
+// interleaved xyz.
 // ---------------------------------------------------------------------------
 struct GatherDims {
     int n1, n2, n3;
@@ -83,8 +84,10 @@ struct GatherDims {
 
 GatherDims gather_dims(const Dims& d);
 
-// out = f(X), X interleaved (3 floats per point), any displacement
+// out = f(X), X interleaved (3 floats per point), any query points: straight from
+// global memory, or (launch_points_gather) LDS-staged where the grid is large
 void launch_gather1(const GatherDims& g, const float* f, const float* X, float* out, hipStream_t st);
+void launch_points_gather(const GatherDims& g, const float* f, const float* X, float* out, hipStream_t st);
 // out = X, interleaved
 void launch_interleave(int64_t nl, const float* X, float* out, hipStream_t st);
 // RK2 characteristic, Euler predictor and velocity gather fused, any
@@ -111,8 +114,7 @@ int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* bmax
 //   1. the packed plan of the Euler predictor X̃ = (x − σ·ht·v)/2π into P
 //      (launch_set_velocity or launch_predictor_plan);
 //   2. v gathered along it with the corrector as epilogue,
-//      X = (x − σ·ht/2·(v(X̃) + v))/2π (launch_lds_traj_rk2_corrector, bound
-//      <= 4);
+//      X = (x − σ·ht/2·(v(X̃) + v))/2π (launch_lds_traj_rk2_corrector);
 //   3. the plan of X into P (launch_make_plan, which returns its bound).
 // The foot points equal those of launch_trajectory_rk2 up to FMA contraction.
 //
@@ -133,7 +135,7 @@ void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, int dbound,
                                    float ht, float* X, hipStream_t st);
 // RK4 characteristic the same way: the plan of the first stage point
 // (x − σ·ht/2·v)/2π is the predictor's with ht/2; each stage gathers v along the
-// previous point's plan (bound <= 4), accumulates the stage sum f and writes
+// previous point's plan, accumulates the stage sum f and writes
 // the next point into X (the foot point at stage 3), whose plan
 // launch_make_plan builds.  Stage 1
 // writes f into Fout (Fin unused), stage 2 reads Fin and writes Fout (two
@@ -141,8 +143,12 @@ void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, int dbound,
 // be repeated while its chunk length is tuned), stage 3 reads Fin.
 void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, int dbound, const float* const v[3],
                                float sigma, float ht, const float* Fin, float* Fout, float* X, hipStream_t st);
-// The LDS-staged gathers need D <= lds_gather_max_displacement().
-int lds_gather_max_displacement();
+// Whether the gathers of nz fields along a plan of this bound run LDS-staged: the
+// bound is at most kNearBound, or the points are finite and many enough for
+// windows centred per block.  Beyond kNearBound the staged kernels round as the
+// direct ones do, so that this choice moves nothing.
+constexpr int kNearBound = 4;
+bool plan_gather_lds(const GatherDims& g, int dbound, int nz);
 // Update coefficient per point: C = 1 + ht/2·(α·dX + α·(1 + ht·α·dX)·d)
 // with d = ∇·v, dX = d(X).  α = 1 on the adjoint trajectory gives the SL
 // adjoint update λ⁺ = C·λ(X_a); α = ±1 on the state trajectory gives the
