@@ -10,8 +10,8 @@
 // A 3D transform is three passes over HBM:
 //   x3 pass  rows of n3 reals, two rows packed as one complex row
 //            (z = a + i·b), one complex FFT, split by Hermitian symmetry;
-//   x2 pass  batched strided complex FFTs, 16 adjacent columns per block so
-//            that each row access is a 128-byte segment;
+//   x2 pass  batched strided complex FFTs, 16 or more adjacent columns per block
+//            so that each row access is a segment of 128 bytes or more;
 //   x1 pass  same, and this is where k-space operators are fused: the block
 //            holds complete x1 columns, so forward FFT, per-mode multiplier
 //            and inverse FFT happen in one read and one write.
@@ -156,19 +156,21 @@ struct Radices {};
 
 template <int N>
 struct Plan;
-// V = values per thread; Fwd radices; Inv = reverse order.
-template <> struct Plan<8>   { static constexpr int V = 8;  using Fwd = Radices<8>;         using Inv = Radices<8>; };
-template <> struct Plan<16>  { static constexpr int V = 16; using Fwd = Radices<16>;        using Inv = Radices<16>; };
-template <> struct Plan<32>  { static constexpr int V = 16; using Fwd = Radices<16, 2>;     using Inv = Radices<2, 16>; };
-template <> struct Plan<64>  { static constexpr int V = 16; using Fwd = Radices<16, 4>;     using Inv = Radices<4, 16>; };
-template <> struct Plan<128> { static constexpr int V = 16; using Fwd = Radices<16, 8>;     using Inv = Radices<8, 16>; };
-template <> struct Plan<256> { static constexpr int V = 16; using Fwd = Radices<16, 16>;    using Inv = Radices<16, 16>; };
-template <> struct Plan<512> { static constexpr int V = 16; using Fwd = Radices<16, 16, 2>; using Inv = Radices<2, 16, 16>; };
-// lengths with factors 3 and 5 (every radix divides V)
-template <> struct Plan<48>  { static constexpr int V = 12; using Fwd = Radices<4, 4, 3>;     using Inv = Radices<3, 4, 4>; };
-template <> struct Plan<96>  { static constexpr int V = 24; using Fwd = Radices<8, 4, 3>;     using Inv = Radices<3, 4, 8>; };
-template <> struct Plan<150> { static constexpr int V = 30; using Fwd = Radices<2, 3, 5, 5>;  using Inv = Radices<5, 5, 3, 2>; };
-template <> struct Plan<192> { static constexpr int V = 24; using Fwd = Radices<8, 8, 3>;     using Inv = Radices<3, 8, 8>; };
+// V = values per thread; Fwd radices; Inv = reverse order.  Row pairs or columns per
+// block (see Geo): Row and RowWide of small and large x3 passes, Col of the x2 pass,
+// X1 of the x1 passes.
+template <> struct Plan<8> { static constexpr int V =  8, Row = 64, RowWide = 256, Col = 64, X1 = 64; using Fwd = Radices<8>; using Inv = Radices<8>; };
+template <> struct Plan<16> { static constexpr int V = 16, Row = 64, RowWide = 256, Col = 64, X1 = 64; using Fwd = Radices<16>; using Inv = Radices<16>; };
+template <> struct Plan<32> { static constexpr int V = 16, Row = 32, RowWide = 128, Col = 32, X1 = 32; using Fwd = Radices<16, 2>; using Inv = Radices<2, 16>; };
+template <> struct Plan<64> { static constexpr int V = 16, Row = 16, RowWide =  64, Col = 32, X1 = 16; using Fwd = Radices<16, 4>; using Inv = Radices<4, 16>; };
+template <> struct Plan<128> { static constexpr int V = 16, Row =  8, RowWide =  32, Col = 32, X1 = 16; using Fwd = Radices<16, 8>; using Inv = Radices<8, 16>; };
+template <> struct Plan<256> { static constexpr int V = 16, Row = 16, RowWide =  16, Col = 32, X1 = 16; using Fwd = Radices<16, 16>; using Inv = Radices<16, 16>; };
+template <> struct Plan<512> { static constexpr int V = 16, Row =  8, RowWide =   8, Col = 16, X1 =  8; using Fwd = Radices<16, 16, 2>; using Inv = Radices<2, 16, 16>; };
+// lengths with factors 3 and 5
+template <> struct Plan<48> { static constexpr int V = 12, Row = 16, RowWide =  64, Col = 16, X1 = 16; using Fwd = Radices<4, 4, 3>; using Inv = Radices<3, 4, 4>; };
+template <> struct Plan<96> { static constexpr int V = 24, Row = 32, RowWide =  64, Col = 32, X1 = 16; using Fwd = Radices<8, 4, 3>; using Inv = Radices<3, 4, 8>; };
+template <> struct Plan<150> { static constexpr int V = 30, Row = 25, RowWide =  25, Col = 25, X1 = 25; using Fwd = Radices<2, 3, 5, 5>; using Inv = Radices<5, 5, 3, 2>; };
+template <> struct Plan<192> { static constexpr int V = 24, Row =  8, RowWide =  32, Col = 32, X1 = 16; using Fwd = Radices<8, 8, 3>; using Inv = Radices<3, 8, 8>; };
 
 template <class L> struct First;
 template <int R, int... RS> struct First<Radices<R, RS...>> { static constexpr int value = R; };
@@ -267,31 +269,42 @@ __device__ __forceinline__ void fft_regs(c32 (&v)[Plan<N>::V], c32* s, const Lay
 }
 
 // Block geometry: B columns (or row pairs) per block, T threads per column.
-template <int N>
+// Blocks of one or two waves reach more CUs on small grids, wait for fewer waves at
+// their barriers and leave LDS for more blocks; a column block takes at least 16
+// columns, 128-byte segments, and more where they gain by it.  Against 256 threads
+// per block everywhere (µs, outputs identical): gradient of 32³ 27.5 -> 19.5 in all;
+// x2 pass of 96³ 11.7 -> 9.3 with 32 columns for 64, of 64×64×150 8.5 -> 7.2; x1
+// gradient of 64³ 9.3 -> 7.4, of 150³ 31.6 -> 28.4, of 192³ 35.8 -> 32.6 with 16
+// columns for 32; three-field rows of 256×192×150 68 -> 61 and 72 -> 65 with 25 pairs
+// for 51.
+template <int N, int B_>
 struct Geo {
     static constexpr int V = Plan<N>::V;
     static constexpr int T = N / V;
-    static constexpr int B = (T >= 32) ? 8 : ((T >= 16) ? 16 : (256 / T));
+    static constexpr int B = B_;
     static constexpr int THREADS = B * T;
-    static constexpr int LD = B + 1;  // ColLayout pitch (odd: spreads banks)
-    static constexpr int ROW_ELEMS = B * RowLayout<N>::CP;
-    static constexpr int LDS_ELEMS = (N * LD > ROW_ELEMS) ? N * LD : ROW_ELEMS;
+    static constexpr int LD = B | 1;  // ColLayout pitch (odd: spreads banks)
+};
+template <int N, int B>
+struct RowGeo : Geo<N, B> {
+    static constexpr int LDS_ELEMS = B * RowLayout<N>::CP;
+};
+template <int N>
+struct ColGeo : Geo<N, Plan<N>::Col> {
+    static constexpr int LDS_ELEMS = N * Geo<N, Plan<N>::Col>::LD;
+};
+template <int N, int B = Plan<N>::X1>
+struct X1Geo : Geo<N, B> {
+    static constexpr int LDS_ELEMS = N * Geo<N, B>::LD;
 };
 
-// Geometry of the plain column passes (k_col, the x2 passes): Geo<N> with
-// twice the columns per block at N = 256 and 512 (256-byte row segments per
-// block instead of 128; measured: three-field x2 pass at 256³ 82.8 → 79.8
-// µs, the 512³ H2 matvec 29.10 → 28.95 ms, outputs identical).  The fused
-// x1 pass and the row passes keep Geo<N> (wider blocks made them slower).
-template <int N>
-struct ColGeo {
-    static constexpr int V = Plan<N>::V;
-    static constexpr int T = N / V;
-    static constexpr int B = (N == 256 || N == 512) ? 2 * Geo<N>::B : Geo<N>::B;
-    static constexpr int THREADS = B * T;
-    static constexpr int LD = B + 1;
-    static constexpr int LDS_ELEMS = N * LD;
-};
+// Blocks are dealt round-robin over the 8 XCDs; renumbered so that each XCD owns
+// one contiguous range of columns and the cache lines shared by neighbouring blocks
+// stay in one L2.
+__device__ __forceinline__ unsigned xcd_block() {
+    const unsigned nb = gridDim.x, x = blockIdx.x & 7u, r = nb & 7u;
+    return x * (nb >> 3) + (x < r ? x : r) + (blockIdx.x >> 3);
+}
 
 __device__ __forceinline__ int wavenum(int k, int n) { return k > n / 2 ? k - n : (k == n / 2 ? 0 : k); }
 
@@ -349,11 +362,11 @@ struct ColPtrs {  // in place
     int64_t ds;
 };
 
-template <int N>
-__global__ __launch_bounds__(Geo<N>::THREADS) void k_row_r2c(R2CPtrs ptr, int64_t nrows, const c32* __restrict__ tw) {
+template <int N, int B>
+__global__ __launch_bounds__((RowGeo<N, B>::THREADS)) void k_row_r2c(R2CPtrs ptr, int64_t nrows, const c32* __restrict__ tw) {
     const float* __restrict__ in = ptr.in + blockIdx.y * ptr.is;
     c32* __restrict__ out = ptr.out + blockIdx.y * ptr.os;
-    using G = Geo<N>;
+    using G = RowGeo<N, B>;
     __shared__ c32 s[G::LDS_ELEMS];
     constexpr int V = G::V, T = G::T, R0 = First<typename Plan<N>::Fwd>::value,
                   RL = Last<typename Plan<N>::Fwd>::value;
@@ -423,13 +436,14 @@ __device__ __forceinline__ void flat_copy(int n, Load&& load, Use&& use) {
 
 // ADD: some field has an added term (its values are loaded before the
 // transform, in registers the plain pass does not need).
-template <int N, bool ADD>
-__global__ __launch_bounds__(Geo<N>::THREADS) void k_row_c2r(C2RPtrs ptr, int64_t nrows, const c32* __restrict__ tw,
-                                                             float alpha, float beta) {
+template <int N, int B, bool ADD>
+__global__ __launch_bounds__((RowGeo<N, B>::THREADS)) void k_row_c2r(C2RPtrs ptr, int64_t nrows,
+                                                                     const c32* __restrict__ tw, float alpha,
+                                                                     float beta) {
     const c32* __restrict__ in = ptr.in + blockIdx.y * ptr.is;
     float* __restrict__ out = ptr.out + blockIdx.y * ptr.os;
     const float* __restrict__ add = ADD ? ptr.add + blockIdx.y * ptr.as : nullptr;
-    using G = Geo<N>;
+    using G = RowGeo<N, B>;
     __shared__ c32 s[G::LDS_ELEMS];
     constexpr int V = G::V, T = G::T, R0 = First<typename Plan<N>::Inv>::value,
                   RL = Last<typename Plan<N>::Inv>::value;
@@ -614,12 +628,10 @@ __global__ __launch_bounds__(ColGeo<N>::THREADS) void k_col(ColPtrs ptr, ColGeom
     constexpr int V = G::V, T = G::T, R0 = First<L>::value, RL = Last<L>::value;
     const int c = threadIdx.x % G::B;
     const int t = threadIdx.x / G::B;
-    // Blocks are dealt round-robin over the 8 XCDs; remap them so each XCD
-    // owns one contiguous range of columns and the cache lines shared by
-    // neighbouring column groups (rows are not 128-byte aligned) stay in one L2.
-    const unsigned nb = gridDim.x;
-    const unsigned b = (nb % 8 == 0) ? (blockIdx.x & 7u) * (nb >> 3) + (blockIdx.x >> 3) : blockIdx.x;
-    const int64_t cg = static_cast<int64_t>(b) * G::B + c;
+    // x2 rows are never 128-byte aligned (nh is odd), so neighbouring blocks share
+    // cache lines (renumbered only where 8 divided the number of blocks, the
+    // three-field pass of 192³ took 41 µs, now 29)
+    const int64_t cg = static_cast<int64_t>(xcd_block()) * G::B + c;
     const bool valid = cg < geo.ncols;
     const int64_t base = valid ? col_base<N>(geo, cg) : 0;
     c32 v[V];
@@ -685,16 +697,26 @@ struct X1Ptrs {
     int64_t oc;
 };
 
-template <int N, int MODE>
-__global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_fused(X1Ptrs ptr, ColGeom geo, const c32* __restrict__ tw,
-                                                              SpecParams sp, int n2, int n3, int nh) {
-    using G = Geo<N>;
+// The columns of an x1 pass lie side by side, so blocks of 16 share lines only where
+// the planes are not 128-byte aligned: there the blocks are renumbered (128×150×128,
+// multiplier of three fields 20.5 -> 18.2 µs), elsewhere neighbouring blocks are
+// better on different XCDs (512³ gradient, in two stages of 32 and 16: 717 against 768
+// µs).
+__device__ __forceinline__ unsigned x1_block(const ColGeom& g) {
+    return g.estride % 16 != 0 ? xcd_block() : blockIdx.x;
+}
+
+template <int N, int MODE, int B>
+__global__ __launch_bounds__((X1Geo<N, B>::THREADS)) void k_x1_fused(X1Ptrs ptr, ColGeom geo, const c32* __restrict__ tw,
+                                                                   SpecParams sp, int n2, int n3, int nh) {
+    using G = X1Geo<N, B>;
     __shared__ c32 s[G::LDS_ELEMS];
     using LF = typename Plan<N>::Fwd;
     constexpr int V = G::V, T = G::T, R0 = First<LF>::value, RL = Last<LF>::value;
     const int c = threadIdx.x % G::B;
     const int t = threadIdx.x / G::B;
-    const int64_t cg = static_cast<int64_t>(blockIdx.x) * G::B + c;
+    const unsigned blk = x1_block(geo);
+    const int64_t cg = static_cast<int64_t>(blk) * G::B + c;
     const bool valid = cg < geo.ncols;
     const int64_t base = valid ? cg : 0;
     const int k2 = static_cast<int>(static_cast<uint32_t>(cg) / static_cast<uint32_t>(nh));
@@ -844,16 +866,17 @@ __device__ __forceinline__ double norm_factor(const SpecParams& p, double k2) {
 }
 
 template <int N>
-__global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_norm(X1Ptrs ptr, ColGeom geo, const c32* __restrict__ tw,
+__global__ __launch_bounds__(X1Geo<N>::THREADS) void k_x1_norm(X1Ptrs ptr, ColGeom geo, const c32* __restrict__ tw,
                                                              SpecParams sp, int n2, int n3, int nh,
                                                              double* __restrict__ partial) {
-    using G = Geo<N>;
+    using G = X1Geo<N>;
     __shared__ c32 s[G::LDS_ELEMS];
     using LF = typename Plan<N>::Fwd;
     constexpr int V = G::V, T = G::T, R0 = First<LF>::value, RL = Last<LF>::value;
     const int c = threadIdx.x % G::B;
     const int t = threadIdx.x / G::B;
-    const int64_t cg = static_cast<int64_t>(blockIdx.x) * G::B + c;
+    const unsigned blk = x1_block(geo);
+    const int64_t cg = static_cast<int64_t>(blk) * G::B + c;
     const bool valid = cg < geo.ncols;
     const int64_t base = valid ? cg : 0;
     const int k2 = static_cast<int>(static_cast<uint32_t>(cg) / static_cast<uint32_t>(nh));
@@ -895,7 +918,7 @@ __global__ __launch_bounds__(Geo<N>::THREADS) void k_x1_norm(X1Ptrs ptr, ColGeom
     for (int i = threadIdx.x; i < G::THREADS; i += 64) sum += sh[i];
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
-    if (threadIdx.x == 0) partial[static_cast<int64_t>(blockIdx.y) * gridDim.x + blockIdx.x] = sum;
+    if (threadIdx.x == 0) partial[static_cast<int64_t>(blockIdx.y) * gridDim.x + blk] = sum;
 }
 
 // ---------------------------------------------------------------------------
@@ -919,28 +942,48 @@ void dispatch_n(int n, A&&... a) {
     }
 }
 
+// Row pairs of a launch from which the row passes take blocks of 256 threads.
+// Rows of the spectrum are not whole cache lines, so blocks share them at both ends,
+// which small blocks do more often: forward rows of 512×192×192 (147456 pairs in
+// three fields) take 115 µs with 32 pairs per block, 131 with 8, and of 512×128×128
+// (98304) 49 and 53.  Below, the launch is bound by latency and by CUs without a
+// block: 32³ 8.0 and 4.6 µs, 96³ 8.6 and 7.0 (one field), 192³ 44 and 39 (inverse).
+constexpr int64_t kWideRowPairs = int64_t(1) << 16;
+
 template <int N>
 struct RowR2C {
     static void go(const R2CPtrs& p, int ncomp, int64_t nrows, const c32* tw, hipStream_t st) {
-        using G = Geo<N>;
-        const int64_t npairs = (nrows + 1) / 2;
-        const int64_t blocks = (npairs + G::B - 1) / G::B;
-        hipLaunchKernelGGL(k_row_r2c<N>, dim3(static_cast<unsigned>(blocks), ncomp), dim3(G::THREADS), 0, st, p, nrows,
-                           tw);
+        if ((nrows + 1) / 2 * ncomp >= kWideRowPairs)
+            launch<Plan<N>::RowWide>(p, ncomp, nrows, tw, st);
+        else
+            launch<Plan<N>::Row>(p, ncomp, nrows, tw, st);
+    }
+
+    template <int B>
+    static void launch(const R2CPtrs& p, int ncomp, int64_t nrows, const c32* tw, hipStream_t st) {
+        const int64_t blocks = ((nrows + 1) / 2 + B - 1) / B;
+        hipLaunchKernelGGL((k_row_r2c<N, B>), dim3(static_cast<unsigned>(blocks), ncomp), dim3(RowGeo<N, B>::THREADS), 0, st,
+                           p, nrows, tw);
     }
 };
 
 template <int N>
 struct RowC2R {
     static void go(const C2RPtrs& p, int ncomp, int64_t nrows, const c32* tw, float alpha, float beta, hipStream_t st) {
-        using G = Geo<N>;
-        const int64_t npairs = (nrows + 1) / 2;
-        const int64_t blocks = (npairs + G::B - 1) / G::B;
-        const dim3 grid(static_cast<unsigned>(blocks), ncomp);
-        if (p.add)
-            hipLaunchKernelGGL((k_row_c2r<N, true>), grid, dim3(G::THREADS), 0, st, p, nrows, tw, alpha, beta);
+        if ((nrows + 1) / 2 * ncomp >= kWideRowPairs)
+            launch<Plan<N>::RowWide>(p, ncomp, nrows, tw, alpha, beta, st);
         else
-            hipLaunchKernelGGL((k_row_c2r<N, false>), grid, dim3(G::THREADS), 0, st, p, nrows, tw, alpha, beta);
+            launch<Plan<N>::Row>(p, ncomp, nrows, tw, alpha, beta, st);
+    }
+
+    template <int B>
+    static void launch(const C2RPtrs& p, int ncomp, int64_t nrows, const c32* tw, float alpha, float beta,
+                       hipStream_t st) {
+        const dim3 grid(static_cast<unsigned>(((nrows + 1) / 2 + B - 1) / B), ncomp), block(RowGeo<N, B>::THREADS);
+        if (p.add)
+            hipLaunchKernelGGL((k_row_c2r<N, B, true>), grid, block, 0, st, p, nrows, tw, alpha, beta);
+        else
+            hipLaunchKernelGGL((k_row_c2r<N, B, false>), grid, block, 0, st, p, nrows, tw, alpha, beta);
     }
 };
 
@@ -958,43 +1001,56 @@ struct ColPass {
     }
 };
 
+// columns of an x1 pass of 512 from which its blocks take 16 of them
+constexpr int64_t kWideX1Columns = int64_t(1) << 15;
+
 template <int N>
 struct X1Fused {
     static void go(int mode, X1Ptrs p, ColGeom geo, const c32* tw, SpecParams sp, int n2, int n3, int nh, int nfields,
                    hipStream_t st) {
-        using G = Geo<N>;
         CLR_REQUIRE(geo.ncols * N * 8 < (int64_t(1) << 31), kErrInvalidArgument,
                     "spectrum field too large for 32-bit buffer offsets");
-        const int64_t blocks = (geo.ncols + G::B - 1) / G::B;
-        dim3 grid(static_cast<unsigned>(blocks), mode == kFuseMult || mode == kFuseGrad ? nfields : 1);
         switch (mode) {
-            case kFuseMult:
-                hipLaunchKernelGGL((k_x1_fused<N, kFuseMult>), grid, dim3(G::THREADS), 0, st, p, geo, tw, sp, n2, n3, nh);
-                break;
-            case kFuseGrad:
-                hipLaunchKernelGGL((k_x1_fused<N, kFuseGrad>), grid, dim3(G::THREADS), 0, st, p, geo, tw, sp, n2, n3, nh);
-                break;
-            case kFuseProject:
-                hipLaunchKernelGGL((k_x1_fused<N, kFuseProject>), grid, dim3(G::THREADS), 0, st, p, geo, tw, sp, n2, n3,
-                                   nh);
-                break;
-            default:
-                hipLaunchKernelGGL((k_x1_fused<N, kFuseDiv>), grid, dim3(G::THREADS), 0, st, p, geo, tw, sp, n2, n3, nh);
-                break;
+            case kFuseMult: launch<kFuseMult>(p, geo, tw, sp, n2, n3, nh, nfields, st); break;
+            case kFuseGrad: launch<kFuseGrad>(p, geo, tw, sp, n2, n3, nh, nfields, st); break;
+            case kFuseProject: launch<kFuseProject>(p, geo, tw, sp, n2, n3, nh, 1, st); break;
+            default: launch<kFuseDiv>(p, geo, tw, sp, n2, n3, nh, 1, st); break;
         }
+    }
+
+    template <int MODE>
+    static void launch(const X1Ptrs& p, const ColGeom& geo, const c32* tw, const SpecParams& sp, int n2, int n3, int nh,
+                       int nfields, hipStream_t st) {
+        // At 512 points a column has 32 threads: 8 columns make a block of 256 threads
+        // with 64-byte segments, 16 one of 512 with 128-byte segments.  The wide block
+        // is better once the launch is bound by memory (multiplier of three fields /
+        // gradient, µs: 512³ 1150 -> 915 / 789 -> 654, 512×256×256 394 -> 328 / 194 ->
+        // 187), the narrow one below (512×192×192 128 : 132 / 92 : 101, 512×96×96
+        // projection 58 : 64).
+        if constexpr (N == 512) {
+            if (geo.ncols >= kWideX1Columns) return launch_b<MODE, 16>(p, geo, tw, sp, n2, n3, nh, nfields, st);
+        }
+        launch_b<MODE, Plan<N>::X1>(p, geo, tw, sp, n2, n3, nh, nfields, st);
+    }
+
+    template <int MODE, int B>
+    static void launch_b(const X1Ptrs& p, const ColGeom& geo, const c32* tw, const SpecParams& sp, int n2, int n3, int nh,
+                         int nfields, hipStream_t st) {
+        const dim3 grid(static_cast<unsigned>((geo.ncols + B - 1) / B), nfields);
+        hipLaunchKernelGGL((k_x1_fused<N, MODE, B>), grid, dim3(X1Geo<N, B>::THREADS), 0, st, p, geo, tw, sp, n2, n3, nh);
     }
 };
 
 template <int N>
 struct X1Blocks {
-    static void go(int64_t ncols, int64_t* blocks) { *blocks = (ncols + Geo<N>::B - 1) / Geo<N>::B; }
+    static void go(int64_t ncols, int64_t* blocks) { *blocks = (ncols + X1Geo<N>::B - 1) / X1Geo<N>::B; }
 };
 
 template <int N>
 struct X1Norm {
     static void go(X1Ptrs p, ColGeom geo, const c32* tw, SpecParams sp, int n2, int n3, int nh, int ncomp, double* partial,
                    hipStream_t st) {
-        using G = Geo<N>;
+        using G = X1Geo<N>;
         CLR_REQUIRE(geo.ncols * N * 8 < (int64_t(1) << 31), kErrInvalidArgument,
                     "spectrum field too large for 32-bit buffer offsets");
         const dim3 grid(static_cast<unsigned>((geo.ncols + G::B - 1) / G::B), ncomp);
