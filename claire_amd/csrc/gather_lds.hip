@@ -836,40 +836,41 @@ struct RhsP {
 
 // Src = SrcF32 (plain) or SrcBfp (mixed form: the Newton-invariant gradient
 // fields stored as 16-bit block floating point, accumulated in FP32).
-// Each wave of the streaming kernels covers kStreamK consecutive runs of 64
+// On large grids each wave of the streaming kernels covers K = 2 consecutive runs of 64
 // float4 (1 KB of FP32) of every stream, lane l taking float4 l of each run,
 // so each of the 30-odd streams is read in 2 KB bursts.  Measured at 256³
 // (outputs identical): k_inc_state_rhs 399 → 367 µs and k_body_force 256 →
 // 243 µs with two runs per wave; four runs (227 VGPRs for the right-hand
 // sides) were slower than two.  A microbenchmark of 30 read and 4 write
 // streams gave 5.6, 6.2 and 6.6 TB/s for one, two and four runs.
-constexpr int kStreamK = 2;
 __device__ __forceinline__ int64_t stream_base(int k) {
     return static_cast<int64_t>(blockIdx.x) * 256 * k + (threadIdx.x >> 6) * 64 * k + (threadIdx.x & 63);
 }
 
-template <class Src>
+template <class Src, int K>
 __global__ __launch_bounds__(256) void k_inc_state_rhs(int64_t nl4, int nt, float hthalf, RhsP<Src> p) {
-    const int64_t i0 = stream_base(kStreamK);
+    const int64_t i0 = stream_base(K);
     const int64_t nl = nl4 * 4;
-    float4 x0[kStreamK], x1[kStreamK], x2[kStreamK], v0[kStreamK], v1[kStreamK], v2[kStreamK];
+    float4 x0[K], x1[K], x2[K], v0[K], v1[K], v2[K];
 #pragma unroll
-    for (int k = 0; k < kStreamK; ++k) {
+    for (int k = 0; k < K; ++k) {
         const int64_t i = min(i0 + 64 * k, nl4 - 1);  // past the end: reload the last group, never stored
         x0[k] = ld4(p.vx[0], i); x1[k] = ld4(p.vx[1], i); x2[k] = ld4(p.vx[2], i);
         v0[k] = ld4(p.vt[0], i); v1[k] = ld4(p.vt[1], i); v2[k] = ld4(p.vt[2], i);
     }
-    for (int j = 0; j < nt; ++j) {
-        float4 a0[kStreamK], a1[kStreamK], a2[kStreamK], c0[kStreamK], c1[kStreamK], c2[kStreamK];
+    // blockIdx.y selects a group of consecutive time steps (one group on large grids)
+    const int jn = (nt + gridDim.y - 1) / gridDim.y, j0 = blockIdx.y * jn, j1 = min(j0 + jn, nt);
+    for (int j = j0; j < j1; ++j) {
+        float4 a0[K], a1[K], a2[K], c0[K], c1[K], c2[K];
 #pragma unroll
-        for (int k = 0; k < kStreamK; ++k) {
+        for (int k = 0; k < K; ++k) {
             const int64_t i = min(i0 + 64 * k, nl4 - 1);
             a0[k] = p.gX.load(3 * j, nl, i); a1[k] = p.gX.load(3 * j + 1, nl, i); a2[k] = p.gX.load(3 * j + 2, nl, i);
             c0[k] = p.gm.load(3 * (j + 1), nl, i); c1[k] = p.gm.load(3 * (j + 1) + 1, nl, i);
             c2[k] = p.gm.load(3 * (j + 1) + 2, nl, i);
         }
 #pragma unroll
-        for (int k = 0; k < kStreamK; ++k) {
+        for (int k = 0; k < K; ++k) {
             const int64_t i = i0 + 64 * k;
             if (i >= nl4) continue;
             float4 s;
@@ -902,37 +903,46 @@ struct BodyP {
     float* b[3];
 };
 
-template <class Src>
+template <class Src, int K, int J>
 __global__ __launch_bounds__(256) void k_body_force(int64_t nl4, int nt, float ht, float hd, BodyP<Src> p) {
-    const int64_t i0 = stream_base(kStreamK);
+    const int64_t i0 = stream_base(K);
     const int64_t nl = nl4 * 4;
-    float4 s[kStreamK][3];
+    float4 s[K][3];
 #pragma unroll
-    for (int k = 0; k < kStreamK; ++k)
+    for (int k = 0; k < K; ++k)
 #pragma unroll
         for (int d = 0; d < 3; ++d) s[k][d] = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int j = 0; j <= nt; ++j) {
-        const float w = (j == 0 || j == nt) ? 0.5f * ht : ht;
-        float4 l[kStreamK], g[kStreamK][3];
+    for (int j0 = 0; j0 <= nt; j0 += J) {  // J time steps in flight
+        float4 l[J][K], g[J][K][3];
 #pragma unroll
-        for (int k = 0; k < kStreamK; ++k) {
-            const int64_t i = min(i0 + 64 * k, nl4 - 1);  // past the end: reload the last group, never stored
-            l[k] = ld4(p.lam + static_cast<int64_t>(j) * nl, i);
+        for (int jj = 0; jj < J; ++jj) {
+            const int j = min(j0 + jj, nt);
 #pragma unroll
-            for (int d = 0; d < 3; ++d) g[k][d] = p.gm.load(3 * (nt - j) + d, nl, i);
+            for (int k = 0; k < K; ++k) {
+                const int64_t i = min(i0 + 64 * k, nl4 - 1);  // past the end: reload the last group, never stored
+                l[jj][k] = ld4(p.lam + static_cast<int64_t>(j) * nl, i);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) g[jj][k][d] = p.gm.load(3 * (nt - j) + d, nl, i);
+            }
         }
 #pragma unroll
-        for (int k = 0; k < kStreamK; ++k)
+        for (int jj = 0; jj < J; ++jj) {
+            const int j = j0 + jj;
+            if (j > nt) break;
+            const float w = (j == 0 || j == nt) ? 0.5f * ht : ht;
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                s[k][d].x += w * g[k][d].x * l[k].x;
-                s[k][d].y += w * g[k][d].y * l[k].y;
-                s[k][d].z += w * g[k][d].z * l[k].z;
-                s[k][d].w += w * g[k][d].w * l[k].w;
-            }
+            for (int k = 0; k < K; ++k)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    s[k][d].x += w * g[jj][k][d].x * l[jj][k].x;
+                    s[k][d].y += w * g[jj][k][d].y * l[jj][k].y;
+                    s[k][d].z += w * g[jj][k][d].z * l[jj][k].z;
+                    s[k][d].w += w * g[jj][k][d].w * l[jj][k].w;
+                }
+        }
     }
 #pragma unroll
-    for (int k = 0; k < kStreamK; ++k) {
+    for (int k = 0; k < K; ++k) {
         const int64_t i = i0 + 64 * k;
         if (i >= nl4) continue;
 #pragma unroll
@@ -1268,14 +1278,26 @@ void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, int 
     }
 }
 
+// Points from which the streaming kernels are bound by memory and take two runs per
+// wave.  Below, they wait for their loads with too few waves to hide them: one run per
+// wave, four of the body force's time steps in flight at once, and the right-hand
+// sides' time steps shared out over up to four groups of blocks (each time step is
+// independent of the others).  Body force 6.4 -> 4.4 µs at 32³, 10.3 -> 6.6 at 64³;
+// right-hand sides 6.9 -> 2.9 and 9.8 -> 8.4, but 21.8 -> 27.5 at 96³ and 157 -> 241
+// at 192³, where every group reads the velocities again.
+constexpr int64_t kStreamPoints = int64_t(1) << 19;
+unsigned stream_blocks(int64_t nl4, int k) { return static_cast<unsigned>((nl4 + 256 * k - 1) / (256 * k)); }
+
 template <class Src>
 void body_force(int64_t nl, int nt, float ht, float hd, const float* lam, const Src& gm, float* const b[3],
                 hipStream_t st) {
     CLR_REQUIRE(nl % 4 == 0, kErrInvalidArgument, "grid size must be a multiple of 4 points");
     const int64_t nl4 = nl / 4;
     BodyP<Src> p{lam, gm, {b[0], b[1], b[2]}};
-    const int nb = static_cast<int>((nl4 + 256 * kStreamK - 1) / (256 * kStreamK));
-    hipLaunchKernelGGL((k_body_force<Src>), dim3(nb), dim3(256), 0, st, nl4, nt, ht, hd, p);
+    if (nl < kStreamPoints)
+        hipLaunchKernelGGL((k_body_force<Src, 1, 4>), dim3(stream_blocks(nl4, 1)), dim3(256), 0, st, nl4, nt, ht, hd, p);
+    else
+        hipLaunchKernelGGL((k_body_force<Src, 2, 1>), dim3(stream_blocks(nl4, 2)), dim3(256), 0, st, nl4, nt, ht, hd, p);
 }
 
 template <class Src>
@@ -1285,8 +1307,11 @@ void inc_state_rhs(int64_t nl, int nt, float ht, const float* const vx[3], const
     CLR_REQUIRE(nt >= 1, kErrInvalidArgument, "nt must be >= 1");
     const int64_t nl4 = nl / 4;
     RhsP<Src> p{{vx[0], vx[1], vx[2]}, {vt[0], vt[1], vt[2]}, gX, gm, s, mt1};
-    const int nb = static_cast<int>((nl4 + 256 * kStreamK - 1) / (256 * kStreamK));
-    hipLaunchKernelGGL((k_inc_state_rhs<Src>), dim3(nb), dim3(256), 0, st, nl4, nt, 0.5f * ht, p);
+    if (nl < kStreamPoints)
+        hipLaunchKernelGGL((k_inc_state_rhs<Src, 1>), dim3(stream_blocks(nl4, 1), std::min(nt, 4)), dim3(256), 0, st, nl4,
+                           nt, 0.5f * ht, p);
+    else
+        hipLaunchKernelGGL((k_inc_state_rhs<Src, 2>), dim3(stream_blocks(nl4, 2)), dim3(256), 0, st, nl4, nt, 0.5f * ht, p);
 }
 
 int64_t bfp16_blocks(int64_t nl) { return (nl / 4 + kBfpBlock4 - 1) / kBfpBlock4; }
