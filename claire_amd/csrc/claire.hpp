@@ -509,7 +509,7 @@ class CLAIRE {
     std::unique_ptr<SemiLagrangian> m_SL;
 
     std::unique_ptr<VecField> m_VelocityField, m_IncVelocityField, m_BodyForce, m_IncBodyForce, m_WorkVecField1;
-    DeviceArray<float> m_TemplateImage, m_ReferenceImage;
+    DeviceArray<float> m_ReferenceImage;
     DeviceArray<float> m_State;          // (nt+1)·nl
     DeviceArray<float> m_Adjoint;        // λ at t = 0
     DeviceArray<float> m_IncState[2];    // ping-pong m̃
