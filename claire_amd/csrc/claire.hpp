@@ -331,6 +331,8 @@ class SemiLagrangian {
     int Interpolate(VecField* vo, const VecField* vi, const std::string& flag);
     // Out-of-place gathers along a trajectory (no aliasing allowed).
     void Gather(float* xo, const float* xi, const std::string& flag);
+    // n fields, one after another in memory, in launches of several
+    void GatherSeries(const float* in, float* out, int n, const std::string& flag);
     void Gather3(const float* const in[3], float* const out[3], const std::string& flag);
     // Trajectory X into out (3 floats per point, normalized by 2π; the
     // reference's m_X)
