@@ -58,7 +58,17 @@ __device__ __forceinline__ float wrap_q(float q, float hh) {
 
 // Rescaled index-space coordinate u = q·N + 3 (rescale_xyz, src/interp3.cpp:44-47).
 __device__ __forceinline__ float index_coord(float q, int n, float hh) {
-    return wrap_q(q, hh) * static_cast<float>(n) + 3.0f;
+    return fmaf(wrap_q(q, hh), static_cast<float>(n), 3.0f);
+}
+
+// Euler predictor (x − s·v)/2π of one axis at grid index i.  The rounding is
+// spelled out because a plan's displacement bound and the plan itself come from
+// different kernels: left to the compiler, x − s·v and x + s·v of one kernel
+// shared their products and rounded differently from the plan's, and a point
+// within a rounding of a cell boundary then lay outside the window its bound
+// promised.
+__device__ __forceinline__ float euler_predictor(float hx, int i, float s, float v) {
+    return static_cast<float>(over_2pi(static_cast<double>(fmaf(hx, static_cast<float>(i), -(s * v)))));
 }
 
 // Grid index of the first stencil node before the periodic wrap: floor(u) − 4.

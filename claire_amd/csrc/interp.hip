@@ -260,8 +260,8 @@ __global__ __launch_bounds__(kThreads) void k_make_plan(GatherDims g, HH hh, con
     block_max_to(need, bmax);
 }
 
-// Plan of the Euler predictor X̃ = (x − σ·ht·v)/2π, with the same float and
-// double steps as k_traj_rk2 (bounded grid, like k_make_plan).
+// Plan of the Euler predictor X̃ = (x − σ·ht·v)/2π (bounded grid, like
+// k_make_plan).
 //   SETV = false: the plan alone, its bound known already.
 //   SETV = true:  the first pass over a new velocity, which it copies to `vout`
 //                 (unless that is where it lies): the predictor's plan for σ and
@@ -293,10 +293,9 @@ __global__ __launch_bounds__(kThreads) void k_predictor_plan(GatherDims g, HH hh
             for (int d = 0; d < 3; ++d) vn[d] = v.in[d][i + stride];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            const float x = tp.hx[d] * static_cast<float>(gw.idx[d]);
-            q[d] = static_cast<float>(over_2pi(static_cast<double>(x - tp.sht * vd[d])));
+            q[d] = euler_predictor(tp.hx[d], gw.idx[d], tp.sht, vd[d]);
             if constexpr (SETV) {
-                r[d] = static_cast<float>(over_2pi(static_cast<double>(x + tp.sht * vd[d])));
+                r[d] = euler_predictor(tp.hx[d], gw.idx[d], -tp.sht, vd[d]);
                 need[2] |= fabsf(vd[d]) > 0.0f;
                 if (vout) vout[d * g.nl + i] = vd[d];
             }
