@@ -32,6 +32,7 @@ thread_local std::string g_err;
 template <class F>
 int guard(F&& f) {
     try {
+        claire_amd::note_pending_error();
         f();
         return CLR_OK;
     } catch (const Error& e) {

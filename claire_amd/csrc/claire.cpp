@@ -25,6 +25,16 @@ Dims make_dims(const int nx[3]) {
     return d;
 }
 
+namespace {
+thread_local bool g_pending_error = false;
+}  // namespace
+
+void note_pending_error() { g_pending_error = hipPeekAtLastError() != hipSuccess; }
+
+void check_launches() {
+    if (!g_pending_error) CLR_HIP_CHECK(hipGetLastError());
+}
+
 }  // namespace claire_amd
 
 namespace reg {
@@ -120,7 +130,7 @@ void Reducer::SumPartialsTo(const double* partial, int np, int slot) {
 
 void Reducer::Fetch(double* out, int nslots) {
     CLR_REQUIRE(nslots >= 1 && nslots <= kSlots, kErrInvalidArgument, "reduction slot count out of range");
-    CLR_HIP_CHECK(hipGetLastError());  // a launch that failed wrote no result
+    check_launches();  // a launch that failed wrote no result
     CLR_HIP_CHECK(hipStreamSynchronize(m_Opt->stream));
     std::copy(m_Host.get(), m_Host.get() + nslots, out);
 }
@@ -469,6 +479,8 @@ int SemiLagrangian::Which(const std::string& flag) const {
 
 bool SemiLagrangian::SetVelocity(const float* v, VecField* dst) {
     const size_t n = 3 * static_cast<size_t>(m_Opt->domain.nl);
+    ForgetVelocity();     // until the bounds are known
+    m_Valid[0] = false;   // its plan is overwritten
     m_P[0].resize(n);
     // bytes: v read (12), copied (12) and the plan written (12) per point
     KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 36.0 * m_Opt->domain.nl);
@@ -478,7 +490,6 @@ bool SemiLagrangian::SetVelocity(const float* v, VecField* dst) {
     m_PredBound[1] = b.dbound[1];
     m_PredOrder = m_Opt->rkorder;
     m_PredInPlan = true;
-    m_Valid[0] = false;  // its plan is gone
     return b.zero;
 }
 
@@ -707,7 +718,7 @@ void CLAIRE::RequireVelocity() const { CLR_REQUIRE(m_HaveVelocity, kErrState, "v
 
 int CLAIRE::SetControlVariable(const float* v) {
     CLR_REQUIRE(v != nullptr, kErrInvalidArgument, "null input vector");
-    m_HaveVelocity = true;
+    m_HaveVelocity = false;  // until the new one is in place
     DropTrajectories();
     m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;
     ++m_GraphEpoch;
@@ -719,6 +730,7 @@ int CLAIRE::SetControlVariable(const float* v) {
         m_VelocityField->SetComponents(v);
         m_VelocityIsZero = m_Red->AbsMax(m_VelocityField->m_X1, 3 * m_Opt.domain.nl) == 0.0;
     }
+    m_HaveVelocity = true;
     return 0;
 }
 

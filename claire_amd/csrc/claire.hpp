@@ -324,7 +324,10 @@ class SemiLagrangian {
     // computed from `dst` afterwards use them.
     bool SetVelocity(const float* v, VecField* dst);
     // The velocity field changed without SetVelocity.
-    void ForgetVelocity() { m_PredOrder = 0; }
+    void ForgetVelocity() {
+        m_PredOrder = 0;
+        m_PredInPlan = false;
+    }
     // flag "state" (σ = +1) or "adjoint" (σ = −1)
     int ComputeTrajectory(const VecField* v, const std::string& flag);
     int Interpolate(float* xo, const float* xi, const std::string& flag);

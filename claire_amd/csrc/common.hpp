@@ -34,6 +34,13 @@ enum Status : int {
                                       std::string(#expr) + ": " + hipGetErrorString(_e));                  \
     } while (0)
 
+// Throws if a kernel launch of this entry point failed: before the host reads
+// pinned words that the kernel was to write.  HIP keeps one last error per
+// thread; one that was pending when the entry point began (another library's)
+// says nothing about its launches and is left alone.
+void check_launches();
+void note_pending_error();  // at the start of an entry point
+
 #define CLR_REQUIRE(cond, code, msg)                                                                       \
     do {                                                                                                   \
         if (!(cond)) throw ::claire_amd::Error((code), (msg));                                             \

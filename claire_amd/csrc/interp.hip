@@ -451,7 +451,7 @@ void launch_trajectory_rk4_stage(int stage, const Dims& d, const float* const v[
 namespace {
 // The bound of a plan launch of nb blocks, after waiting for the stream.
 int plan_bound(const int* bmax, int nb, hipStream_t st) {
-    CLR_HIP_CHECK(hipGetLastError());  // a launch that failed wrote no maxima
+    check_launches();  // a launch that failed wrote no maxima
     CLR_HIP_CHECK(hipStreamSynchronize(st));
     return *std::max_element(bmax, bmax + nb);
 }

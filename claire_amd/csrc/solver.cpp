@@ -172,7 +172,7 @@ int Optimizer::Pcg(const float* g, double rtol, const GNOptions& opt, GNReport& 
                 PcgIteration(false, opt);
         }
         ++runs;
-        CLR_HIP_CHECK(hipGetLastError());  // a launch that failed wrote no state
+        check_launches();  // a launch that failed wrote no state
         CLR_HIP_CHECK(hipStreamSynchronize(Stream()));
         hs = *m_HostState.get();
         its = hs.k;
