@@ -279,7 +279,7 @@ void SpectralOps::Gradients(float* g, int64_t gs, int64_t gc, const float* f, in
 }
 
 int SpectralOps::SeriesFields(int n) const {
-    const int64_t most = std::max<int64_t>(1, kSeriesPoints / m_Opt->domain.nl);
+    const int64_t most = std::clamp<int64_t>(kSeriesPoints / m_Opt->domain.nl, 1, FFTPlan3D::kMaxFields / 3);
     const int groups = static_cast<int>((n + most - 1) / most);
     return (n + groups - 1) / groups;
 }
@@ -604,7 +604,8 @@ constexpr int64_t kGatherSeriesPoints = int64_t(1) << 26;
 void SemiLagrangian::GatherSeries(const float* in, float* out, int n, const std::string& flag) {
     const TrajectoryPlan tp = Plan(flag);
     const GatherDims g = gather_dims(m_Opt->domain);
-    const int most = static_cast<int>(std::min<int64_t>(n, std::max<int64_t>(kGatherSeriesPoints / g.nl / 3, 1) * 3));
+    const int most = static_cast<int>(
+        std::min<int64_t>(n, std::clamp<int64_t>(kGatherSeriesPoints / g.nl / 3, 1, kMaxGatherFields / 3) * 3));
     std::vector<const float*> f(most);
     std::vector<float*> o(most);
     for (int k0 = 0; k0 < n; k0 += most) {

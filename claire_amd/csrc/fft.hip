@@ -1116,18 +1116,18 @@ FFTPlan3D::~FFTPlan3D() {
 }
 
 void FFTPlan3D::x3_r2c(const float* in, int64_t is, c32* out, int64_t os, int n, hipStream_t st) const {
-    CLR_REQUIRE(n >= 1 && n <= 65535, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
+    CLR_REQUIRE(n >= 1 && n <= kMaxFields, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
     const R2CPtrs p{in, is, out, os};
     dispatch_n<RowR2C>(dims.n[2], p, n, static_cast<int64_t>(dims.n[0]) * dims.n[1], tw[2], st);
 }
 void FFTPlan3D::x3_c2r(const c32* in, int64_t is, float* out, int64_t os, int n, hipStream_t st, float alpha,
                        const float* add, int64_t as, float beta) const {
-    CLR_REQUIRE(n >= 1 && n <= 65535, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
+    CLR_REQUIRE(n >= 1 && n <= kMaxFields, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
     const C2RPtrs p{in, is, out, os, add, as};
     dispatch_n<RowC2R>(dims.n[2], p, n, static_cast<int64_t>(dims.n[0]) * dims.n[1], tw[2], alpha, beta, st);
 }
 void FFTPlan3D::x2(c32* data, int64_t ds, int n, int dir, hipStream_t st) const {
-    CLR_REQUIRE(n >= 1 && n <= 65535, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
+    CLR_REQUIRE(n >= 1 && n <= kMaxFields, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
     const ColPtrs p{data, ds};
     dispatch_n<ColPass>(dims.n[1], p, n, geom_x2(dims), dir, tw[1], st);
 }
@@ -1155,7 +1155,7 @@ void FFTPlan3D::x1_norm(const c32* in, int64_t is, int n, const SpecParams& sp, 
 }
 
 void FFTPlan3D::x1_grad(const c32* in, int64_t is, c32* out, int64_t os, int64_t oc, int n, hipStream_t st) const {
-    CLR_REQUIRE(n >= 1 && n <= 65535, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
+    CLR_REQUIRE(n >= 1 && n <= kMaxFields, kErrInvalidArgument, "1 to 65535 fields per FFT pass");
     const X1Ptrs p{in, is, out, os, oc};
     SpecParams sp{};
     sp.scale = dims.scale;

@@ -28,8 +28,10 @@ class FFTPlan3D {
     FFTPlan3D(const FFTPlan3D&) = delete;
     FFTPlan3D& operator=(const FFTPlan3D&) = delete;
 
-    // Individual passes over n fields in one launch, field f at in + f·is (and
-    // out + f·os, add + f·as): a vector field's components or a time series.
+    // Individual passes over n fields in one launch (blockIdx.y), field f at in +
+    // f·is (and out + f·os, add + f·as): a vector field's components or a time
+    // series.
+    static constexpr int kMaxFields = 65535;
     void x3_r2c(const float* in, int64_t is, c32* out, int64_t os, int n, hipStream_t st) const;
     // out = alpha·x + beta·add (add may be null, or equal out with as = os)
     void x3_c2r(const c32* in, int64_t is, float* out, int64_t os, int n, hipStream_t st, float alpha = 1.f,
@@ -166,10 +168,12 @@ struct TrajectoryPlan {
 
 // Gathers along a trajectory.  Vector fields are nf equally spaced component
 // pointers.  They run the LDS-staged kernels when dbound allows, else the
-// direct kernels on the raw foot points.
+// direct kernels on the raw foot points (which take the field from blockIdx.y:
+// at most kMaxGatherFields of them).
 //   gather:          out_d = f_d(X)
 //   inc_state_step:  out = ±(f(X) − s)   (m̃^{j+1} = m̃^j(X_s) − s_j; negated for λ̃⁰ = −m̃^nt)
 //   adjoint_step:    out = C·f(X)        (λ^{j+1} = C·λ^j(X_a))
+constexpr int kMaxGatherFields = 65535;
 void launch_plan_gather(const TrajectoryPlan& tp, const GatherDims& g, const float* const f[], int nf,
                         float* const out[], hipStream_t st);
 void launch_plan_inc_state_step(const TrajectoryPlan& tp, const GatherDims& g, const float* mt, const float* sj,
