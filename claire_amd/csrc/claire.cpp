@@ -284,10 +284,14 @@ int SpectralOps::SeriesFields(int n) const {
     return (n + groups - 1) / groups;
 }
 
+void SpectralOps::ReserveSeries(int n) {
+    m_SeriesSpec.resize(SeriesSpectra(n) * static_cast<size_t>(m_Opt->domain.nlc));
+}
+
 void SpectralOps::GradSeries(float* g, const float* f, int n) {
     const Dims& d = m_Opt->domain;
     const int per = SeriesFields(n);
-    if (per > 1) m_SeriesSpec.resize(3 * static_cast<size_t>(per) * d.nlc);
+    ReserveSeries(n);
     for (int j = 0; j < n; j += per)
         Gradients(g + 3 * j * d.nl, 3 * d.nl, d.nl, f + j * d.nl, d.nl, std::min(per, n - j),
                   per > 1 ? m_SeriesSpec.get() : m_Spec.get());
@@ -477,11 +481,27 @@ int SemiLagrangian::Which(const std::string& flag) const {
     throw Error(kErrInvalidArgument, "flag wrong");  // src/SemiLagrangian.cpp:221-223
 }
 
-bool SemiLagrangian::SetVelocity(const float* v, VecField* dst) {
+bool SemiLagrangian::Capturing() const {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;  // never of the null stream
+    return m_Opt->stream && hipStreamIsCapturing(m_Opt->stream, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+}
+
+void SemiLagrangian::Reserve() {
     const size_t n = 3 * static_cast<size_t>(m_Opt->domain.nl);
+    for (int w = 0; w < 2; ++w) {
+        m_X[w].resize(n);
+        m_P[w].resize(n);
+    }
+    if (m_Opt->rkorder == 4) {
+        m_F.resize(n);
+        m_F2.resize(n);
+    }
+}
+
+bool SemiLagrangian::SetVelocity(const float* v, VecField* dst) {
     ForgetVelocity();     // until the bounds are known
     m_Valid[0] = false;   // its plan is overwritten
-    m_P[0].resize(n);
+    Reserve();
     // bytes: v read (12), copied (12) and the plan written (12) per point
     KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 36.0 * m_Opt->domain.nl);
     const VelocityBounds b = launch_set_velocity(m_Opt->domain, v, dst->m_X1, PredictorStep(), m_P[0].get(),
@@ -496,31 +516,28 @@ bool SemiLagrangian::SetVelocity(const float* v, VecField* dst) {
 int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag) {
     const int w = Which(flag);
     CLR_REQUIRE(m_Opt->rkorder == 2 || m_Opt->rkorder == 4, kErrInvalidArgument, "rk order must be 2 or 4");
-    if (m_PredOrder != m_Opt->rkorder) {
+    const bool capturing = Capturing();
+    if (!capturing && m_PredOrder != m_Opt->rkorder) {
         // the velocity was set before the scheme or the time integrator was
         VecField same(m_Opt, v->m_X1);
         SetVelocity(v->m_X1, &same);
     }
     const int64_t nl = m_Opt->domain.nl;
-    const size_t n = 3 * static_cast<size_t>(nl);
-    m_X[w].resize(n);
-    m_P[w].resize(n);
+    Reserve();
     float* const X = m_X[w].get();
     uint32_t* const P = m_P[w].get();
     const GatherDims g = gather_dims(m_Opt->domain);
     const float* vc[3] = {v->m_X1, v->m_X2, v->m_X3};
     const float sigma = w == 0 ? 1.0f : -1.0f;
     const float ht = m_Opt->GetTimeStepSize();
-    int db = m_PredBound[w];
+    int db = capturing ? kNoBound : m_PredBound[w];
     if (plan_gather_lds(g, db, 3) && !(w == 0 && m_PredInPlan)) {
         // bytes: v read (12) + plan written (12) per point
         KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 24.0 * nl);
         launch_predictor_plan(m_Opt->domain, vc, sigma, PredictorStep(), P, m_Opt->stream);
     }
-    if (w == 0) m_PredInPlan = false;
+    if (w == 0 && !capturing) m_PredInPlan = false;
     if (m_Opt->rkorder == 4) {
-        m_F.resize(n);
-        m_F2.resize(n);
         float* const fbuf[4] = {nullptr, m_F.get(), m_F2.get(), nullptr};
         for (int stage = 1; stage <= 3; ++stage) {
             if (plan_gather_lds(g, db, 3)) {
@@ -550,6 +567,11 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
         // bytes: v read (12) + v gathered (12) + X written (12) per point
         KernelScope k(m_Opt->prof, "gather_traj_rk2", 36.0 * nl);
         launch_trajectory_rk2(m_Opt->domain, vc, sigma, ht, X, m_Opt->stream);
+    }
+    if (capturing) {
+        m_D[w] = kNoBound;  // and no plan, which eager calls may hold with its bound
+        m_Valid[w] = true;
+        return 0;
     }
     // bytes: X read (12) + packed plan written (12) per point
     KernelScope k(m_Opt->prof, "gather_plan", 24.0 * nl);
@@ -684,6 +706,7 @@ CLAIRE::CLAIRE(const RegOpt& opt) : m_Opt(opt) {
     m_Scalar.resize(nl);
     m_AdjCoeff.resize(nl);
     m_VtX.resize(3 * nl);
+    m_Spectral->ReserveSeries(m_Opt.nt + 1);
 }
 
 CLAIRE::~CLAIRE() {
@@ -768,10 +791,12 @@ void CLAIRE::EnsureTrajectory(const std::string& flag) {
 
 void CLAIRE::EnsureStateTrajectory() {
     RequireVelocity();
+    NoteCapture();
     if (m_StateTrajValid) return;
     m_SL->ComputeTrajectory(m_VelocityField.get(), "state");
-    m_StateTrajValid = true;
+    m_StateTrajValid = !m_SL->Capturing();  // else captured, not computed
     ++m_GraphEpoch;
+    if (m_KeepBoth && m_StateTrajValid) EnsureAdjointTrajectory();
 }
 
 void CLAIRE::EnsureDivergence() {
@@ -779,11 +804,12 @@ void CLAIRE::EnsureDivergence() {
     if (m_DivValid) return;
     const float* vc[3] = {m_VelocityField->m_X1, m_VelocityField->m_X2, m_VelocityField->m_X3};
     m_Spectral->Div(m_Scalar.get(), vc);
-    m_DivValid = true;
+    m_DivValid = !m_SL->Capturing();
 }
 
 void CLAIRE::EnsureAdjointTrajectory() {
     RequireVelocity();
+    NoteCapture();
     if (m_AdjTrajValid) return;
     m_SL->ComputeTrajectory(m_VelocityField.get(), "adjoint");
     // the adjoint update coefficient at every point from ∇·v
@@ -798,8 +824,9 @@ void CLAIRE::EnsureAdjointTrajectory() {
         launch_plan_adjoint_coeff(m_SL->Plan("adjoint"), gather_dims(m_Opt.domain), m_Scalar.get(),
                                   m_Opt.GetTimeStepSize(), 1.0f, m_AdjCoeff.get(), m_Opt.stream);
     }
-    m_AdjTrajValid = true;
+    m_AdjTrajValid = !m_SL->Capturing();
     ++m_GraphEpoch;
+    if (m_KeepBoth && m_AdjTrajValid) EnsureStateTrajectory();
 }
 
 int CLAIRE::SolveStateEquation() {
@@ -823,11 +850,10 @@ int CLAIRE::SolveStateEquation() {
             // ht·dX)·d), d = ∇·v, dX = d(X_s): the α = −1 form of the
             // coefficient on the state trajectory (src/CLAIRE.cpp:2813-2835)
             EnsureDivergence();
-            m_StateCoeff.resize(static_cast<size_t>(nl));
             KernelScope k(m_Opt.prof, "gather_state_coeff", 24.0 * nl);
             launch_plan_adjoint_coeff(tp, g, m_Scalar.get(), m_Opt.GetTimeStepSize(), -1.0f, m_StateCoeff.get(),
                                       m_Opt.stream);
-            m_StateCoeffValid = true;
+            m_StateCoeffValid = !m_SL->Capturing();
         }
         for (int j = 0; j < nt; ++j) {
             KernelScope k(m_Opt.prof, "continuity_step", 24.0 * nl);
@@ -931,6 +957,7 @@ int CLAIRE::SetRKOrder(int order) {
 int CLAIRE::SetPDEType(int type) {
     CLR_REQUIRE(type == 0 || type == 1, kErrInvalidArgument, "pde type must be 0 (continuity) or 1 (transport)");
     if (type != m_Opt.pdetype) {
+        if (type == 0) m_StateCoeff.resize(static_cast<size_t>(m_Opt.domain.nl));
         m_Opt.pdetype = type;
         DropTrajectories();
         m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;

@@ -246,6 +246,7 @@ class SpectralOps {
     // 2322 -> 2257 at 192³, 4.34 ms either way at 256³ (one field per launch).
     void GradSeries(float* g, const float* f, int n);
     static constexpr int64_t kSeriesPoints = int64_t(1) << 24;
+    void ReserveSeries(int n);
     // half spectra GradSeries keeps beside the three of the other operators
     size_t SeriesSpectra(int n) const { return SeriesFields(n) > 1 ? 3 * static_cast<size_t>(SeriesFields(n)) : 0; }
     void Div(float* d, const float* const v[3]);
@@ -265,7 +266,7 @@ class SpectralOps {
     void Gradients(float* g, int64_t gs, int64_t gc, const float* f, int64_t fs, int n, c32* spec);
     int SeriesFields(int n) const;
     DeviceArray<c32> m_Spec;        // three half spectra
-    DeviceArray<c32> m_SeriesSpec;  // GradSeries, allocated on its first call
+    DeviceArray<c32> m_SeriesSpec;  // GradSeries
     DeviceArray<double> m_NormPartial;  // block sums of Norm3, allocated on its first call
 };
 
@@ -328,8 +329,12 @@ class SemiLagrangian {
         m_PredOrder = 0;
         m_PredInPlan = false;
     }
-    // flag "state" (σ = +1) or "adjoint" (σ = −1)
+    // flag "state" (σ = +1) or "adjoint" (σ = −1).  While the stream is being
+    // captured the direct kernels form the foot points alone: a wait for the
+    // displacement bound that the others are chosen by is not possible there.
     int ComputeTrajectory(const VecField* v, const std::string& flag);
+    // Whether the stream is being captured into a graph.
+    bool Capturing() const;
     int Interpolate(float* xo, const float* xi, const std::string& flag);
     int Interpolate(VecField* vo, const VecField* vi, const std::string& flag);
     // Out-of-place gathers along a trajectory (no aliasing allowed).
@@ -350,6 +355,7 @@ class SemiLagrangian {
 
   private:
     int Which(const std::string& flag) const;
+    void Reserve();  // the buffers of both trajectories (none can be allocated in a capture)
     const RegOpt* m_Opt;
     float PredictorStep() const { return (m_Opt->rkorder == 4 ? 0.5f : 1.0f) * m_Opt->GetTimeStepSize(); }
     DeviceArray<float> m_X[2];  // foot points, one component per field
@@ -466,6 +472,10 @@ class CLAIRE {
     void EnsureStateTrajectory();
     void EnsureAdjointTrajectory();
     void EnsureDivergence();  // m_Scalar = ∇·v
+    // Called before a trajectory is used.
+    void NoteCapture() {
+        if (m_Opt.stream != m_CaptureStream && m_SL->Capturing()) m_KeepBoth = true;
+    }
     void DropTrajectories() { m_StateTrajValid = m_AdjTrajValid = m_DivValid = m_StateCoeffValid = false; }
     void EnsureStateGradients();
     void EnsureGradientsAtStateTrajectory();
@@ -540,6 +550,10 @@ class CLAIRE {
     bool m_HaveVelocity = false, m_HaveIncVelocity = false, m_HaveTemplate = false, m_HaveReference = false;
     bool m_VelocityIsZero = false;
     bool m_StateTrajValid = false, m_AdjTrajValid = false, m_DivValid = false, m_StateCoeffValid = false;
+    // A trajectory was used while a caller captured its stream.  The caller may
+    // replay that graph at another velocity, after any call that used to form
+    // both trajectories: from then on they are formed together.
+    bool m_KeepBoth = false;
     bool m_StateValid = false, m_GradMValid = false, m_GradMXValid = false;
 };
 

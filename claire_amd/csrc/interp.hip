@@ -210,7 +210,7 @@ __device__ __forceinline__ void block_max_to(int (&v)[K], int* bmax) {
 }
 
 // Encodes the three axes of foot point q at grid index idx; returns the
-// displacement bound this point needs (1 << 20 when not encodable).
+// displacement bound this point needs (kNoBound when not encodable).
 __device__ __forceinline__ int encode_point(const GatherDims& g, const HH& hh, const float q[3], const int idx[3],
                                             PlanPt& pt) {
     const int n[3] = {g.n1, g.n2, g.n3};
@@ -220,7 +220,7 @@ __device__ __forceinline__ int encode_point(const GatherDims& g, const HH& hh, c
         const float u = index_coord(q[a], n[a], hh.h[a]);
         int lo = 0;
         if (!plan_encode(u, idx[a], n[a], pt.w[a], lo)) {
-            need = 1 << 20;
+            need = kNoBound;
             pt.w[a] = 0u;  // t = 1, o = 0: never read
             continue;
         }
@@ -232,7 +232,7 @@ __device__ __forceinline__ int encode_point(const GatherDims& g, const HH& hh, c
 // Packed plan of a trajectory (gather_device.hpp) and the smallest D such
 // that every stencil lies within [i − D − 1, i + D + 2] per axis (the window
 // of the LDS-staged gathers).  Points that cannot be encoded (non-finite
-// coordinates) set D to 1 << 20, which routes every gather along this
+// coordinates) set D to kNoBound, which routes every gather along this
 // trajectory to the direct kernels on the raw foot points.
 //
 // Each block writes its maximum into its own word of a host-resident array,

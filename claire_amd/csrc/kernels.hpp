@@ -107,10 +107,11 @@ void launch_trajectory_rk4_stage(int stage, const Dims& d, const float* const v[
 // fraction t ∈ [1,2) of the rescaled coordinate u = q·N + 3 and the offset of
 // the first stencil node from the point (layout in gather_device.hpp).
 // Returns the per-axis stencil displacement bound D in cells (synchronizes
-// the stream); 1 << 20 when a foot point is not finite.  n <= 512 per axis.
+// the stream); kNoBound when a foot point is not finite.  n <= 512 per axis.
 // `bmax`: 3·kPlanBlocks ints of pinned host memory that the device can write
 // (the blocks' bounds; one launch at a time may use them).
 constexpr int kPlanBlocks = 2048;
+constexpr int kNoBound = 1 << 20;
 int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* bmax, hipStream_t st);
 // RK2 characteristic through the LDS-staged gather, in three passes:
 //   1. the packed plan of the Euler predictor X̃ = (x − σ·ht·v)/2π into P
