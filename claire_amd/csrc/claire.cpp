@@ -473,7 +473,7 @@ int Regularization::GetExtremeEigValsInvOp(ScalarType& emin, ScalarType& emax) {
 // ---------------------------------------------------------------------------
 // SemiLagrangian (src/SemiLagrangian.cpp)
 // ---------------------------------------------------------------------------
-SemiLagrangian::SemiLagrangian(const RegOpt* opt) : m_Opt(opt), m_PlanMax(3 * kPlanBlocks) {}
+SemiLagrangian::SemiLagrangian(const RegOpt* opt) : m_Opt(opt), m_PlanWords(2 * kPlanBlocks) {}
 
 int SemiLagrangian::Which(const std::string& flag) const {
     if (flag == "state") return 0;
@@ -505,9 +505,9 @@ bool SemiLagrangian::SetVelocity(const float* v, VecField* dst) {
     // bytes: v read (12), copied (12) and the plan written (12) per point
     KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 36.0 * m_Opt->domain.nl);
     const VelocityBounds b = launch_set_velocity(m_Opt->domain, v, dst->m_X1, PredictorStep(), m_P[0].get(),
-                                                 m_PlanMax.get(), m_Opt->stream);
-    m_PredBound[0] = b.dbound[0];
-    m_PredBound[1] = b.dbound[1];
+                                                 m_PlanWords.get(), m_Opt->stream);
+    m_PredBound[0] = b.bound[0];
+    m_PredBound[1] = b.bound[1];
     m_PredOrder = m_Opt->rkorder;
     m_PredInPlan = true;
     return b.zero;
@@ -530,7 +530,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
     const float* vc[3] = {v->m_X1, v->m_X2, v->m_X3};
     const float sigma = w == 0 ? 1.0f : -1.0f;
     const float ht = m_Opt->GetTimeStepSize();
-    int db = capturing ? kNoBound : m_PredBound[w];
+    PlanBound db = capturing ? PlanBound{kNoBound, 0.0f} : m_PredBound[w];
     if (plan_gather_lds(g, db, 3) && !(w == 0 && m_PredInPlan)) {
         // bytes: v read (12) + plan written (12) per point
         KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 24.0 * nl);
@@ -550,7 +550,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
                 if (stage == 3) break;
                 // bytes: point read (12) + plan (12)
                 KernelScope k(m_Opt->prof, "gather_plan", 24.0 * nl);
-                db = launch_make_plan(g, X, P, m_PlanMax.get(), m_Opt->stream);
+                db = launch_make_plan(g, X, P, m_PlanWords.get(), m_Opt->stream);
             } else {
                 // this stage's point is not for the LDS gathers, and so, nearly
                 // always, are the later stages' (their plans are not formed)
@@ -569,13 +569,13 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
         launch_trajectory_rk2(m_Opt->domain, vc, sigma, ht, X, m_Opt->stream);
     }
     if (capturing) {
-        m_D[w] = kNoBound;  // and no plan, which eager calls may hold with its bound
+        m_Bound[w] = PlanBound{kNoBound, 0.0f};  // and no plan, which eager calls may hold with its bound
         m_Valid[w] = true;
         return 0;
     }
     // bytes: X read (12) + packed plan written (12) per point
     KernelScope k(m_Opt->prof, "gather_plan", 24.0 * nl);
-    m_D[w] = launch_make_plan(g, X, P, m_PlanMax.get(), m_Opt->stream);
+    m_Bound[w] = launch_make_plan(g, X, P, m_PlanWords.get(), m_Opt->stream);
     m_Valid[w] = true;
     return 0;
 }
@@ -583,7 +583,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
 TrajectoryPlan SemiLagrangian::Plan(const std::string& flag) const {
     const int w = Which(flag);
     CLR_REQUIRE(m_Valid[w], kErrState, "trajectory '" + flag + "' has not been computed");
-    return TrajectoryPlan{m_P[w].get(), m_X[w].get(), m_D[w]};
+    return TrajectoryPlan{m_P[w].get(), m_X[w].get(), m_Bound[w]};
 }
 
 bool SemiLagrangian::HasTrajectory(const std::string& flag) const { return m_Valid[Which(flag)]; }

@@ -351,7 +351,7 @@ class SemiLagrangian {
     // LDS-staged kernels where plan_gather_lds says so, else the direct kernels.
     claire_amd::TrajectoryPlan Plan(const std::string& flag) const;
     bool HasTrajectory(const std::string& flag) const;
-    int DisplacementBound(const std::string& flag) const { return m_D[Which(flag)]; }
+    int DisplacementBound(const std::string& flag) const { return m_Bound[Which(flag)].d; }
 
   private:
     int Which(const std::string& flag) const;
@@ -365,14 +365,14 @@ class SemiLagrangian {
     // updates an operand in place)
     DeviceArray<float> m_F, m_F2;
     DeviceArray<float> m_Tmp;  // in-place interpolation (the reference's ghost copy), kept between calls
-    PinnedArray<int> m_PlanMax;  // the plan kernels' block maxima (displacement bounds)
+    PinnedArray<int> m_PlanWords;  // what the plan kernels' blocks found
     // What SetVelocity found, for the characteristic scheme m_PredOrder (0: not
     // known); m_PredInPlan while m_P[0] still holds the predictor's plan.
     int m_PredOrder = 0;
-    int m_PredBound[2] = {0, 0};
+    claire_amd::PlanBound m_PredBound[2] = {};
     bool m_PredInPlan = false;
     bool m_Valid[2] = {false, false};
-    int m_D[2] = {0, 0};
+    claire_amd::PlanBound m_Bound[2] = {};
 };
 
 class CLAIRE {

@@ -298,12 +298,13 @@ __global__ __launch_bounds__(kLThreads) __attribute__((amdgpu_waves_per_eu(LdsGe
                 for (int k = 0; k < PTS; ++k) {
                     const float* p = (b < 3) ? reinterpret_cast<const float*>(ldsb + base[k][a]) + b * G::PITCH
                                              : reinterpret_cast<const float*>(ldsb + base3[k][a]);
-                    const float r = w3[k][0] * p[0] + w3[k][1] * p[1] + w3[k][2] * p[2] + w3[k][3] * p[3];
-                    sa[k] += w2[k][b] * r;
+                    // spelled out: left to the compiler, one row of the second point
+                    // of the bound-4 kernel was summed in another order
+                    sa[k] = fmaf(w2[k][b], row_sum(w3[k], p[0], p[1], p[2], p[3]), sa[k]);
                 }
             }
 #pragma unroll
-            for (int k = 0; k < PTS; ++k) v[k] += w1[k][a] * sa[k];
+            for (int k = 0; k < PTS; ++k) v[k] = fmaf(w1[k][a], sa[k], v[k]);
         }
         {
             const uint32_t pb = static_cast<uint32_t>(x1) * plane4;
@@ -1200,14 +1201,30 @@ void check_lds_dims(const GatherDims& g) {
 // and 145 : 360.  Three fields: 64³ 13.7 : 13.7 and 18.6 : 25.1; 96³ 27.2 : 36.8
 // and 34.7 : 58.2; 256³ 271 : 392.
 constexpr int64_t kFarPoints = int64_t(1) << 19;
+// Share of far-apart points (PlanBound::spread) up to which they are the faster
+// ones, by the kernel they replace: one that a bound of 4 cells suffices for, or
+// the direct one.  In µs against that kernel, scalar and three fields, for smooth
+// fields of up to so many cells and for noise:
+//   bound 4    96³  3.5 smooth (spread 0.03) 14.4 : 15.5  28 : 37
+//             128³  the same (0.02) 21.6 : 23.7  46 : 60, noise 2.8 36 : 31  100 : 88
+//             256³  the same (0.00) 98 : 144  291 : 401, (above 0.05) 272 : 206  754 : 614
+//   above 4    96³  9 smooth (0.68) 29.3 : 23.5  62 : 62
+//             128³  9 smooth (0.65) 40.7 : 47.2  114 : 129, 20 smooth (0.96) 79 : 58  213 : 166
+//             256³  9 smooth (0.38) 204 : 288  497 : 856, 20 smooth (0.88) 453 : 394  1064 : 1218
+//                   noise 5 (0.66) 624 : 767  1925 : 2458, 30 (1.00) 2013 : 1794  8340 : 5022
+constexpr float kMostSpread[2] = {0.05f, 0.65f};
+
+bool centred_windows(const GatherDims& g, PlanBound b, int nz) {
+    return g.nl * nz >= kFarPoints && b.spread <= kMostSpread[b.d > kNearBound];
+}
 
 template <class Epi>
-void dispatch(int dbound, const GatherDims& g, const uint32_t* P, const float* f, int64_t fzstride, int nz,
+void dispatch(PlanBound bound, const GatherDims& g, const uint32_t* P, const float* f, int64_t fzstride, int nz,
               const Epi& epi, hipStream_t st) {
     check_lds_dims(g);
-    CLR_REQUIRE(plan_gather_lds(g, dbound, nz), kErrInvalidArgument, "displacement bound too large for the LDS gather");
-    if (dbound > 2) {
-        if (g.nl * nz >= kFarPoints) return launch_lds<kPtsPlan>(g, P, f, fzstride, nz, epi, st);
+    CLR_REQUIRE(plan_gather_lds(g, bound, nz), kErrInvalidArgument, "displacement bound too large for the LDS gather");
+    if (bound.d > 2) {
+        if (centred_windows(g, bound, nz)) return launch_lds<kPtsPlan>(g, P, f, fzstride, nz, epi, st);
         return launch_lds<-4>(g, P, f, fzstride, nz, epi, st);
     }
     // The pair layout (two blocks per CU) is faster than the one-value layout
@@ -1225,13 +1242,13 @@ void dispatch(int dbound, const GatherDims& g, const uint32_t* P, const float* f
         launch_lds<-2>(g, P, f, fzstride, nz, epi, st);
 }
 
-bool use_lds(const TrajectoryPlan& tp, const GatherDims& g, int nz) { return plan_gather_lds(g, tp.dbound, nz); }
+bool use_lds(const TrajectoryPlan& tp, const GatherDims& g, int nz) { return plan_gather_lds(g, tp.bound, nz); }
 
 }  // namespace
 
-bool plan_gather_lds(const GatherDims& g, int dbound, int nz) {
-    if (dbound < 0 || dbound > kPlanMaxN) return false;  // no plan: a point is not finite
-    return dbound <= kNearBound || g.nl * nz >= kFarPoints;
+bool plan_gather_lds(const GatherDims& g, PlanBound b, int nz) {
+    if (b.d < 0 || b.d > kPlanMaxN) return false;  // no plan: a point is not finite
+    return b.d <= kNearBound || centred_windows(g, b, nz);
 }
 
 void launch_points_gather(const GatherDims& g, const float* f, const float* X, float* out, hipStream_t st) {
@@ -1252,40 +1269,40 @@ void launch_plan_gather(const TrajectoryPlan& tp, const GatherDims& g, const flo
     for (int d = 2; d < nf; ++d)
         CLR_REQUIRE(f[d] - f[d - 1] == fz && out[d] - out[d - 1] == oz, kErrInvalidArgument,
                     "vector gather needs equally spaced components");
-    dispatch(tp.dbound, g, tp.P, f[0], fz, nf, EpiPlain{out[0], oz}, st);
+    dispatch(tp.bound, g, tp.P, f[0], fz, nf, EpiPlain{out[0], oz}, st);
 }
 
 void launch_plan_inc_state_step(const TrajectoryPlan& tp, const GatherDims& g, const float* mt, const float* sj,
                                 float* out, int negate, hipStream_t st) {
     if (!use_lds(tp, g, 1)) return launch_direct_inc_state_step(g, tp.X, mt, sj, out, negate, st);
     CLR_REQUIRE(mt != out, kErrInvalidArgument, "semi-Lagrangian step cannot run in place");
-    dispatch(tp.dbound, g, tp.P, mt, 0, 1, EpiIncStep{sj, out, negate ? -1.0f : 1.0f}, st);
+    dispatch(tp.bound, g, tp.P, mt, 0, 1, EpiIncStep{sj, out, negate ? -1.0f : 1.0f}, st);
 }
 
 void launch_plan_adjoint_step(const TrajectoryPlan& tp, const GatherDims& g, const float* C, const float* lam,
                               float* out, hipStream_t st) {
     if (!use_lds(tp, g, 1)) return launch_direct_adjoint_step(g, tp.X, C, lam, out, st);
     CLR_REQUIRE(lam != out, kErrInvalidArgument, "semi-Lagrangian step cannot run in place");
-    dispatch(tp.dbound, g, tp.P, lam, 0, 1, EpiAdjStep{C, out}, st);
+    dispatch(tp.bound, g, tp.P, lam, 0, 1, EpiAdjStep{C, out}, st);
 }
 
 void launch_plan_adjoint_coeff(const TrajectoryPlan& tp, const GatherDims& g, const float* divv, float ht, float alpha,
                                float* C, hipStream_t st) {
     if (!use_lds(tp, g, 1)) return launch_adjoint_coeff(g, tp.X, divv, ht, alpha, C, st);
     CLR_REQUIRE(divv != C, kErrInvalidArgument, "coefficient cannot overwrite ∇·v");
-    dispatch(tp.dbound, g, tp.P, divv, 0, 1, EpiAdjCoeff{divv, C, ht, alpha}, st);
+    dispatch(tp.bound, g, tp.P, divv, 0, 1, EpiAdjCoeff{divv, C, ht, alpha}, st);
 }
 
-void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, int dbound, const float* const v[3], float sigma,
+void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, PlanBound bound, const float* const v[3], float sigma,
                                    float ht, float* X, hipStream_t st) {
     const GatherDims g = gather_dims(d);
     const int64_t vz = v[1] - v[0];
     CLR_REQUIRE(v[2] - v[1] == vz && vz == g.nl, kErrInvalidArgument, "velocity components must be contiguous");
-    EpiTrajRk2 e{v[0], X, g.nl, d.hx[0], d.hx[1], d.hx[2], sigma * (0.5f * ht), dbound > kNearBound, 0};
-    dispatch(dbound, g, P, v[0], vz, 3, e, st);
+    EpiTrajRk2 e{v[0], X, g.nl, d.hx[0], d.hx[1], d.hx[2], sigma * (0.5f * ht), bound.d > kNearBound, 0};
+    dispatch(bound, g, P, v[0], vz, 3, e, st);
 }
 
-void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, int dbound, const float* const v[3],
+void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, PlanBound bound, const float* const v[3],
                                float sigma, float ht, const float* Fin, float* Fout, float* X, hipStream_t st) {
     const GatherDims g = gather_dims(d);
     const int64_t vz = v[1] - v[0];
@@ -1299,16 +1316,16 @@ void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, int 
     const double s6 = static_cast<double>(sigma) * (static_cast<double>(ht) / 6.0);
     switch (stage) {
         case 1: {
-            EpiTrajRk4<1> e{v[0], X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * hthalf, s6, dbound > kNearBound, 0};
-            return dispatch(dbound, g, P, v[0], vz, 3, e, st);
+            EpiTrajRk4<1> e{v[0], X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * hthalf, s6, bound.d > kNearBound, 0};
+            return dispatch(bound, g, P, v[0], vz, 3, e, st);
         }
         case 2: {
             EpiTrajRk4<2> e{Fin, X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * ht, s6, false, 0};
-            return dispatch(dbound, g, P, v[0], vz, 3, e, st);
+            return dispatch(bound, g, P, v[0], vz, 3, e, st);
         }
         case 3: {
             EpiTrajRk4<3> e{Fin, X, X, g.nl, hx[0], hx[1], hx[2], 0.0f, s6, false, 0};  // no second output
-            return dispatch(dbound, g, P, v[0], vz, 3, e, st);
+            return dispatch(bound, g, P, v[0], vz, 3, e, st);
         }
         default:
             throw Error(kErrInvalidArgument, "RK4 stage must be 1, 2 or 3");

@@ -192,39 +192,59 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk4(GatherDims g, HH hh, Rk4P
     }
 }
 
-// Block maxima of K values into bmax[k·kPlanBlocks + blockIdx.x].
+// What a block found, in one word of host memory per direction: the largest
+// displacement bound above a sum of `low`, which is the same for a wave's lanes
+// (the host reads lines that the device has just written, which costs it more than
+// the kernel's whole fold).  Points per block stay below 2^20.
+constexpr int kLowBits = 20, kTopBound = 2047;
+static_assert(kPlanMaxN < kTopBound, "a bound must fit above the sum");
+
 template <int K>
-__device__ __forceinline__ void block_max_to(int (&v)[K], int* bmax) {
-    __shared__ int sh[K][kThreads / 64];
+__device__ __forceinline__ void block_words_to(int (&need)[K], const int (&low)[K], int* words) {
+    __shared__ int sh[2 * K][kThreads / 64];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v[k] = max(v[k], __shfl_xor(v[k], o, 64));
-        if ((threadIdx.x & 63) == 0) sh[k][threadIdx.x >> 6] = v[k];
+        for (int o = 32; o > 0; o >>= 1) need[k] = max(need[k], __shfl_xor(need[k], o, 64));
+        if ((threadIdx.x & 63) == 0) {
+            sh[2 * k][threadIdx.x >> 6] = min(need[k], kTopBound);
+            sh[2 * k + 1][threadIdx.x >> 6] = low[k];
+        }
     }
     __syncthreads();
     if (threadIdx.x < K) {
-        const int* m = sh[threadIdx.x];
-        bmax[threadIdx.x * kPlanBlocks + blockIdx.x] = max(max(m[0], m[1]), max(m[2], m[3]));
+        const int* m = sh[2 * threadIdx.x];
+        const int* c = sh[2 * threadIdx.x + 1];
+        words[threadIdx.x * kPlanBlocks + blockIdx.x] =
+            max(max(m[0], m[1]), max(m[2], m[3])) << kLowBits | (c[0] + c[1] + c[2] + c[3]);
     }
 }
 
-// Encodes the three axes of foot point q at grid index idx; returns the
-// displacement bound this point needs (kNoBound when not encodable).
+// Lanes of the wave whose stencil offsets o and those of the lane 32 away (half a
+// wave of points is as wide as a gather tile) are kFarApart cells or more apart,
+// all axes together.  An axis counts modulo 256 cells: enough for a share.
+__device__ __forceinline__ int spread_lanes(const int o[3]) {
+    constexpr unsigned kFarApart = 6;
+    const unsigned w = ((o[0] + 128) & 255) | ((o[1] + 128) & 255) << 8 | ((o[2] + 128) & 255) << 16;
+    return __popcll(__ballot(__builtin_amdgcn_sad_u8(w, __shfl_xor(w, 32, 64), 0u) >= kFarApart));
+}
+
+// Encodes the three axes of foot point q at grid index idx, stencil offsets o;
+// returns the displacement bound this point needs (kNoBound when not encodable).
 __device__ __forceinline__ int encode_point(const GatherDims& g, const HH& hh, const float q[3], const int idx[3],
-                                            PlanPt& pt) {
+                                            PlanPt& pt, int o[3]) {
     const int n[3] = {g.n1, g.n2, g.n3};
     int need = 0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         const float u = index_coord(q[a], n[a], hh.h[a]);
-        int lo = 0;
-        if (!plan_encode(u, idx[a], n[a], pt.w[a], lo)) {
+        o[a] = 0;
+        if (!plan_encode(u, idx[a], n[a], pt.w[a], o[a])) {
             need = kNoBound;
             pt.w[a] = 0u;  // t = 1, o = 0: never read
             continue;
         }
-        need = max(need, max(-lo - 1, lo + 1));
+        need = max(need, max(-o[a] - 1, o[a] + 1));
     }
     return need;
 }
@@ -235,18 +255,18 @@ __device__ __forceinline__ int encode_point(const GatherDims& g, const HH& hh, c
 // coordinates) set D to kNoBound, which routes every gather along this
 // trajectory to the direct kernels on the raw foot points.
 //
-// Each block writes its maximum into its own word of a host-resident array,
-// which the host reduces after the wait that it needs anyway: no word to clear
+// Each block writes what it found into its own word of a host-resident array,
+// which the host folds after the wait that it needs anyway: no word to clear
 // before the launch and no copy after it.  One word for all blocks made the
 // kernels wait for up to 2048 atomics on one address.  Measured with the
 // division-free x/2π (gather_device.hpp): set velocity + both trajectories +
 // one gather at 64³ 281 -> 188 µs, 96³ 391 -> 262, 128³ 462 -> 343, 256³
 // 1703 -> 1627, outputs identical.
-static_assert(kPlanBlocks >= 1 && kThreads == 256, "block_max_to folds four waves");
+static_assert(kPlanBlocks >= 1 && kThreads == 256, "block_words_to folds four waves");
 
 __global__ __launch_bounds__(kThreads) void k_make_plan(GatherDims g, HH hh, const float* __restrict__ X,
-                                                        PlanPt* __restrict__ P, int* __restrict__ bmax) {
-    int need[1] = {0};
+                                                        PlanPt* __restrict__ P, int* __restrict__ words) {
+    int need[1] = {0}, count[1] = {0}, o[3];
     const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
     const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     GridWalk gw(g, i0, stride);
@@ -254,10 +274,11 @@ __global__ __launch_bounds__(kThreads) void k_make_plan(GatherDims g, HH hh, con
         float q[3];
         load_point(X, g.nl, i, q);
         PlanPt pt;
-        need[0] = max(need[0], encode_point(g, hh, q, gw.idx, pt));
+        need[0] = max(need[0], encode_point(g, hh, q, gw.idx, pt, o));
+        count[0] += spread_lanes(o);
         P[i] = pt;
     }
-    block_max_to(need, bmax);
+    block_words_to(need, count, words);
 }
 
 // Plan of the Euler predictor X̃ = (x − σ·ht·v)/2π (bounded grid, like
@@ -273,8 +294,9 @@ __global__ __launch_bounds__(kThreads) void k_make_plan(GatherDims g, HH hh, con
 // 342 to 285 at 128³, 1602 to 1451 at 256³ and 12.5 to 11.5 ms at 512³.
 template <bool SETV>
 __global__ __launch_bounds__(kThreads) void k_predictor_plan(GatherDims g, HH hh, TrajParams tp, P3 v, float* vout,
-                                                             PlanPt* __restrict__ P, int* __restrict__ bmax) {
-    int need[3] = {0, 0, 0};
+                                                             PlanPt* __restrict__ P, int* __restrict__ words) {
+    int need[2] = {0, 0}, count = 0, o[3];
+    bool nonzero = false;
     const int64_t stride = static_cast<int64_t>(gridDim.x) * kThreads;
     const int64_t i0 = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     GridWalk gw(g, i0, stride);
@@ -296,19 +318,23 @@ __global__ __launch_bounds__(kThreads) void k_predictor_plan(GatherDims g, HH hh
             q[d] = euler_predictor(tp.hx[d], gw.idx[d], tp.sht, vd[d]);
             if constexpr (SETV) {
                 r[d] = euler_predictor(tp.hx[d], gw.idx[d], -tp.sht, vd[d]);
-                need[2] |= fabsf(vd[d]) > 0.0f;
+                nonzero = nonzero || fabsf(vd[d]) > 0.0f;
                 if (vout) vout[d * g.nl + i] = vd[d];
             }
         }
         PlanPt pt;
-        const int a = encode_point(g, hh, q, gw.idx, pt);
+        const int a = encode_point(g, hh, q, gw.idx, pt, o);
         P[i] = pt;
         if constexpr (SETV) {
+            count += spread_lanes(o);
             need[0] = max(need[0], a);
-            need[1] = max(need[1], encode_point(g, hh, r, gw.idx, pt));
+            need[1] = max(need[1], encode_point(g, hh, r, gw.idx, pt, o));
         }
     }
-    if constexpr (SETV) block_max_to(need, bmax);
+    if constexpr (SETV) {
+        const int low[2] = {count, __ballot(nonzero) != 0};
+        block_words_to(need, low, words);
+    }
 }
 
 // Points given per component, interleaved: 3 floats per point.
@@ -449,34 +475,55 @@ void launch_trajectory_rk4_stage(int stage, const Dims& d, const float* const v[
 }
 
 namespace {
-// The bound of a plan launch of nb blocks, after waiting for the stream.
-int plan_bound(const int* bmax, int nb, hipStream_t st) {
-    check_launches();  // a launch that failed wrote no maxima
+// The blocks' words of one direction folded: the largest bound, and the sum.
+struct PlanWords {
+    int d = 0;
+    int64_t sum = 0;
+    PlanWords(const int* words, int nb) {
+        for (int i = 0; i < nb; ++i) {
+            d = std::max(d, words[i] >> kLowBits);
+            sum += words[i] & ((1 << kLowBits) - 1);
+        }
+        if (d == kTopBound) d = kNoBound;
+    }
+};
+
+void wait_for_words(hipStream_t st) {
+    check_launches();  // a launch that failed wrote none
     CLR_HIP_CHECK(hipStreamSynchronize(st));
-    return *std::max_element(bmax, bmax + nb);
+}
+
+int plan_blocks(const GatherDims& g) {
+    CLR_REQUIRE(g.nl / kPlanBlocks < (1 << kLowBits) - kThreads, kErrInvalidArgument, "grid too large for a plan");
+    return std::min(nblocks_for(g.nl), kPlanBlocks);
 }
 }  // namespace
 
-int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* bmax, hipStream_t st) {
+PlanBound launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* words, hipStream_t st) {
     require_plan_size(g);
-    const int nb = std::min(nblocks_for(g.nl), kPlanBlocks);
+    const int nb = plan_blocks(g);
     hipLaunchKernelGGL(k_make_plan, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g), X, reinterpret_cast<PlanPt*>(P),
-                       bmax);
-    return plan_bound(bmax, nb, st);
+                       words);
+    wait_for_words(st);
+    const PlanWords w(words, nb);
+    return PlanBound{w.d, static_cast<float>(w.sum) / static_cast<float>(g.nl)};
 }
 
-VelocityBounds launch_set_velocity(const Dims& d, const float* v, float* vout, float ht, uint32_t* P, int* bmax,
+VelocityBounds launch_set_velocity(const Dims& d, const float* v, float* vout, float ht, uint32_t* P, int* words,
                                    hipStream_t st) {
     const GatherDims g = gather_dims(d);
     require_plan_size(g);
     P3 p{{v, v + g.nl, v + 2 * g.nl}, {nullptr, nullptr, nullptr}};
-    const int nb = std::min(nblocks_for(g.nl), kPlanBlocks);
+    const int nb = plan_blocks(g);
     hipLaunchKernelGGL(k_predictor_plan<true>, dim3(nb), dim3(kThreads), 0, st, g, make_hh(g),
-                       traj_params(d, 1.0f, ht), p, v == vout ? nullptr : vout, reinterpret_cast<PlanPt*>(P), bmax);
+                       traj_params(d, 1.0f, ht), p, v == vout ? nullptr : vout, reinterpret_cast<PlanPt*>(P), words);
+    wait_for_words(st);
+    const PlanWords w0(words, nb), w1(words + kPlanBlocks, nb);
+    const float spread = static_cast<float>(w0.sum) / static_cast<float>(g.nl);
     VelocityBounds b;
-    b.dbound[0] = plan_bound(bmax, nb, st);
-    b.dbound[1] = *std::max_element(bmax + kPlanBlocks, bmax + kPlanBlocks + nb);
-    b.zero = *std::max_element(bmax + 2 * kPlanBlocks, bmax + 2 * kPlanBlocks + nb) == 0;
+    b.bound[0] = PlanBound{w0.d, spread};
+    b.bound[1] = PlanBound{w1.d, spread};
+    b.zero = w1.sum == 0;
     return b;
 }
 

@@ -108,11 +108,17 @@ void launch_trajectory_rk4_stage(int stage, const Dims& d, const float* const v[
 // the first stencil node from the point (layout in gather_device.hpp).
 // Returns the per-axis stencil displacement bound D in cells (synchronizes
 // the stream); kNoBound when a foot point is not finite.  n <= 512 per axis.
-// `bmax`: 3·kPlanBlocks ints of pinned host memory that the device can write
-// (the blocks' bounds; one launch at a time may use them).
+// `words`: 2·kPlanBlocks ints of pinned host memory that the device can write
+// (what the blocks found; one launch at a time may use them).
 constexpr int kPlanBlocks = 2048;
 constexpr int kNoBound = 1 << 20;
-int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* bmax, hipStream_t st);
+// What the choice of a gather kernel goes by.
+struct PlanBound {
+    int d;         // displacement bound
+    float spread;  // share of the points displaced by six cells or more, all axes
+                   // together, against the point 32 further on in memory
+};
+PlanBound launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* words, hipStream_t st);
 // RK2 characteristic through the LDS-staged gather, in three passes:
 //   1. the packed plan of the Euler predictor X̃ = (x − σ·ht·v)/2π into P
 //      (launch_set_velocity or launch_predictor_plan);
@@ -122,19 +128,19 @@ int launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int* bmax
 // The foot points equal those of launch_trajectory_rk2 up to FMA contraction.
 //
 // First pass over a new velocity v (3·nl): copies it to vout (unless v ==
-// vout), writes the predictor's plan for σ = +1 and returns the displacement
-// bounds of the predictors for σ = +1 and −1 and whether v is zero
+// vout), writes the predictor's plan for σ = +1 and returns the bounds of the
+// predictors for σ = +1 and −1 (whose spread is the same) and whether v is zero
 // (synchronizes the stream).
 struct VelocityBounds {
-    int dbound[2];
+    PlanBound bound[2];
     bool zero;
 };
-VelocityBounds launch_set_velocity(const Dims& d, const float* v, float* vout, float ht, uint32_t* P, int* bmax,
+VelocityBounds launch_set_velocity(const Dims& d, const float* v, float* vout, float ht, uint32_t* P, int* words,
                                    hipStream_t st);
 // The predictor's plan alone.
 void launch_predictor_plan(const Dims& d, const float* const v[3], float sigma, float ht, uint32_t* P,
                            hipStream_t st);
-void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, int dbound, const float* const v[3], float sigma,
+void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, PlanBound bound, const float* const v[3], float sigma,
                                    float ht, float* X, hipStream_t st);
 // RK4 characteristic the same way: the plan of the first stage point
 // (x − σ·ht/2·v)/2π is the predictor's with ht/2; each stage gathers v along the
@@ -144,14 +150,13 @@ void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, int dbound,
 // writes f into Fout (Fin unused), stage 2 reads Fin and writes Fout (two
 // distinct buffers: no launch updates an operand in place, so a gather may
 // be repeated while its chunk length is tuned), stage 3 reads Fin.
-void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, int dbound, const float* const v[3],
+void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, PlanBound bound, const float* const v[3],
                                float sigma, float ht, const float* Fin, float* Fout, float* X, hipStream_t st);
 // Whether the gathers of nz fields along a plan of this bound run LDS-staged: the
-// bound is at most kNearBound, or the points are finite and many enough for
-// windows centred per block.  Beyond kNearBound the staged kernels round as the
-// direct ones do, so that this choice moves nothing.
+// bound is at most kNearBound, or the points are finite, many enough for windows
+// centred per block and close enough together for most to lie in them.
 constexpr int kNearBound = 4;
-bool plan_gather_lds(const GatherDims& g, int dbound, int nz);
+bool plan_gather_lds(const GatherDims& g, PlanBound bound, int nz);
 // Update coefficient per point: C = 1 + ht/2·(α·dX + α·(1 + ht·α·dX)·d)
 // with d = ∇·v, dX = d(X).  α = 1 on the adjoint trajectory gives the SL
 // adjoint update λ⁺ = C·λ(X_a); α = ±1 on the state trajectory gives the
@@ -160,15 +165,15 @@ void launch_adjoint_coeff(const GatherDims& g, const float* X, const float* divv
                           hipStream_t st);
 
 // A trajectory as the gathers see it: the packed plan, the raw foot points
-// (one component per field) and the plan's displacement bound.
+// (one component per field) and the plan's bound.
 struct TrajectoryPlan {
     const uint32_t* P;
     const float* X;
-    int dbound;
+    PlanBound bound;
 };
 
 // Gathers along a trajectory.  Vector fields are nf equally spaced component
-// pointers.  They run the LDS-staged kernels when dbound allows, else the
+// pointers.  They run the LDS-staged kernels where plan_gather_lds says so, else the
 // direct kernels on the raw foot points (which take the field from blockIdx.y:
 // at most kMaxGatherFields of them).
 //   gather:          out_d = f_d(X)

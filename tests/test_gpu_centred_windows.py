@@ -108,3 +108,47 @@ def test_points_at_infinity(oracle):
     X[bad] = 0.25
     want = oracle.interp(f, X, prec="f32")
     assert np.abs(got - want)[~bad].max() <= 2e-6 * np.abs(f).max()
+
+
+@pytest.mark.parametrize("order", [2, 4])
+@pytest.mark.parametrize("cells", [2.8, 3.9, 8.0])
+def test_displacements_of_noise(cells, order, oracle):
+    """Points too far apart for centred windows take the kernels without them, which
+    round as the others do."""
+    print(f"\n[gpu case] noise of {cells} cells, rk{order}", flush=True)
+    rng = np.random.default_rng(5)
+    v = _velocity((rng.random(SHAPE + (3,)) - 0.5) * 2 * cells)
+    f = synth.gaussian_blobs(SHAPE, count=12, seed=1)
+    c = Claire(SHAPE, nt=NT, rk_order=order)
+    try:
+        c.set_velocity(v)
+        X = c.trajectory(STATE)
+        got = c.interp_scalar(f, STATE), c.interp_vector(v, STATE)
+        points = c.interp_points(f, X)
+    finally:
+        c.close()
+    # 12 roundings a side of sums that are at most 1.25^3 of the largest value
+    assert np.abs(got[0] - oracle.interp(f, X, prec="f32")).max() <= 4e-6 * np.abs(f).max()
+    assert np.array_equal(points, got[0])
+    for a in range(3):
+        assert np.abs(got[1][a] - oracle.interp(v[a], X, prec="f32")).max() <= 4e-6 * np.abs(v).max()
+
+
+@pytest.mark.parametrize("cells", [3.5, 6.0])
+def test_bits_do_not_depend_on_the_kernel(cells):
+    """Few points (fixed windows or the direct kernel) against three fields at once
+    (centred windows) and raw points (direct kernel)."""
+    print(f"\n[gpu case] kernels agree at {cells} cells", flush=True)
+    shape = (48, 64, 64)
+    f = synth.gaussian_blobs(shape, count=12, seed=1) + 1.0
+    c = Claire(shape, nt=NT)
+    try:
+        v = synth.bandlimited_velocity(shape, kmax=3, cfl=1.0, nt=NT, seed=2)
+        h = np.array([2.0 * np.pi / n for n in shape], np.float32).reshape(3, 1, 1, 1)
+        c.set_velocity(v * np.float32(cells * NT) / np.abs(v / h).max())
+        want = c.interp_points(f, c.trajectory(STATE))
+        assert np.array_equal(c.interp_scalar(f, STATE), want)
+        for got in c.interp_vector(np.stack([f, f, f]), STATE):
+            assert np.array_equal(got, want)
+    finally:
+        c.close()
