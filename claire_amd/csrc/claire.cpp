@@ -284,14 +284,13 @@ int SpectralOps::SeriesFields(int n) const {
     return (n + groups - 1) / groups;
 }
 
-void SpectralOps::ReserveSeries(int n) {
-    m_SeriesSpec.resize(SeriesSpectra(n) * static_cast<size_t>(m_Opt->domain.nlc));
-}
-
 void SpectralOps::GradSeries(float* g, const float* f, int n) {
     const Dims& d = m_Opt->domain;
     const int per = SeriesFields(n);
-    ReserveSeries(n);
+    if (per > 1) {
+        AllocationsInCapture alloc;
+        m_SeriesSpec.resize(3 * static_cast<size_t>(per) * d.nlc);
+    }
     for (int j = 0; j < n; j += per)
         Gradients(g + 3 * j * d.nl, 3 * d.nl, d.nl, f + j * d.nl, d.nl, std::min(per, n - j),
                   per > 1 ? m_SeriesSpec.get() : m_Spec.get());
@@ -486,12 +485,11 @@ bool SemiLagrangian::Capturing() const {
     return m_Opt->stream && hipStreamIsCapturing(m_Opt->stream, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
 }
 
-void SemiLagrangian::Reserve() {
+void SemiLagrangian::Reserve(int w) {
     const size_t n = 3 * static_cast<size_t>(m_Opt->domain.nl);
-    for (int w = 0; w < 2; ++w) {
-        m_X[w].resize(n);
-        m_P[w].resize(n);
-    }
+    AllocationsInCapture alloc;
+    m_X[w].resize(n);
+    m_P[w].resize(n);
     if (m_Opt->rkorder == 4) {
         m_F.resize(n);
         m_F2.resize(n);
@@ -501,7 +499,7 @@ void SemiLagrangian::Reserve() {
 bool SemiLagrangian::SetVelocity(const float* v, VecField* dst) {
     ForgetVelocity();     // until the bounds are known
     m_Valid[0] = false;   // its plan is overwritten
-    Reserve();
+    m_P[0].resize(3 * static_cast<size_t>(m_Opt->domain.nl));
     // bytes: v read (12), copied (12) and the plan written (12) per point
     KernelScope k(m_Opt->prof, "gather_traj_rk2_plan", 36.0 * m_Opt->domain.nl);
     const VelocityBounds b = launch_set_velocity(m_Opt->domain, v, dst->m_X1, PredictorStep(), m_P[0].get(),
@@ -523,7 +521,7 @@ int SemiLagrangian::ComputeTrajectory(const VecField* v, const std::string& flag
         SetVelocity(v->m_X1, &same);
     }
     const int64_t nl = m_Opt->domain.nl;
-    Reserve();
+    Reserve(w);
     float* const X = m_X[w].get();
     uint32_t* const P = m_P[w].get();
     const GatherDims g = gather_dims(m_Opt->domain);
@@ -706,7 +704,6 @@ CLAIRE::CLAIRE(const RegOpt& opt) : m_Opt(opt) {
     m_Scalar.resize(nl);
     m_AdjCoeff.resize(nl);
     m_VtX.resize(3 * nl);
-    m_Spectral->ReserveSeries(m_Opt.nt + 1);
 }
 
 CLAIRE::~CLAIRE() {
@@ -850,6 +847,10 @@ int CLAIRE::SolveStateEquation() {
             // ht·dX)·d), d = ∇·v, dX = d(X_s): the α = −1 form of the
             // coefficient on the state trajectory (src/CLAIRE.cpp:2813-2835)
             EnsureDivergence();
+            {
+                AllocationsInCapture alloc;
+                m_StateCoeff.resize(static_cast<size_t>(nl));
+            }
             KernelScope k(m_Opt.prof, "gather_state_coeff", 24.0 * nl);
             launch_plan_adjoint_coeff(tp, g, m_Scalar.get(), m_Opt.GetTimeStepSize(), -1.0f, m_StateCoeff.get(),
                                       m_Opt.stream);
@@ -957,7 +958,6 @@ int CLAIRE::SetRKOrder(int order) {
 int CLAIRE::SetPDEType(int type) {
     CLR_REQUIRE(type == 0 || type == 1, kErrInvalidArgument, "pde type must be 0 (continuity) or 1 (transport)");
     if (type != m_Opt.pdetype) {
-        if (type == 0) m_StateCoeff.resize(static_cast<size_t>(m_Opt.domain.nl));
         m_Opt.pdetype = type;
         DropTrajectories();
         m_StateValid = m_GradMValid = m_GradMXValid = m_HalfValid = false;

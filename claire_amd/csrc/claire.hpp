@@ -66,6 +66,19 @@ class DeviceArray {
     size_t n_ = 0;
 };
 
+// While it lives, this thread may allocate device memory although a stream of it is
+// being captured (an allocation is no stream operation).
+class AllocationsInCapture {
+  public:
+    AllocationsInCapture() { (void)hipThreadExchangeStreamCaptureMode(&m_); }
+    ~AllocationsInCapture() { (void)hipThreadExchangeStreamCaptureMode(&m_); }
+    AllocationsInCapture(const AllocationsInCapture&) = delete;
+    AllocationsInCapture& operator=(const AllocationsInCapture&) = delete;
+
+  private:
+    hipStreamCaptureMode m_ = hipStreamCaptureModeRelaxed;
+};
+
 // Owning allocation of pinned host memory that kernels write to and the host
 // reads after a stream synchronization.
 template <class T>
@@ -246,7 +259,6 @@ class SpectralOps {
     // 2322 -> 2257 at 192³, 4.34 ms either way at 256³ (one field per launch).
     void GradSeries(float* g, const float* f, int n);
     static constexpr int64_t kSeriesPoints = int64_t(1) << 24;
-    void ReserveSeries(int n);
     // half spectra GradSeries keeps beside the three of the other operators
     size_t SeriesSpectra(int n) const { return SeriesFields(n) > 1 ? 3 * static_cast<size_t>(SeriesFields(n)) : 0; }
     void Div(float* d, const float* const v[3]);
@@ -266,7 +278,7 @@ class SpectralOps {
     void Gradients(float* g, int64_t gs, int64_t gc, const float* f, int64_t fs, int n, c32* spec);
     int SeriesFields(int n) const;
     DeviceArray<c32> m_Spec;        // three half spectra
-    DeviceArray<c32> m_SeriesSpec;  // GradSeries
+    DeviceArray<c32> m_SeriesSpec;  // GradSeries, allocated on its first call
     DeviceArray<double> m_NormPartial;  // block sums of Norm3, allocated on its first call
 };
 
@@ -355,7 +367,7 @@ class SemiLagrangian {
 
   private:
     int Which(const std::string& flag) const;
-    void Reserve();  // the buffers of both trajectories (none can be allocated in a capture)
+    void Reserve(int w);  // the buffers that forming trajectory w takes
     const RegOpt* m_Opt;
     float PredictorStep() const { return (m_Opt->rkorder == 4 ? 0.5f : 1.0f) * m_Opt->GetTimeStepSize(); }
     DeviceArray<float> m_X[2];  // foot points, one component per field
