@@ -724,15 +724,14 @@ int CLAIRE::SetMatVecGraphs(bool on) {
 }
 
 size_t CLAIRE::DeviceBytes() const {
-    const size_t nl = static_cast<size_t>(m_Opt.domain.nl), nt = static_cast<size_t>(m_Opt.nt);
-    const size_t floats = 5 * 3 * nl + 2 * nl + (nt + 1) * nl + nl + 3 * nl + 4 * nl + (nt + 1) * 3 * nl +
-                          nt * 3 * nl + nt * nl + nt * nl + nl + 2 * 3 * nl;
-    const size_t halves = m_Opt.precision == 1 ? (2 * nt + 1) * 3 * nl : 0;
-    const size_t scales = m_Opt.precision == 1 ? (2 * nt + 1) * 3 * static_cast<size_t>(bfp16_blocks(nl)) : 0;
-    const size_t rk4 = m_Opt.rkorder == 4 ? 6 * nl : 0;  // the two RK4 stage sums
-    const size_t cont = m_Opt.pdetype == 0 ? nl : 0;      // continuity-equation coefficient
-    const size_t rk2 = m_Opt.pdesolver == 0 ? 6 * nl : 0;  // RK2 integrator work
-    return (floats + rk4 + cont + rk2 + scales) * 4 + halves * 2 + (3 + m_Spectral->SeriesSpectra(m_Opt.nt + 1)) * static_cast<size_t>(m_Opt.domain.nlc) * 8;
+    size_t n = m_Red->DeviceBytes() + m_Spectral->DeviceBytes() + m_SL->DeviceBytes();
+    for (const auto& v : {&m_VelocityField, &m_IncVelocityField, &m_BodyForce, &m_IncBodyForce, &m_WorkVecField1})
+        n += (*v)->DeviceBytes();
+    for (const auto* a : {&m_ReferenceImage, &m_State, &m_Adjoint, &m_IncState[0], &m_IncState[1], &m_IncAdjointT0,
+                          &m_GradM, &m_GradMX, &m_S, &m_Lam, &m_Scalar, &m_AdjCoeff, &m_StateCoeff, &m_Rk2Work,
+                          &m_VtX, &m_GradMScale, &m_GradMXScale})
+        n += a->bytes();
+    return n + m_GradM16.bytes() + m_GradMX16.bytes();
 }
 
 void CLAIRE::RequireVelocity() const { CLR_REQUIRE(m_HaveVelocity, kErrState, "velocity field not set"); }

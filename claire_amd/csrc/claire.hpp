@@ -60,6 +60,7 @@ class DeviceArray {
     }
     T* get() const { return p_; }
     size_t size() const { return n_; }
+    size_t bytes() const { return n_ * sizeof(T); }
 
   private:
     T* p_ = nullptr;
@@ -212,6 +213,7 @@ class Reducer {
     // Device address of the result slots (read by kernels that consume the
     // products without a host round trip).
     const double* Slots() const { return m_Result.get(); }
+    size_t DeviceBytes() const { return m_Partial.bytes() + m_Result.bytes(); }
 
   private:
     const RegOpt* m_Opt;
@@ -237,6 +239,7 @@ class VecField {
     int Scale(ScalarType a);
     int AXPY(ScalarType a, const VecField* x);
     int WAXPY(ScalarType a, const VecField* x, const VecField* y);
+    size_t DeviceBytes() const { return m_Storage.bytes(); }
 
   private:
     const RegOpt* m_Opt;
@@ -259,8 +262,6 @@ class SpectralOps {
     // 2322 -> 2257 at 192³, 4.34 ms either way at 256³ (one field per launch).
     void GradSeries(float* g, const float* f, int n);
     static constexpr int64_t kSeriesPoints = int64_t(1) << 24;
-    // half spectra GradSeries keeps beside the three of the other operators
-    size_t SeriesSpectra(int n) const { return SeriesFields(n) > 1 ? 3 * static_cast<size_t>(SeriesFields(n)) : 0; }
     void Div(float* d, const float* const v[3]);
     // out_d = alpha·F⁻¹(m(k)·F(in_d)) + beta·add_d, d = 0..2
     void Multiplier3(const claire_amd::SpecParams& sp, const float* const in[3], float* const out[3], float alpha,
@@ -271,6 +272,7 @@ class SpectralOps {
     // b ← b + F⁻¹[x̂] with the projection of sp.op (kOpProjStokes or
     // kOpProjRelaxed), in place on the three components.
     void Project(const claire_amd::SpecParams& sp, float* const b[3]);
+    size_t DeviceBytes() const { return m_Spec.bytes() + m_SeriesSpec.bytes() + m_NormPartial.bytes(); }
 
   private:
     const RegOpt* m_Opt;
@@ -363,6 +365,10 @@ class SemiLagrangian {
     // LDS-staged kernels where plan_gather_lds says so, else the direct kernels.
     claire_amd::TrajectoryPlan Plan(const std::string& flag) const;
     bool HasTrajectory(const std::string& flag) const;
+    size_t DeviceBytes() const {
+        return m_X[0].bytes() + m_X[1].bytes() + m_P[0].bytes() + m_P[1].bytes() + m_F.bytes() + m_F2.bytes() +
+               m_Tmp.bytes();
+    }
     int DisplacementBound(const std::string& flag) const { return m_Bound[Which(flag)].d; }
 
   private:

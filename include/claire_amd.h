@@ -197,7 +197,9 @@ int clr_apply_projection(clr_ctx* ctx, float* v);
  * reports the graphs currently held. */
 int clr_set_matvec_graphs(clr_ctx* ctx, int on);
 int clr_matvec_graph_count(clr_ctx* ctx, int* count);
-/* Device memory held by the context (bytes); no reference counterpart. */
+/* Device memory that the problem holds (bytes), work buffers that some calls
+ * allocate on first use among it, the solver's vectors (clr_solve_gn) not; no
+ * reference counterpart. */
 int clr_device_bytes(clr_ctx* ctx, size_t* bytes);
 
 /* CLAIREBase::SetControlVariable (src/CLAIREBase.cpp:393) --
