@@ -37,8 +37,12 @@ struct Axis {
 // x/2π as the float/double steps of the characteristic divide it
 // (src/SemiLagrangian.cpp:235-278): the product with 1/2π and one correction of
 // the quotient, three FP64 operations instead of a division's dozen.  Equal to
-// the division in double for every finite FP32 x (checked over all of them),
-// and 0, ±inf and NaN give what it gives.
+// the division for every double that over- or underflows nowhere on the way, FP32
+// values and the stage sums of RK4 among them: the product is less than one unit in
+// the last place off (1/2π, rounded to nearest, is 0.21 units off), its remainder is
+// exact, and one such correction then rounds to nearest (Markstein, IBM J. Res. Dev.
+// 34 (1990) 111).  ±0, ±inf and NaN give what the division gives, but for the sign
+// of −0.
 constexpr double kTwoPi = 2.0 * 3.14159265358979323846;
 __device__ __forceinline__ double over_2pi(double x) {
     constexpr double inv = 1.0 / kTwoPi;
