@@ -12,6 +12,7 @@ MAIN = r"""
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <initializer_list>
 #define __device__
 #define __forceinline__ inline
 %s
