@@ -65,14 +65,18 @@ __device__ __forceinline__ float index_coord(float q, int n, float hh) {
     return fmaf(wrap_q(q, hh), static_cast<float>(n), 3.0f);
 }
 
-// Euler predictor (x − s·v)/2π of one axis at grid index i.  The rounding is
-// spelled out because a plan's displacement bound and the plan itself come from
-// different kernels: left to the compiler, x − s·v and x + s·v of one kernel
-// shared their products and rounded differently from the plan's, and a point
-// within a rounding of a cell boundary then lay outside the window its bound
-// promised.
-__device__ __forceinline__ float euler_predictor(float hx, int i, float s, float v) {
+// Points of a characteristic on one axis from grid index i, over 2π: (x − s·v)/2π,
+// every point but RK4's last, which takes its step in double.  The roundings are
+// spelled out because the same point is formed by different kernels.  Left to the
+// compiler, the bound of a predictor's plan came from another rounding than the plan,
+// and a point within a rounding of a cell boundary lay outside the window that its
+// bound promised; and foot points depended on which kernels their displacement chose.
+__device__ __forceinline__ float foot_point(float hx, int i, float s, float v) {
     return static_cast<float>(over_2pi(static_cast<double>(fmaf(hx, static_cast<float>(i), -(s * v)))));
+}
+__device__ __forceinline__ float foot_point_rk4(float hx, int i, double s6, float f) {
+    const float x = hx * static_cast<float>(i);
+    return static_cast<float>(over_2pi(fma(-s6, static_cast<double>(f), static_cast<double>(x))));
 }
 
 // Grid index of the first stencil node before the periodic wrap: floor(u) − 4.
@@ -323,7 +327,7 @@ struct EpiAdjCoeff {
 // Corrector of the RK2 characteristic (src/SemiLagrangian.cpp:235-278) for
 // component z = blockIdx.y, gathered along the Euler predictor's plan:
 // X_z = (x_z − σ·ht/2·(v_z(X̃) + v_z(x)))/2π, stored per component (out +
-// z·zstride); aux is v_z at the point.  Same expressions as k_traj_rk2.
+// z·zstride); aux is v_z at the point.
 struct EpiTrajRk2 {
     static constexpr bool kRowFrom1 = true;
     static constexpr bool kHasAux = true;
@@ -334,7 +338,6 @@ struct EpiTrajRk2 {
     int64_t zstride;
     float hx0, hx1, hx2;  // grid spacings
     float shth;  // σ·ht/2
-    bool far;    // bound above kNearBound: x rounded first, the order of k_traj_rk2
     int z;
     float hz;  // spacing of axis z, set by select
     __device__ void select(int zz) {
@@ -348,10 +351,7 @@ struct EpiTrajRk2 {
     __device__ const float* auxp() const { return v; }
     __device__ float* outp() const { return out; }
     __device__ float apply_at(float vx, float vl, int i1, int i2, int i3) const {
-        const int idx = z == 0 ? i1 : (z == 1 ? i2 : i3);
-        const float i = static_cast<float>(idx), u = vx + vl;
-        const float t = far ? fmaf(-shth, u, hz * i) : fmaf(hz, i, -(shth * u));
-        return static_cast<float>(over_2pi(static_cast<double>(t)));
+        return foot_point(hz, z == 0 ? i1 : (z == 1 ? i2 : i3), shth, vx + vl);
     }
 };
 
@@ -376,7 +376,6 @@ struct EpiTrajRk4 {
     float hx0, hx1, hx2;  // grid spacings
     float step;  // σ·ht/2 (stage 1), σ·ht (stage 2)
     double s6;   // σ·(ht/6) (stage 3)
-    bool far;    // stage 1 as in EpiTrajRk2
     int z;
     float hz;  // spacing of axis z, set by select
     __device__ void select(int zz) {
@@ -393,14 +392,10 @@ struct EpiTrajRk4 {
     __device__ float* outp2() const { return f; }
     __device__ float apply_at(float vx, float av, int i1, int i2, int i3) const {
         const int idx = z == 0 ? i1 : (z == 1 ? i2 : i3);
-        const float i = static_cast<float>(idx);
-        if constexpr (STAGE < 3) {
-            const float t = STAGE == 1 && far ? fmaf(-step, vx, hz * i) : fmaf(hz, i, -(step * vx));
-            return static_cast<float>(over_2pi(static_cast<double>(t)));
-        } else {
-            const float x = hz * i, fs = av + vx;
-            return static_cast<float>(over_2pi(static_cast<double>(x) - s6 * static_cast<double>(fs)));
-        }
+        if constexpr (STAGE < 3)
+            return foot_point(hz, idx, step, vx);
+        else
+            return foot_point_rk4(hz, idx, s6, av + vx);
     }
     __device__ float apply2(float vx, float av) const {
         return static_cast<float>(static_cast<double>(av) + 2.0 * static_cast<double>(vx));

@@ -1298,7 +1298,7 @@ void launch_lds_traj_rk2_corrector(const Dims& d, const uint32_t* P, PlanBound b
     const GatherDims g = gather_dims(d);
     const int64_t vz = v[1] - v[0];
     CLR_REQUIRE(v[2] - v[1] == vz && vz == g.nl, kErrInvalidArgument, "velocity components must be contiguous");
-    EpiTrajRk2 e{v[0], X, g.nl, d.hx[0], d.hx[1], d.hx[2], sigma * (0.5f * ht), bound.d > kNearBound, 0};
+    EpiTrajRk2 e{v[0], X, g.nl, d.hx[0], d.hx[1], d.hx[2], sigma * (0.5f * ht), 0};
     dispatch(bound, g, P, v[0], vz, 3, e, st);
 }
 
@@ -1316,15 +1316,15 @@ void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, Plan
     const double s6 = static_cast<double>(sigma) * (static_cast<double>(ht) / 6.0);
     switch (stage) {
         case 1: {
-            EpiTrajRk4<1> e{v[0], X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * hthalf, s6, bound.d > kNearBound, 0};
+            EpiTrajRk4<1> e{v[0], X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * hthalf, s6, 0};
             return dispatch(bound, g, P, v[0], vz, 3, e, st);
         }
         case 2: {
-            EpiTrajRk4<2> e{Fin, X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * ht, s6, false, 0};
+            EpiTrajRk4<2> e{Fin, X, Fout, g.nl, hx[0], hx[1], hx[2], sigma * ht, s6, 0};
             return dispatch(bound, g, P, v[0], vz, 3, e, st);
         }
         case 3: {
-            EpiTrajRk4<3> e{Fin, X, X, g.nl, hx[0], hx[1], hx[2], 0.0f, s6, false, 0};  // no second output
+            EpiTrajRk4<3> e{Fin, X, X, g.nl, hx[0], hx[1], hx[2], 0.0f, s6, 0};  // no second output
             return dispatch(bound, g, P, v[0], vz, 3, e, st);
         }
         default:

@@ -108,24 +108,18 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk2(GatherDims g, HH hh, Traj
     if (i >= g.nl) return;
     int idx[3];
     grid_index(g, i, idx);
-    const float x[3] = {tp.hx[0] * static_cast<float>(idx[0]), tp.hx[1] * static_cast<float>(idx[1]),
-                        tp.hx[2] * static_cast<float>(idx[2])};
     float vl[3], q[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         vl[d] = v.in[d][i];
-        const float t = x[d] - tp.sht * vl[d];
-        q[d] = static_cast<float>(over_2pi(static_cast<double>(t)));
+        q[d] = foot_point(tp.hx[d], idx[d], tp.sht, vl[d]);
     }
     Stencil S;
     setup_stencil(q, g, hh.h, S);
     float vx[3];
     eval_stencil<3>(v.in, S, g, vx);
 #pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const float t = x[d] - tp.shth * (vx[d] + vl[d]);
-        X[d * g.nl + i] = static_cast<float>(over_2pi(static_cast<double>(t)));
-    }
+    for (int d = 0; d < 3; ++d) X[d * g.nl + i] = foot_point(tp.hx[d], idx[d], tp.shth, vx[d] + vl[d]);
 }
 
 // SemiLagrangian::ComputeTrajectoryRK4 (src/SemiLagrangian.cpp:297-459), in
@@ -145,28 +139,19 @@ struct Rk4Params {
     double s6;    // σ·(ht/6.0)
 };
 
-__device__ __forceinline__ void grid_point(const GatherDims& g, const float hx[3], int64_t i, float x[3]) {
-    int idx[3];
-    grid_index(g, i, idx);
-    x[0] = hx[0] * static_cast<float>(idx[0]);
-    x[1] = hx[1] * static_cast<float>(idx[1]);
-    x[2] = hx[2] * static_cast<float>(idx[2]);
-}
-
 template <int STAGE>
 __global__ __launch_bounds__(kThreads) void k_traj_rk4(GatherDims g, HH hh, Rk4Params tp, P3 v,
                                                        float* __restrict__ X, const float* Fin, float* Fout, int nblocks) {
     const int64_t i = point_index(nblocks);
     if (i >= g.nl) return;
-    float x[3];
-    grid_point(g, tp.hx, i, x);
+    int idx[3];
+    grid_index(g, i, idx);
     float vl[3], q[3];
     if constexpr (STAGE == 1) {
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
             vl[d] = v.in[d][i];
-            const float t = x[d] - tp.shth * vl[d];
-            q[d] = static_cast<float>(over_2pi(static_cast<double>(t)));
+            q[d] = foot_point(tp.hx[d], idx[d], tp.shth, vl[d]);
         }
     } else {
         load_point(X, g.nl, i, q);
@@ -179,15 +164,12 @@ __global__ __launch_bounds__(kThreads) void k_traj_rk4(GatherDims g, HH hh, Rk4P
     for (int d = 0; d < 3; ++d) {
         if constexpr (STAGE == 1) {
             Fout[d * g.nl + i] = static_cast<float>(static_cast<double>(vl[d]) + 2.0 * static_cast<double>(vx[d]));
-            const float t = x[d] - tp.shth * vx[d];
-            X[d * g.nl + i] = static_cast<float>(over_2pi(static_cast<double>(t)));
+            X[d * g.nl + i] = foot_point(tp.hx[d], idx[d], tp.shth, vx[d]);
         } else if constexpr (STAGE == 2) {
             Fout[d * g.nl + i] = static_cast<float>(static_cast<double>(Fin[d * g.nl + i]) + 2.0 * static_cast<double>(vx[d]));
-            const float t = x[d] - tp.sht * vx[d];
-            X[d * g.nl + i] = static_cast<float>(over_2pi(static_cast<double>(t)));
+            X[d * g.nl + i] = foot_point(tp.hx[d], idx[d], tp.sht, vx[d]);
         } else {
-            const float f = Fin[d * g.nl + i] + vx[d];
-            X[d * g.nl + i] = static_cast<float>(over_2pi(static_cast<double>(x[d]) - tp.s6 * static_cast<double>(f)));
+            X[d * g.nl + i] = foot_point_rk4(tp.hx[d], idx[d], tp.s6, Fin[d * g.nl + i] + vx[d]);
         }
     }
 }
@@ -315,9 +297,9 @@ __global__ __launch_bounds__(kThreads) void k_predictor_plan(GatherDims g, HH hh
             for (int d = 0; d < 3; ++d) vn[d] = v.in[d][i + stride];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            q[d] = euler_predictor(tp.hx[d], gw.idx[d], tp.sht, vd[d]);
+            q[d] = foot_point(tp.hx[d], gw.idx[d], tp.sht, vd[d]);
             if constexpr (SETV) {
-                r[d] = euler_predictor(tp.hx[d], gw.idx[d], -tp.sht, vd[d]);
+                r[d] = foot_point(tp.hx[d], gw.idx[d], -tp.sht, vd[d]);
                 nonzero = nonzero || fabsf(vd[d]) > 0.0f;
                 if (vout) vout[d * g.nl + i] = vd[d];
             }

@@ -125,7 +125,7 @@ PlanBound launch_make_plan(const GatherDims& g, const float* X, uint32_t* P, int
 //   2. v gathered along it with the corrector as epilogue,
 //      X = (x − σ·ht/2·(v(X̃) + v))/2π (launch_lds_traj_rk2_corrector);
 //   3. the plan of X into P (launch_make_plan, which returns its bound).
-// The foot points equal those of launch_trajectory_rk2 up to FMA contraction.
+// The foot points equal those of launch_trajectory_rk2.
 //
 // First pass over a new velocity v (3·nl): copies it to vout (unless v ==
 // vout), writes the predictor's plan for σ = +1 and returns the bounds of the

@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import claire_amd
-from claire_amd import ADJOINT, Claire, DeviceArray, synth
+from claire_amd import ADJOINT, STATE, Claire, DeviceArray, synth
 
 pytestmark = pytest.mark.gpu
 NT = 4
@@ -127,3 +127,30 @@ def test_replay_at_a_new_velocity(rk_order, graphs):
     finally:
         p.c.close()
         q.c.close()
+
+
+@pytest.mark.parametrize("rk_order", [2, 4])
+@pytest.mark.parametrize("cells", [1.5, 3.5, 7.0, 25.0])
+def test_foot_points_do_not_depend_on_the_kernel(cells, rk_order, graphs):
+    """In a capture the direct kernels form the trajectories, else those that suit
+    the displacement: fixed windows, centred ones or the direct kernels."""
+    print(f"\n[gpu case] foot points of {cells} cells rk{rk_order}", flush=True)
+    shape = (64, 96, 96)  # three fields have more than 2^19 points
+    h = np.array([2.0 * np.pi / n for n in shape], np.float32).reshape(3, 1, 1, 1)
+    v = synth.bandlimited_velocity(shape, kmax=4, cfl=1.0, nt=NT, seed=5)
+    v *= np.float32(cells * NT) / np.abs(v / h).max()
+    d, X = DeviceArray.from_host(v), DeviceArray(shape + (3,))
+    c = Claire(shape, nt=NT, rk_order=rk_order, stream=graphs.stream.value)
+    try:
+        for flag in (STATE, ADJOINT):
+            call = lambda: claire_amd._check(claire_amd.lib().clr_trajectory(c.ctx, flag, ctypes.c_void_p(X.ptr)))
+            c.set_velocity_device(d)
+            g = graphs.capture(call)
+            graphs.replay(g)
+            direct = X.download()
+            c.set_velocity_device(d)
+            call()
+            graphs.sync()
+            assert np.array_equal(X.download(), direct)
+    finally:
+        c.close()
