@@ -584,8 +584,6 @@ TrajectoryPlan SemiLagrangian::Plan(const std::string& flag) const {
     return TrajectoryPlan{m_P[w].get(), m_X[w].get(), m_Bound[w]};
 }
 
-bool SemiLagrangian::HasTrajectory(const std::string& flag) const { return m_Valid[Which(flag)]; }
-
 void SemiLagrangian::GetTrajectory(const std::string& flag, float* out) const {
     const int w = Which(flag);
     CLR_REQUIRE(m_Valid[w], kErrState, "trajectory '" + flag + "' has not been computed");

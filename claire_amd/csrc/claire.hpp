@@ -364,7 +364,6 @@ class SemiLagrangian {
     // per-axis stencil displacement bound in cells.  Gathers along it use the
     // LDS-staged kernels where plan_gather_lds says so, else the direct kernels.
     claire_amd::TrajectoryPlan Plan(const std::string& flag) const;
-    bool HasTrajectory(const std::string& flag) const;
     size_t DeviceBytes() const {
         return m_X[0].bytes() + m_X[1].bytes() + m_P[0].bytes() + m_P[1].bytes() + m_F.bytes() + m_F2.bytes() +
                m_Tmp.bytes();

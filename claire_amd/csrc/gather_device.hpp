@@ -124,12 +124,6 @@ __device__ __forceinline__ void setup_stencil(const float q[3], const GatherDims
     setup_axis(q[2], g.n3, hh[2], S.a3);
 }
 
-__device__ __forceinline__ void setup_stencil_u(const float u[3], const GatherDims& g, Stencil& S) {
-    setup_axis_u(u[0], g.n1, S.a1);
-    setup_axis_u(u[1], g.n2, S.a2);
-    setup_axis_u(u[2], g.n3, S.a3);
-}
-
 // Σ_c w[c]·f_c with the FMA chain starting at node 1: the order of every
 // contraction but that of the pair-layout gather within its window.
 __device__ __forceinline__ float row_sum(const float w[4], float f0, float f1, float f2, float f3) {

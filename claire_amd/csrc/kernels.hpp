@@ -265,12 +265,6 @@ struct PcgState {
 };
 // s.rz = slots[2], s.k = 0, s.done = 0, tolerances as given
 void launch_pcg_init(PcgState* s, const double* slots, double tol, double bnorm, int kmax, hipStream_t st);
-// k += 1; α = rz/pᵀw, or stop (before the updates) when pᵀw is not positive
-void launch_pcg_alpha(PcgState* s, const double* slots, hipStream_t st);
-// ‖r‖ test and the limit, else β = rᵀz_new/rᵀz, rz = rᵀz_new
-void launch_pcg_beta(PcgState* s, const double* slots, hipStream_t st);
-// y += (sign > 0 ? α : −α)·x unless stopped
-void launch_axpy_pcg(const PcgState* s, int sign, const float* x, float* y, int64_t n, hipStream_t st);
 // p = β·p + z unless stopped
 void launch_xpay_pcg(const PcgState* s, float* p, const float* z, int64_t n, hipStream_t st);
 // d += α·p and r −= α·w in one launch unless stopped

@@ -81,16 +81,6 @@ __device__ __forceinline__ void pcg_beta(PcgState* s, double rr, double rz_new) 
     s->beta = static_cast<float>(rz_new / s->rz);
     s->rz = rz_new;
 }
-__global__ void k_pcg_alpha(PcgState* s, const double* __restrict__ slots) { pcg_alpha(s, slots[0]); }
-__global__ void k_pcg_beta(PcgState* s, const double* __restrict__ slots) { pcg_beta(s, slots[1], slots[2]); }
-__global__ __launch_bounds__(kThreads) void k_axpy_pcg(const PcgState* __restrict__ s, int sign,
-                                                       const float* __restrict__ x, float* __restrict__ y,
-                                                       int64_t n) {
-    if (s->done) return;
-    const float a = sign > 0 ? s->a : s->na;
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (i < n) y[i] = a * x[i] + y[i];
-}
 // d += α·p and r −= α·w in one pass (the two updates of a CG step)
 __global__ __launch_bounds__(kThreads) void k_axpy2_pcg(const PcgState* __restrict__ s, const float* __restrict__ p,
                                                         float* __restrict__ d, const float* __restrict__ w,
@@ -329,9 +319,9 @@ __global__ __launch_bounds__(kThreads) void k_reduce_partial_dot2(const float* _
 }
 
 // Final sums of the CG products, then the CG scalar step on thread 0:
-//   NSUM = 1: slots[0] = pᵀw, then α (as k_pcg_alpha);
-//   NSUM = 2: slots[1] = rᵀr, slots[2] = rᵀz, then the stopping test and β
-//             (as k_pcg_beta), and the state copied to *host.
+//   NSUM = 1: slots[0] = pᵀw, then k += 1 and α, or the stop when pᵀw is not positive;
+//   NSUM = 2: slots[1] = rᵀr, slots[2] = rᵀz, then the stopping test and β,
+//             and the state copied to *host.
 template <int NSUM>
 __global__ __launch_bounds__(kThreads) void k_reduce_final_pcg(const double* __restrict__ partial, int np,
                                                                double* __restrict__ slots, PcgState* s,
@@ -391,15 +381,6 @@ void launch_sub(const float* x, const float* y, float* z, int64_t n, hipStream_t
 }
 void launch_pcg_init(PcgState* s, const double* slots, double tol, double bnorm, int kmax, hipStream_t st) {
     hipLaunchKernelGGL(k_pcg_init, dim3(1), dim3(1), 0, st, s, slots, tol, bnorm, kmax);
-}
-void launch_pcg_alpha(PcgState* s, const double* slots, hipStream_t st) {
-    hipLaunchKernelGGL(k_pcg_alpha, dim3(1), dim3(1), 0, st, s, slots);
-}
-void launch_pcg_beta(PcgState* s, const double* slots, hipStream_t st) {
-    hipLaunchKernelGGL(k_pcg_beta, dim3(1), dim3(1), 0, st, s, slots);
-}
-void launch_axpy_pcg(const PcgState* s, int sign, const float* x, float* y, int64_t n, hipStream_t st) {
-    if (n > 0) hipLaunchKernelGGL(k_axpy_pcg, dim3(blocks_for(n)), dim3(kThreads), 0, st, s, sign, x, y, n);
 }
 void launch_axpy2_pcg(const PcgState* s, const float* p, float* d, const float* w, float* r, int64_t n,
                       hipStream_t st) {
