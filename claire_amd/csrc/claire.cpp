@@ -828,7 +828,6 @@ int CLAIRE::SolveStateEquation() {
     CLR_REQUIRE(m_HaveTemplate, kErrState, "template image not set");
     const int64_t nl = m_Opt.domain.nl;
     const int nt = m_Opt.nt;
-    // the SL solves and the continuity equation need the trajectories
     float* m = m_State.get();
     // m^0 = mT (src/CLAIRE.cpp:1896) is where the template is kept (with a copy in
     // every solve an objective took 560 µs at 192³, 541 without)

@@ -272,11 +272,11 @@ __device__ __forceinline__ void fft_regs(c32 (&v)[Plan<N>::V], c32* s, const Lay
 // Blocks of one or two waves reach more CUs on small grids, wait for fewer waves at
 // their barriers and leave LDS for more blocks; a column block takes at least 16
 // columns, 128-byte segments, and more where they gain by it.  Against 256 threads
-// per block everywhere (µs, outputs identical): gradient of 32³ 27.5 -> 19.5 in all;
-// x2 pass of 96³ 11.7 -> 9.3 with 32 columns for 64, of 64×64×150 8.5 -> 7.2; x1
-// gradient of 64³ 9.3 -> 7.4, of 150³ 31.6 -> 28.4, of 192³ 35.8 -> 32.6 with 16
-// columns for 32; three-field rows of 256×192×150 68 -> 61 and 72 -> 65 with 25 pairs
-// for 51.
+// per block everywhere (µs; the outputs differ by 4e-8 of their norm at most, where
+// the compiler fuses other products): gradient of 32³ 27.5 -> 19.5 in all; x2 pass of
+// 96³ 11.7 -> 9.3 with 32 columns for 64, of 64×64×150 8.5 -> 7.2; x1 gradient of 64³
+// 9.3 -> 7.4, of 150³ 31.6 -> 28.4, of 192³ 35.8 -> 32.6 with 16 columns for 32;
+// three-field rows of 256×192×150 68 -> 61 and 72 -> 65 with 25 pairs for 51.
 template <int N, int B_>
 struct Geo {
     static constexpr int V = Plan<N>::V;

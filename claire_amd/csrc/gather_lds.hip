@@ -13,8 +13,9 @@
 //     (low side) and D+2 (high side) cells in x2 and x3, where D is the exact
 //     per-axis stencil displacement bound of the plan (D <= 2 covers CFL 2),
 //     so every stencil of the tile lies inside the ring by construction; larger
-//     displacements, and raw query points, take windows centred per block, with
-//     the few points outside them read from global memory (see PointMode);
+//     displacements, and raw query points, take windows centred per block on
+//     large grids, and the points outside them are read from global memory (see
+//     PointMode; centred_windows and launch_points_gather say when);
 //   * the ring has one spare slot: while the block evaluates plane x1 the
 //     global loads of plane x1+D+3 and of the next plane's query points are
 //     in flight and land in the spare slot / registers afterwards, so each
@@ -382,8 +383,10 @@ struct PairGeo {
 // For the last two the window of a block is centred on the mean offset of a
 // sample of its points (a smooth deformation is nearly rigid over a tile), and a
 // point whose stencil is not inside reads it from global memory, in the
-// arithmetic of the direct kernels.  A block whose sample lies mostly outside
-// (scattered points) stages nothing and takes the direct way throughout.
+// arithmetic of the direct kernels.  A block with less than 60% of its sample
+// inside (scattered points) stages nothing and takes the direct way throughout:
+// with 75% the gather at points of 256³ moved by noise of ±2.5 cells took 599 µs,
+// 556 with 60, and for ±3 cells 601, 655 with 60.
 enum PointMode { kPtsNear = 0, kPtsPlan = 1, kPtsRaw = 2 };
 // most planes per block of the last two (one bit of a mask each; raw points keep
 // to 32 bits and to input planes one step ahead, or the kernel runs out of
@@ -1085,11 +1088,11 @@ std::vector<int> chunk_candidates(int n1, int64_t tiles, int per_cu, int most) {
 // of a gather shape (bound D, grid, number of fields) times the candidates on
 // the launch stream, each kTuneRuns times in turn, and keeps the one with the
 // shortest run for every later launch of that shape (a single run each had kept
-// a length up to 10% slower than the best).  The chunk length only changes how the planes are
-// split among blocks, not the arithmetic of any point, so every candidate
-// writes the same output; repeating a launch is harmless because no gather
-// writes a buffer it reads (the launchers check it: the steps refuse to run in
-// place, and the RK4 stage sums ping-pong between two buffers).  Tuning is
+// a length up to 10% slower than the best).  The chunk length only changes how the
+// planes are split among blocks, not the arithmetic of any point, so every
+// candidate writes the same output; repeating a launch is harmless because no
+// gather writes a buffer it reads (the launchers check it: the steps refuse to run
+// in place, and the RK4 stage sums ping-pong between two buffers).  Tuning is
 // skipped while the stream is being captured into a graph;
 // CLAIRE_AMD_GATHER_TUNE=0 turns it off (the model's first choice is used).
 // Launches with centred windows always take the model's first choice: how long
@@ -1097,7 +1100,8 @@ std::vector<int> chunk_candidates(int n1, int64_t tiles, int per_cu, int most) {
 // so the first call's points would decide for all later ones, and a call at raw
 // points would wait for its stream.  Over smooth maps of CFL 2.5 to 9 at 96³ to
 // 512³ that choice is 2.8% (geometric mean) off the best length of each input
-// and within 6% of the one timed at CFL 2.5.
+// and within 6% of the one timed at CFL 2.5; at CFL 13 shorter chunks, which drift
+// less, would win (three fields of 128³ 86 µs with 13 planes, 109 with its choice).
 constexpr int kTuneRuns = 3;
 struct ShapeKey {
     int d, n1, n2, n3, nz;
@@ -1195,23 +1199,26 @@ void check_lds_dims(const GatherDims& g) {
 
 // Points of a launch from which bounds above 2 take centred windows (kPtsPlan).
 // Finding the centres costs a block about 2 µs, which small launches, one block
-// per CU, do not hide.  Centred windows against the D <= 4 kernel at CFL 4.5 and
-// the direct kernels at CFL 9, one field: 64³ 8.5 : 6.8 µs (CFL 4.5); 96³
-// 14.2 : 15.8 and 18.4 : 22.0; 128³ 21.0 : 22.9 and 25.8 : 45.3; 256³ 93 : 140
-// and 145 : 360.  Three fields: 64³ 13.7 : 13.7 and 18.6 : 25.1; 96³ 27.2 : 36.8
-// and 34.7 : 58.2; 256³ 271 : 392.
+// per CU, do not hide.  Centred windows against the kernel they replace (D <= 4 up
+// to CFL 4, else the direct one), one field: 64³ 8.5 : 6.8 µs (CFL 4); 96³ 14.5 :
+// 15.5 (CFL 3.5) and 20.9 : 20.9 (CFL 6); 128³ 21.6 : 23.6 and 27 : 41; 256³ 102 :
+// 152 and 130 : 266.  Three fields: 64³ 13.7 : 13.7 (CFL 4); 96³ 28 : 38 and 36 :
+// 56; 128³ 47 : 61 and 62 : 117; 256³ 301 : 419 and 360 : 792.
 constexpr int64_t kFarPoints = int64_t(1) << 19;
 // Share of far-apart points (PlanBound::spread) up to which they are the faster
 // ones, by the kernel they replace: one that a bound of 4 cells suffices for, or
 // the direct one.  In µs against that kernel, scalar and three fields, for smooth
 // fields of up to so many cells and for noise:
-//   bound 4    96³  3.5 smooth (spread 0.03) 14.4 : 15.5  28 : 37
-//             128³  the same (0.02) 21.6 : 23.7  46 : 60, noise 2.8 36 : 31  100 : 88
-//             256³  the same (0.00) 98 : 144  291 : 401, (above 0.05) 272 : 206  754 : 614
-//   above 4    96³  9 smooth (0.68) 29.3 : 23.5  62 : 62
-//             128³  9 smooth (0.65) 40.7 : 47.2  114 : 129, 20 smooth (0.96) 79 : 58  213 : 166
-//             256³  9 smooth (0.38) 204 : 288  497 : 856, 20 smooth (0.88) 453 : 394  1064 : 1218
-//                   noise 5 (0.66) 624 : 767  1925 : 2458, 30 (1.00) 2013 : 1794  8340 : 5022
+//   bound 4    96³  3.5 smooth (spread 0.03) 14.5 : 15.5  28 : 38
+//             128³  the same (0.02) 21.6 : 23.6  47 : 61, noise 2.8 36 : 31  101 : 87
+//             256³  the same (0.00) 102 : 152  301 : 419, noise 2.8 273 : 205  751 : 610
+//   above 4    96³  9 smooth (0.68) 29.0 : 22.4  63 : 60
+//             128³  9 smooth (0.65) 40.9 : 43.1  115 : 123, 20 smooth (0.96) 81 : 51  209 : 147
+//             256³  9 smooth (0.38) 204 : 274  498 : 812, 20 smooth (0.88) 450 : 336  1061 : 1029
+//                   noise 5 (0.66) 615 : 630  1898 : 1983, 30 (1.00) 1997 : 1453  8293 : 4428
+// Some cases lie on the wrong side of a line that is one number for all grids: 96³
+// 9 smooth scalar keeps the windows (29.1 µs), noise of 5 cells at 128³ too (83 :
+// 70), three fields of 64³ at 8 cells 33 : 28.
 constexpr float kMostSpread[2] = {0.05f, 0.65f};
 
 bool centred_windows(const GatherDims& g, PlanBound b, int nz) {
@@ -1252,10 +1259,17 @@ bool plan_gather_lds(const GatherDims& g, PlanBound b, int nz) {
 }
 
 void launch_points_gather(const GatherDims& g, const float* f, const float* X, float* out, hipStream_t st) {
-    // Raw points cost the centred windows their encoding too: image warps by
-    // smooth maps of CFL 2 to 9 at 128³ take 25-38 µs against 44-47 directly, at
-    // 192×150×256 and CFL 6 69 : 125, at 256³ and CFL 3 121 : 357; at 96³ 17.5 :
-    // 19.3 (CFL 2) and 22.5 : 20.9 (CFL 6), at 64³ 10.2 : 7.8.
+    // Raw points cost the centred windows their encoding too.  Smooth maps in µs
+    // against the direct kernel: 64³ CFL 2 10.1 : 7.7; 96³ CFL 2 18.0 : 18.9, CFL 8
+    // 25.8 : 21.3; 128³ CFL 3 26 : 38, CFL 9 40 : 42; 192×150×256 CFL 3 67 : 99, CFL 9
+    // 88 : 102; 256³ CFL 3 134 : 259, CFL 9 163 : 263.  The points stay on the device,
+    // so nothing is known of them here, and each block decides for itself.  Blocks of
+    // 512 threads with an equal count of planes balance direct reads worse than the
+    // direct kernel's small blocks do, so scattered points pay for it.  At 128³,
+    // 192×150×256 and 256³: noise of ±2 cells 35 : 68, 105 : 199, 203 : 473; ±4 86 :
+    // 71, 348 : 255, 720 : 647; ±8 107 : 118, 570 : 424, 1150 : 1044; one point in ten
+    // anywhere 62 : 46, 271 : 214, 630 : 530; all anywhere 319 : 316, 1886 : 1857, 4923 :
+    // 4917; folding maps of CFL 20 77 : 50, 193 : 110, 368 : 301.
     if (g.nl < (int64_t(1) << 20)) return launch_gather1(g, f, X, out, st);
     check_lds_dims(g);
     launch_lds<kPtsRaw>(g, X, f, 0, 1, EpiPlain{out, 0}, st);

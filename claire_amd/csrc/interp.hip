@@ -10,8 +10,10 @@
 //     whether the LDS-staged gathers can be used;
 //   * direct gathers (one thread per point, stencil rows read from global
 //     memory as unaligned 16-byte loads) for what the LDS-staged gathers do not
-//     take: small grids with query points anywhere or displacements beyond their
-//     windows, and trajectories with points that are not finite.
+//     take: raw query points on small grids, displacements of more than four
+//     cells on small grids or where neighbouring points go far apart, trajectories
+//     with points that are not finite, and calls in a caller's own graph capture
+//     (no host wait, so no displacement bound).
 #include <algorithm>
 
 #include "gather_device.hpp"
@@ -243,7 +245,7 @@ __device__ __forceinline__ int encode_point(const GatherDims& g, const HH& hh, c
 // kernels wait for up to 2048 atomics on one address.  Measured with the
 // division-free x/2π (gather_device.hpp): set velocity + both trajectories +
 // one gather at 64³ 281 -> 188 µs, 96³ 391 -> 262, 128³ 462 -> 343, 256³
-// 1703 -> 1627, outputs identical.
+// 1703 -> 1627.
 static_assert(kPlanBlocks >= 1 && kThreads == 256, "block_words_to folds four waves");
 
 __global__ __launch_bounds__(kThreads) void k_make_plan(GatherDims g, HH hh, const float* __restrict__ X,

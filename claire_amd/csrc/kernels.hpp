@@ -154,7 +154,8 @@ void launch_lds_traj_rk4_stage(int stage, const Dims& d, const uint32_t* P, Plan
                                float sigma, float ht, const float* Fin, float* Fout, float* X, hipStream_t st);
 // Whether the gathers of nz fields along a plan of this bound run LDS-staged: the
 // bound is at most kNearBound, or the points are finite, many enough for windows
-// centred per block and close enough together for most to lie in them.
+// centred per block and close enough together for most to lie in them.  The direct
+// kernels take the rest; the two agree up to roundings (other products are fused).
 constexpr int kNearBound = 4;
 bool plan_gather_lds(const GatherDims& g, PlanBound bound, int nz);
 // Update coefficient per point: C = 1 + ht/2·(α·dX + α·(1 + ht·α·dX)·d)
