@@ -1212,14 +1212,12 @@ constexpr int64_t kFarPoints = int64_t(1) << 19;
 //   bound 4    96³  3.5 smooth (spread 0.03) 14.5 : 15.5  28 : 38
 //             128³  the same (0.02) 21.6 : 23.6  47 : 61, noise 2.8 36 : 31  101 : 87
 //             256³  the same (0.00) 102 : 152  301 : 419, noise 2.8 273 : 205  751 : 610
-//   above 4    96³  9 smooth (0.68) 29.0 : 22.4  63 : 60
-//             128³  9 smooth (0.65) 40.9 : 43.1  115 : 123, 20 smooth (0.96) 81 : 51  209 : 147
-//             256³  9 smooth (0.38) 204 : 274  498 : 812, 20 smooth (0.88) 450 : 336  1061 : 1029
-//                   noise 5 (0.66) 615 : 630  1898 : 1983, 30 (1.00) 1997 : 1453  8293 : 4428
-// Some cases lie on the wrong side of a line that is one number for all grids: 96³
-// 9 smooth scalar keeps the windows (29.1 µs), noise of 5 cells at 128³ too (83 :
-// 70), three fields of 64³ at 8 cells 33 : 28.
-constexpr float kMostSpread[2] = {0.05f, 0.65f};
+//   above 4    96³  8 smooth (0.4 to 0.45) 25.3 : 22.3  51 : 60, 9 (0.5 to 0.55) 29 : 22.6  62 : 60
+//             128³  9 smooth (0.45 to 0.5) 40 : 43  114 : 123, 20 (> 0.65) 81 : 51  209 : 147
+//       192×150×256 10 smooth (< 0.4) 114 : 110  280 : 322, 12 (0.5 to 0.55) 146 : 113  351 : 333
+//             256³  9 smooth (< 0.4) 204 : 278  500 : 826, 12 (0.5 to 0.55) 399 : 285  743 : 857
+//        noise 5 (0.5 to 0.55)  128³ 83 : 70  251 : 207, 256³ 610 : 627  1873 : 2001
+constexpr float kMostSpread[2] = {0.05f, 0.5f};
 
 bool centred_windows(const GatherDims& g, PlanBound b, int nz) {
     return g.nl * nz >= kFarPoints && b.spread <= kMostSpread[b.d > kNearBound];
